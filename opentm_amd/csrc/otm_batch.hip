@@ -245,6 +245,14 @@ struct OpTail {  // one workgroup per cell: the tail V-cycle from level C.tail d
   }
 };
 
+struct OpCoarsestRows {  // cells without a tail: the coarsest product by rows
+  static constexpr int kThreads = kBlock;
+  __device__ void operator()(const CellDev& C, const Ent& e, int lb, int) const {
+    const int l = C.nlev - 1;
+    coarsest_rows_body(C.g[l], C.Binv, C.f[l], ucur(C, e.par, l), lb);
+  }
+};
+
 template <typename XT>
 struct OpInitResid {
   static constexpr int kThreads = kBlock;
@@ -410,11 +418,32 @@ struct OpPackFp16 {  // what 0: clear scale, 1: |coupling| max, 2: pack
   }
 };
 
-struct OpCoarsestInvert {  // one workgroup per cell, work matrix in dynamic LDS (n <= kInvertLdsMax)
-  static constexpr int kThreads = kFactorThreads;
+struct OpCoarsestInvert {  // one workgroup per cell (n <= kInvertLdsMax)
+  static constexpr int kThreads = kBlock;
   __device__ void operator()(const CellDev& C, const Ent&, int, int) const {
-    extern __shared__ double A[];
-    coarsest_invert_lds_body(C.g[C.nlev - 1], C.st_w[C.nlev - 1], A, C.Binv_w);
+    coarsest_invert_small_body(C.g[C.nlev - 1], C.st_w[C.nlev - 1], C.Binv_w);
+  }
+};
+
+// Larger coarsest levels, the single-cell launches' bodies for all cells at
+// once; what -2: diagonal, -1: assembly, >= 0: that elimination step.
+struct OpGj {
+  static constexpr int kThreads = kBlock;
+  int what;
+  __device__ void operator()(const CellDev& C, const Ent&, int lb, int) const {
+    const Geom& g = C.g[C.nlev - 1];
+    const float* st = C.st_w[C.nlev - 1];
+    const GjWork W = gj_work(g, C.cB, C.Binv_w);
+    if (what == -2) gj_diag_body(g, st, W, lb);
+    else if (what == -1) gj_assemble_body(g, st, W, lb);
+    else gj_step_body(g, W, what, lb);
+  }
+};
+
+struct OpGjSymmetrise {
+  static constexpr int kThreads = kBlock;
+  __device__ void operator()(const CellDev& C, const Ent&, int lb, int) const {
+    gj_symmetrise_body(C.g[C.nlev - 1], C.cB, C.Binv_w, (long long)lb * kBlock + threadIdx.x);
   }
 };
 
@@ -605,16 +634,6 @@ void add_op(otm_batch* b, const std::vector<Member*>& set, Op op, std::function<
   });
 }
 
-template <class Op>
-void add_op_lds(otm_batch* b, const std::vector<Member*>& set, Op op, std::function<long long(const Member&)> blocks,
-                size_t lds) {
-  CellDev* cells = b->dcells;
-  hipStream_t s = b->s;
-  add_launch(b, set, blocks, 1, [cells, s, op, lds](const Ent* e, int n, unsigned grid) {
-    hipLaunchKernelGGL(kb_run<Op>, dim3(grid), dim3(Op::kThreads), lds, s, e, n, cells, op);
-  });
-}
-
 void flush(otm_batch* b) {
   if (b->plan.empty()) {
     b->plan_ents.clear();
@@ -700,8 +719,11 @@ void plan_vcycle(otm_batch* b, std::vector<Member*>& V) {
       return (long long)nblk(restrict8(cg) ? 8 * cg.nn : cg.nn);
     });
   }
-  // bottom: every member's tail
-  add_op(b, V, OpTail{}, one);
+  // bottom: every member's tail, or its coarsest level alone
+  std::vector<Member*> tails, rows;
+  for (Member* m : V) (m->c->tail + 1 < m->nlev ? tails : rows).push_back(m);
+  add_op(b, tails, OpTail{}, one);
+  add_op(b, rows, OpCoarsestRows{}, [](const Member& m) { return coarsest_row_blocks(m.c->lv.back().g); });
   // up
   for (int l = maxlev - 2; l >= 0; l--) {
     std::vector<Member*> S = at(l, false);
@@ -907,8 +929,7 @@ struct OpZeroX {
 void plan_setup(otm_batch* b, std::vector<Member>& tmp, const std::vector<const float*>& src, int pitch, bool cold) {
   std::vector<Member*> all;
   int maxlev = 0;
-  size_t lds_max = 0;
-  std::vector<Member*> inv_lds, inv_glob;
+  std::vector<Member*> inv_small, inv_large;
   for (size_t i = 0; i < tmp.size(); i++) {
     Member& m = tmp[i];
     otm_ctx* c = m.c;
@@ -922,12 +943,7 @@ void plan_setup(otm_batch* b, std::vector<Member>& tmp, const std::vector<const 
     all.push_back(&m);
     maxlev = std::max(maxlev, m.nlev);
     const long long nc = c->lv.back().g.nn;
-    if (nc <= kInvertLdsMax) {
-      inv_lds.push_back(&m);
-      lds_max = std::max(lds_max, (size_t)(nc * nc) * sizeof(double));
-    } else {
-      inv_glob.push_back(&m);
-    }
+    (nc <= kInvertLdsMax ? inv_small : inv_large).push_back(&m);
   }
   add_op(b, all, OpCopyKappa{}, [](const Member& m) { return (long long)nblk(m.c->g0.nn); });
   if (cold) add_op(b, all, OpZeroX{}, [](const Member& m) { return std::min<long long>(8192, nblk(3 * m.c->g0.nn)); });
@@ -945,21 +961,26 @@ void plan_setup(otm_batch* b, std::vector<Member>& tmp, const std::vector<const 
            [l](const Member& m) { return std::min<long long>(1024, (long long)nblk(m.c->lv[l].g.nn)); });
     add_op(b, P, OpPackFp16{l, 2}, [l](const Member& m) { return (long long)nblk(m.c->lv[l].g.nn); });
   }
-  if (!inv_lds.empty())
-    hip_check(hipFuncSetAttribute((const void*)kb_run<OpCoarsestInvert>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)(kInvertLdsMax * kInvertLdsMax * sizeof(double))),
-              "hipFuncSetAttribute");
-  add_op_lds(b, inv_lds, OpCoarsestInvert{}, one, lds_max);
-  // larger coarsest levels: the blocked multi-workgroup inverse, per cell
-  for (Member* m : inv_glob) {
-    const otm_ctx* c = m->c;
-    const Geom g = c->lv.back().g;
-    const float* st = c->lv.back().st;
-    double* B = c->cB;
-    double* Binv = c->cBinv;
-    hipStream_t s = b->s;
-    b->plan.push_back({[s, g, st, B, Binv](const Ent*) { launch_coarsest_blocked(s, g, st, B, Binv); }, 0});
+  add_op(b, inv_small, OpCoarsestInvert{}, one);
+  // larger coarsest levels: each elimination step of all cells in one launch
+  auto tiles = [](const Member& m) {
+    const long long t = gj_tiles(m.c->lv.back().g);
+    return t * t;
+  };
+  add_op(b, inv_large, OpGj{-2}, [](const Member& m) { return (long long)nblk(32 * m.c->lv.back().g.nn); });
+  add_op(b, inv_large, OpGj{-1}, tiles);
+  int steps = 0;
+  for (Member* m : inv_large) steps = std::max(steps, gj_steps(m->c->lv.back().g));
+  for (int k = 0; k < steps; k++) {
+    std::vector<Member*> S;
+    for (Member* m : inv_large)
+      if (k < gj_steps(m->c->lv.back().g)) S.push_back(m);
+    add_op(b, S, OpGj{k}, tiles);
   }
+  add_op(b, inv_large, OpGjSymmetrise{}, [](const Member& m) {
+    const long long n = m.c->lv.back().g.nn;
+    return (long long)nblk(n * n);
+  });
 }
 
 // Adds a context as a member in slot `slot` (its CellDev is uploaded at

@@ -342,15 +342,45 @@ __device__ inline void prolong_body(const Geom& fg, const Geom& cg, const float*
   }
 }
 
-// u = Binv f for right-hand side k, row i, FP64 accumulation.
-__device__ inline void coarsest_solve_body(const Geom& g, const double* __restrict__ Binv,
-                                           const float* __restrict__ f, float* __restrict__ u, int i, int k) {
-  const int n = (int)g.nn;
-  if (i >= n) return;
-  const float* fk = f + (long long)k * n;
-  double s = 0.0;
-  for (int j = 0; j < n; j++) s += Binv[(long long)i * n + j] * (double)fk[j];
-  u[(long long)k * n + i] = (float)s;
+// u = Binv f on the coarsest level for the three load cases, FP64
+// accumulation: one wave takes two rows of Binv (lanes stride the columns,
+// so a row is read in whole cache lines and the load cases' values serve
+// both rows) and adds its lanes' sums in a fixed order.
+// Bound by reading Binv once, 8 n^2 bytes, and below a few hundred nodes by
+// latency. One workgroup inside the tail kernel, a thread per (row, load
+// case) walking its row alone, took 6367 us at n = 1331, 479 us at 576 and
+// 56 us at 216; spread over the chip 7.5, 4 and 3.5 us.
+constexpr int kCoarsestRows = 2 * kWaves;  // rows of one block
+__host__ __device__ inline long long coarsest_row_blocks(const Geom& g) {
+  return (g.nn + kCoarsestRows - 1) / kCoarsestRows;
+}
+__device__ inline void coarsest_rows_body(const Geom& g, const double* __restrict__ Binv,
+                                          const float* __restrict__ f, float* __restrict__ u, int lb) {
+  const int n = (int)g.nn, lane = threadIdx.x & 63;
+  const int i0 = lb * kCoarsestRows + 2 * ((int)threadIdx.x >> 6);
+  if (i0 >= n) return;
+  const int i1 = i0 + 1 < n ? i0 + 1 : i0;
+  const double* __restrict__ r0 = Binv + (long long)i0 * n;
+  const double* __restrict__ r1 = Binv + (long long)i1 * n;
+  double s0[OTM_NRHS] = {0, 0, 0}, s1[OTM_NRHS] = {0, 0, 0};
+#pragma unroll 4
+  for (int j = lane; j < n; j += 64) {
+    const double b0 = r0[j], b1 = r1[j];
+#pragma unroll
+    for (int k = 0; k < OTM_NRHS; k++) {
+      const double fv = (double)f[k * n + j];
+      s0[k] += b0 * fv;
+      s1[k] += b1 * fv;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < OTM_NRHS; k++) {
+    const double v0 = wave_sum(s0[k]), v1 = wave_sum(s1[k]);
+    if (lane == 0) {
+      u[k * n + i0] = (float)v0;
+      u[k * n + i1] = (float)(i1 == i0 ? v0 : v1);
+    }
+  }
 }
 
 // Brick smoother for stored-stencil levels. One 512-thread workgroup owns an
@@ -680,102 +710,405 @@ __device__ inline void stencil_pack_body(const Geom& g, const float* __restrict_
 // null-space projection, grid.cpp:272-310, :432-510). The result is its
 // explicit inverse Binv, so every V-cycle's coarsest solve is one small
 // dense matrix-vector product on the device.
-constexpr int kFactorThreads = 1024;
-constexpr int kInvertLdsMax = 128;  // n*n doubles in LDS up to n = 128 (128 KiB)
+//
+// The inverse is a blocked Gauss-Jordan elimination of the SPD matrix (no
+// pivoting), kGjB pivots per step, K the step's pivot rows, O all others:
+//   D = A_KK^-1,  A_KK <- D,  A_KO <- D A_KO,  A_OK <- -A_OK D,
+//   A_OO <- A_OO - A_OK (D A_KO),
+// the products in FP64 matrix instructions. With the columns of K in the
+// old pivot rows replaced by the identity and the old A_OK by zero, all four
+// are one rule: R = D A_K:, rows of K become R, other rows A - A_:K R.
+constexpr int kGjB = 32;            // pivots per step
+constexpr int kGjTile = 64;         // tile edge of a workgroup
+constexpr int kInvertLdsMax = 64;   // one workgroup holds the matrix in LDS up to this size
 
-__device__ inline void coarsest_assemble(const Geom& g, const float* __restrict__ st, double* B, double* red,
-                                         double* alpha_sh) {
+// Row strides (doubles) of the LDS operands: 16 rows 34 apart, and two rows
+// 80 apart, start on different banks.
+constexpr int kGjStrideC = kGjB + 2, kGjStrideR = kGjTile + 16;
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+// Entry (i, j), i != j, of the symmetrised coarse matrix: the mean of the
+// two stencil entries that describe the coupling (a coarsest edge has at
+// least 3 nodes, so there is one pair), 0 between nodes that do not touch.
+// ci and cj are the nodes' coordinates packed by gj_coord.
+__device__ inline int gj_coord(const Geom& g, int i) {
+  int x, y, z;
+  split_node(g.nx, g.ny, i, x, y, z);
+  return x | (y << 10) | (z << 20);
+}
+__device__ inline double gj_offdiag(const Geom& g, const float* __restrict__ st, int i, int ci, int j, int cj) {
   const int n = (int)g.nn;
-  const int tid = threadIdx.x, bs = blockDim.x;
-  for (int i = tid; i < n * n; i += bs) B[i] = 0.0;
-  __syncthreads();
-  for (int v = tid; v < n; v += bs) {
-    const int x = v % g.nx, y = (v / g.nx) % g.ny, z = v / (g.nx * g.ny);
-    for (int o = 0; o < 27; o++) {
-      const int w = wrapm(x + o % 3 - 1, g.nx) + g.nx * (wrapm(y + (o / 3) % 3 - 1, g.ny) +
-                                                         g.ny * wrapm(z + o / 9 - 1, g.nz));
-      B[v * n + w] += (double)st[o * n + v];
+  const int dims[3] = {g.nx, g.ny, g.nz};
+  int o = 0, w = 1;
+  bool touch = true;
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    int d = ((cj >> (10 * a)) & 1023) - ((ci >> (10 * a)) & 1023);
+    if (d == dims[a] - 1) d = -1;
+    else if (d == 1 - dims[a]) d = 1;
+    touch = touch && d >= -1 && d <= 1;
+    o += w * (d + 1);
+    w *= 3;
+  }
+  o = touch ? o : 13;  // loads without a branch, so several entries' are in flight
+  const double a = 0.5 * ((double)st[o * n + i] + (double)st[(26 - o) * n + j]);
+  return touch ? a : 0.0;
+}
+
+// Minus the sum of node v's off-diagonal couplings, by 32 lanes (every lane
+// gets it).
+__device__ inline double gj_diag(const Geom& g, const float* __restrict__ st, int v) {
+  const int n = (int)g.nn, o = (int)threadIdx.x & 31;
+  double a = 0.0;
+  if (o < 27 && o != 13) {
+    int x, y, z;
+    split_node(g.nx, g.ny, v, x, y, z);
+    const int w = wrapm(x + o % 3 - 1, g.nx) +
+                  g.nx * (wrapm(y + (o / 3) % 3 - 1, g.ny) + g.ny * wrapm(z + o / 9 - 1, g.nz));
+    a = 0.5 * ((double)st[o * n + v] + (double)st[(26 - o) * n + w]);
+  }
+#pragma unroll
+  for (int m = 16; m > 0; m >>= 1) a += __shfl_xor(a, m, 64);
+  return -a;
+}
+
+// 1/v of a pivot (finite, positive): the hardware estimate and two
+// Newton-Raphson steps, within an ulp.
+__device__ inline double gj_rcp(double v) {
+  double r = __builtin_amdgcn_rcp(v);
+  r = fma(fma(-v, r, 1.0), r, r);
+  r = fma(fma(-v, r, 1.0), r, r);
+  return r;
+}
+
+// In-place inverse of the kGjB x kGjB SPD matrix m (LDS, row stride
+// kGjStrideC) by 256 threads: thread t keeps rows 4 (t/32) .. + 3 of column
+// t%32 in registers. Blocked Gauss-Jordan with four pivots a step: the 32
+// threads that own the pivot rows write them to LDS, one barrier, and every
+// thread factors the 4 x 4 pivot block (L D L^T, the scalar elimination's
+// arithmetic) and solves for its column. The elimination keeps the matrix
+// symmetric up to the sign between eliminated and remaining indices, so the
+// pivot columns come from the same rows. Bound by its serial chain, 8 steps
+// of one barrier and four reciprocals each: about 8 us. One pivot a step (32
+// barriers) took 13 us; the matrix in LDS, two barriers, a division and
+// runtime index divisions a step 29 us.
+constexpr int kGjP = 4;  // pivots of such a step
+__device__ __forceinline__ void gj_invert_block(double* m, double (*rows)[kGjP][kGjB]) {
+  const int j = (int)threadIdx.x & 31, ib = (int)threadIdx.x >> 5, i0 = kGjP * ib;
+  double a[kGjP];
+#pragma unroll
+  for (int r = 0; r < kGjP; r++) a[r] = m[(i0 + r) * kGjStrideC + j];
+#pragma unroll 1  // one step's code stays in the instruction cache
+  for (int s = 0; s < kGjB / kGjP; s++) {
+    double(*X)[kGjB] = rows[s & 1];
+    if (ib == s) {
+#pragma unroll
+      for (int r = 0; r < kGjP; r++) X[r][j] = a[r];
+    }
+    __syncthreads();
+    const int k0 = kGjP * s;
+    double P[kGjP][kGjP], L[kGjP][kGjP], d[kGjP], t[kGjP];
+#pragma unroll
+    for (int u = 0; u < kGjP; u++) {
+#pragma unroll
+      for (int v = 0; v < kGjP; v++) P[u][v] = X[u][k0 + v];
+      t[u] = X[u][j];
+    }
+    const bool inK = j >= k0 && j < k0 + kGjP;
+#pragma unroll
+    for (int u = 0; u < kGjP; u++)
+      if (inK) t[u] = j == k0 + u ? 1.0 : 0.0;
+#pragma unroll
+    for (int u = 0; u < kGjP; u++) {
+      d[u] = gj_rcp(P[u][u]);
+#pragma unroll
+      for (int v = u + 1; v < kGjP; v++) {
+        L[v][u] = P[u][v] * d[u];
+#pragma unroll
+        for (int w = u + 1; w <= v; w++) P[w][v] = fma(-L[v][u], P[u][w], P[w][v]);
+        t[v] = fma(-L[v][u], t[u], t[v]);
+      }
+    }
+#pragma unroll
+    for (int u = kGjP - 1; u >= 0; u--) {
+      t[u] *= d[u];
+#pragma unroll
+      for (int v = u + 1; v < kGjP; v++) t[u] = fma(-L[v][u], t[v], t[u]);
+    }
+    const double sign = ib < s ? 1.0 : -1.0;  // minus the pivot columns' entries
+#pragma unroll
+    for (int r = 0; r < kGjP; r++) {
+      double v = inK ? 0.0 : a[r];
+#pragma unroll
+      for (int u = 0; u < kGjP; u++) v = fma(sign * X[u][i0 + r], t[u], v);
+      a[r] = ib == s ? t[r] : v;
     }
   }
-  __syncthreads();
-  for (int i = tid; i < n * n; i += bs) {
-    const int a = i / n, b = i - a * n;
-    if (a < b) {
-      const double m = 0.5 * (B[a * n + b] + B[b * n + a]);
-      B[a * n + b] = m;
-      B[b * n + a] = m;
-    }
-  }
-  __syncthreads();
-  double tr = 0.0;
-  for (int a = tid; a < n; a += bs) {
-    double s = 0.0;
-    for (int b = 0; b < n; b++)
-      if (b != a) s += B[a * n + b];
-    B[a * n + a] = -s;
-    tr += -s;
-  }
-  tr = wave_sum(tr);
-  if ((tid & 63) == 0) red[tid >> 6] = tr;
-  __syncthreads();
-  if (tid == 0) {
-    double s = 0.0;
-    for (int w = 0; w < (bs + 63) / 64; w++) s += red[w];
-    *alpha_sh = s / ((double)n * (double)n);
-  }
-  __syncthreads();
-  const double alpha = *alpha_sh;
-  for (int i = tid; i < n * n; i += bs) B[i] += alpha;
+#pragma unroll
+  for (int r = 0; r < kGjP; r++) m[(i0 + r) * kGjStrideC + j] = a[r];
   __syncthreads();
 }
 
-// In-place Gauss-Jordan inversion of the SPD matrix A (n x n, LDS or global
-// memory): no pivoting is needed; every elimination step updates all n^2
-// entries in parallel between two barriers (2n barriers in total instead of
-// the long dependent chains of a triangular inverse). colk/rowk hold n
-// doubles each. Binv gets the symmetrised inverse.
-__device__ inline void gauss_jordan_invert(int n, double* A, double* colk, double* rowk, double* __restrict__ Binv) {
-  const int tid = threadIdx.x, bs = blockDim.x;
-  for (int k = 0; k < n; k++) {
-    const double ip = 1.0 / A[k * n + k];
-    for (int i = tid; i < n; i += bs) {
-      colk[i] = A[i * n + k];
-      rowk[i] = (i == k ? 1.0 : A[k * n + i]) * ip;
+// One 16 x 16 tile of A B over kGjB terms: A rows (stride sa) and B columns
+// (stride sb) start at a and b. Lane l holds A[l%16][4q + l/16] and
+// B[4q + l/16][l%16] of each instruction, and results (4r + l/16, l%16).
+__device__ __forceinline__ f64x4 gj_mma(const double* a, int sa, const double* b, int sb, f64x4 acc) {
+  const int l = (int)threadIdx.x & 63, lr = l & 15, lk = l >> 4;
+#pragma unroll
+  for (int q = 0; q < kGjB / 4; q++)
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[lr * sa + 4 * q + lk], b[(4 * q + lk) * sb + lr], acc, 0, 0, 0);
+  return acc;
+}
+
+// n <= kInvertLdsMax: one workgroup, the matrix in LDS. Each wave owns 16
+// rows, so after the barrier behind R a step updates them in place. At n =
+// 64, two steps, 29 us; the scalar elimination in LDS, two barriers a pivot,
+// took 67 us (n = 125: 230 us; now four launches of 11 us).
+struct GjSmallLds {
+  double A[kGjTile * kGjStrideR];
+  double R[kGjB * kGjStrideR];
+  double D[kGjB * kGjStrideC];
+  double rows[2][kGjP][kGjB];
+  double diag[kGjTile];
+  int coord[kGjTile];
+};
+__device__ inline void coarsest_invert_small_body(const Geom& g, const float* __restrict__ st,
+                                                  double* __restrict__ Binv) {
+  __shared__ GjSmallLds S;
+  const int n = (int)g.nn, tid = threadIdx.x, l = tid & 63, w = tid >> 6;
+  if (tid < kGjTile) {
+    S.coord[tid] = tid < n ? gj_coord(g, tid) : 0;
+    S.diag[tid] = 0.0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kGjTile * 32 / kBlock; r++) {
+    const int v = (tid >> 5) + (kBlock / 32) * r;
+    const double d = gj_diag(g, st, min(v, n - 1));
+    if ((tid & 31) == 0 && v < n) S.diag[v] = d;
+  }
+  __syncthreads();
+  const double alpha = wave_sum(S.diag[l]) / ((double)n * (double)n);
+  // padded with the identity beyond n
+#pragma unroll 4
+  for (int q = tid; q < kGjTile * kGjTile; q += kBlock) {
+    const int i = q / kGjTile, j = q % kGjTile;
+    const double o = gj_offdiag(g, st, min(i, n - 1), S.coord[i], min(j, n - 1), S.coord[j]);
+    S.A[i * kGjStrideR + j] = (i < n && j < n) ? (i == j ? S.diag[i] : o) + alpha : (i == j ? 1.0 : 0.0);
+  }
+  __syncthreads();
+  for (int k0 = 0; k0 < n; k0 += kGjB) {
+    for (int q = tid; q < kGjB * kGjB; q += kBlock)
+      S.D[(q / kGjB) * kGjStrideC + q % kGjB] = S.A[(k0 + q / kGjB) * kGjStrideR + k0 + q % kGjB];
+    __syncthreads();
+    gj_invert_block(S.D, S.rows);
+    // the pivot rows with the identity in the columns of K
+    for (int q = tid; q < kGjB * kGjB; q += kBlock)
+      S.A[(k0 + q / kGjB) * kGjStrideR + k0 + q % kGjB] = q / kGjB == q % kGjB ? 1.0 : 0.0;
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const f64x4 r = gj_mma(S.D + 16 * h * kGjStrideC, kGjStrideC, S.A + k0 * kGjStrideR + 16 * w, kGjStrideR,
+                             f64x4{0, 0, 0, 0});
+#pragma unroll
+      for (int q = 0; q < 4; q++) S.R[(16 * h + 4 * q + (l >> 4)) * kGjStrideR + 16 * w + (l & 15)] = r[q];
     }
     __syncthreads();
-    if (n <= bs) {
-      const int rstep = bs / n;  // rows updated per pass
-      const int j = tid % n, i0 = tid / n;
-      if (i0 < rstep)
-        for (int i = i0; i < n; i += rstep) {
-          const int q = i * n + j;
-          A[q] = (i == k) ? rowk[j] : ((j == k ? 0.0 : A[q]) - colk[i] * rowk[j]);
-        }
-    } else {
-      for (long long q = tid; q < (long long)n * n; q += bs) {
-        const int i = (int)(q / n), j = (int)(q - (long long)i * n);
-        A[q] = (i == k) ? rowk[j] : ((j == k ? 0.0 : A[q]) - colk[i] * rowk[j]);
+    const bool pivot = 16 * w >= k0 && 16 * w < k0 + kGjB;  // this wave's rows are pivot rows
+    f64x4 out[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const f64x4 acc = gj_mma(S.A + 16 * w * kGjStrideR + k0, kGjStrideR, S.R + 16 * c, kGjStrideR, f64x4{0, 0, 0, 0});
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int i = 16 * w + 4 * q + (l >> 4), j = 16 * c + (l & 15);
+        const bool inK = j >= k0 && j < k0 + kGjB;
+        out[c][q] = pivot ? S.R[(i - k0) * kGjStrideR + j] : (inK ? 0.0 : S.A[i * kGjStrideR + j]) - acc[q];
       }
     }
     __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) S.A[(16 * w + 4 * q + (l >> 4)) * kGjStrideR + 16 * c + (l & 15)] = out[c][q];
+    __syncthreads();
   }
-  for (long long q = tid; q < (long long)n * n; q += bs) {
-    const int a = (int)(q / n), b = (int)(q - (long long)a * n);
-    Binv[q] = 0.5 * (A[(long long)a * n + b] + A[(long long)b * n + a]);
+  for (int q = tid; q < n * n; q += kBlock) {
+    const int i = q / n, j = q - i * n;
+    Binv[q] = 0.5 * (S.A[i * kGjStrideR + j] + S.A[j * kGjStrideR + i]);
   }
 }
 
-// n <= kInvertLdsMax: the work matrix lives in (dynamic) LDS.
-__device__ inline void coarsest_invert_lds_body(const Geom& g, const float* __restrict__ st, double* A,
-                                                double* __restrict__ Binv) {
-  __shared__ double colk[kInvertLdsMax], rowk[kInvertLdsMax];
-  __shared__ double red[kFactorThreads / 64];
-  __shared__ double alpha_sh;
-  coarsest_assemble(g, st, A, red, &alpha_sh);
-  gauss_jordan_invert((int)g.nn, A, colk, rowk, Binv);
+// Larger n: every step is one launch over kGjTile x kGjTile tiles. The step
+// reads one n x n matrix and writes another (every entry changes anyway), so
+// its workgroups need no order among them, and each forms the R columns of
+// its own tile; the workgroup whose tile holds the next pivot block inverts
+// that block right away, and so the serial part runs beside the other tiles.
+// A step is bound by that chain: 11.3 us at n = 216 and 576, 15.6 us at 1331
+// (three launches a step with the 29 us inverse on its own: 51, 53 and 59 us;
+// the whole inverse 370, 1000 and 2500 us before, 100, 230 and 690 us now).
+// Work space of a level: the second n x n matrix, two pivot inverses, the
+// diagonal. The matrices are work and Binv by turns, the last result in work.
+__host__ __device__ inline long long gj_tiles(const Geom& g) { return (g.nn + kGjTile - 1) / kGjTile; }
+__host__ __device__ inline int gj_steps(const Geom& g) { return (int)((g.nn + kGjB - 1) / kGjB); }
+struct GjWork {
+  double *even, *odd;  // the matrix before even / odd steps
+  double* D[2];        // pivot inverse of even / odd steps
+  double* diag;
+};
+__host__ __device__ inline GjWork gj_work(const Geom& g, double* work, double* Binv) {
+  GjWork W;
+  const bool last_even = (gj_steps(g) & 1) == 0;  // the result is in `even`
+  W.even = last_even ? work : Binv;
+  W.odd = last_even ? Binv : work;
+  W.D[0] = work + g.nn * g.nn;
+  W.D[1] = W.D[0] + kGjB * kGjB;
+  W.diag = W.D[1] + kGjB * kGjB;
+  return W;
 }
 
+// Diagonal, 32 lanes per node (8 nodes per block).
+__device__ inline void gj_diag_body(const Geom& g, const float* __restrict__ st, const GjWork& W, int lb) {
+  const int v = lb * (kBlock / 32) + ((int)threadIdx.x >> 5);
+  if (v >= (int)g.nn) return;
+  const double d = gj_diag(g, st, v);
+  if ((threadIdx.x & 31) == 0) W.diag[v] = d;
+}
 
+struct GjLds {
+  double X[kGjB * kGjStrideR];     // old pivot rows of the tile's columns
+  double R[kGjB * kGjStrideR];     // D X
+  double C[kGjTile * kGjStrideC];  // old pivot columns of the tile's rows
+  double D[kGjB * kGjStrideC];     // pivot inverse; then the next pivot block
+  double rows[2][kGjP][kGjB];
+};
+__device__ inline GjLds& gj_lds() {
+  __shared__ GjLds lds;
+  return lds;
+}
+
+// Inverts the pivot block of step s that the workgroup has put in lds.D
+// (identity beyond n) and publishes it for the step.
+__device__ inline void gj_publish_pivot(const GjWork& W, int s) {
+  GjLds& L = gj_lds();
+  __syncthreads();
+  gj_invert_block(L.D, L.rows);
+  for (int q = threadIdx.x; q < kGjB * kGjB; q += kBlock)
+    W.D[s & 1][q] = L.D[(q / kGjB) * kGjStrideC + q % kGjB];
+}
+
+// Tile lb of the matrix, with alpha = tr / n^2 on every entry; the first
+// tile also inverts the first pivot block.
+__device__ inline void gj_assemble_body(const Geom& g, const float* __restrict__ st, const GjWork& W, int lb) {
+  GjLds& L = gj_lds();
+  __shared__ int coord[2][kGjTile];
+  __shared__ double sh[kWaves], alpha_sh;
+  const int n = (int)g.nn, nt = (int)gj_tiles(g), tid = threadIdx.x;
+  const int i0 = (lb / nt) * kGjTile, j0 = (lb % nt) * kGjTile;
+  if (tid < 2 * kGjTile) {
+    const int h = tid / kGjTile, v = (h ? j0 : i0) + tid % kGjTile;
+    coord[h][tid % kGjTile] = v < n ? gj_coord(g, v) : 0;
+  }
+  double tr[1] = {0.0};
+  for (int i = tid; i < n; i += kBlock) tr[0] += W.diag[i];
+  block_sum<1>(tr, sh);
+  if (tid == 0) alpha_sh = tr[0] / ((double)n * (double)n);
+  __syncthreads();
+  const double alpha = alpha_sh;
+#pragma unroll 4
+  for (int q = tid; q < kGjTile * kGjTile; q += kBlock) {
+    const int a = q / kGjTile, b = q % kGjTile, i = i0 + a, j = j0 + b;
+    const int ic = min(i, n - 1), jc = min(j, n - 1);
+    const double o = gj_offdiag(g, st, ic, coord[0][a], jc, coord[1][b]), dg = W.diag[ic];
+    const double v = (i < n && j < n) ? (i == j ? dg : o) + alpha : (i == j ? 1.0 : 0.0);
+    if (i < n && j < n) W.even[(long long)i * n + j] = v;
+    if (lb == 0 && a < kGjB && b < kGjB) L.D[a * kGjStrideC + b] = v;
+  }
+  if (lb == 0) gj_publish_pivot(W, 0);
+}
+
+// Tile lb of elimination step s.
+__device__ inline void gj_step_body(const Geom& g, const GjWork& W, int s, int lb) {
+  GjLds& L = gj_lds();
+  const int n = (int)g.nn, nt = (int)gj_tiles(g), tid = threadIdx.x, l = tid & 63, w = tid >> 6;
+  const int i0 = (lb / nt) * kGjTile, j0 = (lb % nt) * kGjTile, k0 = s * kGjB;
+  const double* __restrict__ src = (s & 1) ? W.odd : W.even;
+  double* __restrict__ dst = (s & 1) ? W.even : W.odd;
+  const double* __restrict__ D = W.D[s & 1];
+  // All loads of the tile in flight together, from clamped positions, before
+  // the first LDS store; entries beyond n become zero (and the identity in
+  // the columns of K) on the way. As guarded loads they waited for each
+  // other.
+  constexpr int kXT = kGjB * kGjTile / kBlock, kDT = kGjB * kGjB / kBlock;
+  double old[4][4], xv[kXT], cv[kXT], dv[kDT];
+#pragma unroll
+  for (int t = 0; t < kDT; t++) dv[t] = D[tid + kBlock * t];
+#pragma unroll
+  for (int t = 0; t < kXT; t++) {
+    const int q = tid + kBlock * t;
+    const int k = min(k0 + q / kGjTile, n - 1), j = min(j0 + q % kGjTile, n - 1);
+    xv[t] = src[(long long)k * n + j];
+    const int i = min(i0 + q / kGjB, n - 1), c = min(k0 + q % kGjB, n - 1);
+    cv[t] = src[(long long)i * n + c];
+  }
+#pragma unroll
+  for (int c = 0; c < 4; c++)
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int i = i0 + 16 * w + 4 * q + (l >> 4), j = j0 + 16 * c + (l & 15);
+      old[c][q] = src[(long long)min(i, n - 1) * n + min(j, n - 1)];
+    }
+#pragma unroll
+  for (int t = 0; t < kDT; t++) {
+    const int q = tid + kBlock * t;
+    L.D[(q / kGjB) * kGjStrideC + q % kGjB] = dv[t];
+  }
+#pragma unroll
+  for (int t = 0; t < kXT; t++) {
+    const int q = tid + kBlock * t;
+    const int k = k0 + q / kGjTile, j = j0 + q % kGjTile;
+    const bool inK = j >= k0 && j < k0 + kGjB;
+    L.X[(q / kGjTile) * kGjStrideR + q % kGjTile] = inK ? (j == k ? 1.0 : 0.0) : ((k < n && j < n) ? xv[t] : 0.0);
+    const int i = i0 + q / kGjB, c = k0 + q % kGjB;
+    L.C[(q / kGjB) * kGjStrideC + q % kGjB] = (i < n && c < n) ? cv[t] : 0.0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const f64x4 r = gj_mma(L.D + 16 * h * kGjStrideC, kGjStrideC, L.X + 16 * w, kGjStrideR, f64x4{0, 0, 0, 0});
+#pragma unroll
+    for (int q = 0; q < 4; q++) L.R[(16 * h + 4 * q + (l >> 4)) * kGjStrideR + 16 * w + (l & 15)] = r[q];
+  }
+  __syncthreads();
+  // k1: the next pivot block, when this tile holds it
+  const int k1 = k0 + kGjB;
+  const bool next = k1 < n && i0 == j0 && k1 >= i0 && k1 < i0 + kGjTile;
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    const f64x4 acc = gj_mma(L.C + 16 * w * kGjStrideC, kGjStrideC, L.R + 16 * c, kGjStrideR, f64x4{0, 0, 0, 0});
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int a = 16 * w + 4 * q + (l >> 4), b = 16 * c + (l & 15), i = i0 + a, j = j0 + b;
+      const bool pivot = i >= k0 && i < k0 + kGjB;
+      const bool inK = j >= k0 && j < k0 + kGjB;
+      const double v = pivot ? L.R[(i - k0) * kGjStrideR + b] : (inK ? 0.0 : old[c][q]) - acc[q];
+      if (i < n && j < n) dst[(long long)i * n + j] = v;
+      if (next && i >= k1 && i < k1 + kGjB && j >= k1 && j < k1 + kGjB)
+        L.D[(i - k1) * kGjStrideC + j - k1] = (i < n && j < n) ? v : (i == j ? 1.0 : 0.0);
+    }
+  }
+  if (next) gj_publish_pivot(W, s + 1);
+}
+
+// Binv from the last step's matrix, made exactly symmetric.
+__device__ inline void gj_symmetrise_body(const Geom& g, const double* __restrict__ work, double* __restrict__ Binv,
+                                          long long q) {
+  const long long n = g.nn;
+  if (q >= n * n) return;
+  const long long a = q / n, b = q - a * n;
+  Binv[q] = 0.5 * (work[a * n + b] + work[b * n + a]);
+}
 
 // ---- one-workgroup tail V-cycle ---------------------------------------------
 // The last levels of a hierarchy (from the first coarse level with at most
@@ -784,18 +1117,17 @@ __device__ inline void coarsest_invert_lds_body(const Geom& g, const float* __re
 // launch and memory latency. One workgroup runs the whole tail V-cycle
 // instead. The stencils of its non-coarsest levels are staged into LDS once
 // (kTailStNodes nodes at most) and the corrections of every tail level stay
-// in LDS; smoothing is exact 8-colour Gauss-Seidel (forward before
-// restriction, reverse after prolongation, so the V-cycle stays symmetric),
-// residuals and restricted right-hand sides go through the level buffers in
-// global memory (visible to the workgroup after each barrier), and the
+// in LDS, with their right-hand sides and the residual being restricted;
+// smoothing is exact 8-colour Gauss-Seidel (forward before restriction,
+// reverse after prolongation, so the V-cycle stays symmetric), and the
 // coarsest level is solved with its explicit inverse. A hierarchy whose
-// coarse levels are all larger keeps only the coarsest level in the tail
-// (up to kTailLdsNodes nodes).
+// coarse levels are all larger has no tail: its coarsest level is solved by
+// coarsest_rows_body.
 constexpr int kTailMaxLevels = 6;
 constexpr int kTailStartNodes = 512;                 // largest first tail level (8^3)
 constexpr int kTailStNodes = 512 + 64 + 8 + 1;       // stencil nodes held in LDS
 constexpr int kTailThreads = 512;  // (1024 would cap registers at 128 and spill)
-constexpr int kTailLdsNodes = 4096;                  // correction nodes held in LDS
+constexpr int kCoarsestMax = 4096;                   // largest coarsest level
 constexpr int kTailBinvNodes = 64;                   // coarsest inverse held in LDS up to this size
 static_assert(kTailStartNodes / 8 <= kTailThreads / 8, "a tail colour step has one node per group of 8 lanes");
 
@@ -901,7 +1233,7 @@ __device__ inline int tail_nodes_before(const TailLevels& T, int l) {
 }
 
 __device__ inline void tail_vcycle_body(const TailLevels& T) {
-  __shared__ float su[OTM_NRHS * kTailLdsNodes];
+  __shared__ float su[OTM_NRHS * kTailStNodes];        // corrections
   __shared__ float sst[27 * kTailStNodes];
   __shared__ float sf[OTM_NRHS * kTailStNodes];        // right-hand sides of the tail levels
   __shared__ float sres[OTM_NRHS * kTailStartNodes];   // residual of the level being restricted

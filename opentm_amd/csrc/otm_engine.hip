@@ -197,9 +197,8 @@ std::vector<Geom> otm::plan_levels(const otm_config& cfg) {
   }
   if (geoms.size() < 2) fail(OTM_E_UNSUPPORTED, "resolution too small for a two-level hierarchy");
   const long long ncoarse = geoms.back().nn;
-  if (ncoarse > 4096) fail(OTM_E_UNSUPPORTED, "coarsest level has " + std::to_string(ncoarse) +
-                                                  " nodes (> 4096); use resolutions with more factors of two");
-  if (ncoarse > kTailLdsNodes) fail(OTM_E_UNSUPPORTED, "coarsest level too large for the tail");
+  if (ncoarse > kCoarsestMax) fail(OTM_E_UNSUPPORTED, "coarsest level has " + std::to_string(ncoarse) +
+                                                          " nodes (> 4096); use resolutions with more factors of two");
   return geoms;
 }
 
@@ -250,8 +249,8 @@ static void build_hierarchy(otm_ctx* c) {
   }
   c->cB = dalloc<double>(coarsest_work_doubles(ncoarse));  // Gauss-Jordan work space
   // the tail V-cycle takes over from the first coarse level with at most
-  // kTailStartNodes nodes whose levels fit the tail's LDS (the coarsest level
-  // alone otherwise). A tail from 16^3 with stencils re-read from global
+  // kTailStartNodes nodes whose levels fit the tail's LDS (a hierarchy with
+  // no such level has no tail). A tail from 16^3 with stencils re-read from global
   // memory measured slower than the separate launches (131 against about
   // 100 us per V-cycle at 128^3); from 8^3 with the stencils in LDS it
   // replaces eleven launches.
@@ -263,7 +262,7 @@ static void build_hierarchy(otm_ctx* c) {
       if (m + 1 < c->lv.size()) st_nodes += c->lv[m].g.nn;
     }
     if (c->lv[l].g.nn <= kTailStartNodes && (int)(c->lv.size() - l) <= kTailMaxLevels &&
-        st_nodes <= kTailStNodes && nodes <= kTailLdsNodes) {
+        st_nodes <= kTailStNodes && nodes <= kTailStNodes) {
       c->tail = (int)l;
       break;
     }
@@ -377,14 +376,14 @@ static void vcycle(otm_ctx* c, size_t l) {
   Level& L = c->lv[l];
   const double nn = (double)L.g.nn;
   const int nsw = (l > 0 && c->cfg.coarse_sweeps > 0) ? c->cfg.coarse_sweeps : c->cfg.pre_sweeps;
-  if ((int)l == c->tail) {
-    ProfScope ps(c, OTM_PROF_COARSE_GS, 0.0);
-    launch_tail_vcycle(c->s, tail_levels(c, nsw, L.u));
-    return;
-  }
   if (l + 1 == c->lv.size()) {
     ProfScope ps(c, OTM_PROF_COARSEST, 8.0 * nn * nn + 24.0 * nn);
     launch_coarsest_solve(c->s, L.g, c->cBinv, L.f, L.u);
+    return;
+  }
+  if ((int)l == c->tail) {
+    ProfScope ps(c, OTM_PROF_COARSE_GS, 0.0);
+    launch_tail_vcycle(c->s, tail_levels(c, nsw, L.u));
     return;
   }
   if (L.brick && l == 0) {

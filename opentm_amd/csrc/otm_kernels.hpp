@@ -74,7 +74,6 @@ void launch_galerkin_next(hipStream_t s, const Geom& fine, const Geom& coarse, c
 void launch_stencil_from_elements(hipStream_t s, const Geom& g, const float* E, float* st);
 // Device doubles the coarsest factorisation needs as work space for n nodes.
 size_t coarsest_work_doubles(long long n);
-void launch_coarsest_blocked(hipStream_t s, const Geom& g, const float* st, double* B, double* Binv);
 void launch_coarsest_factor(hipStream_t s, const Geom& g, const float* st, double* B, double* Binv);
 void launch_coarsest_solve(hipStream_t s, const Geom& g, const double* Binv, const float* f, float* u);
 
