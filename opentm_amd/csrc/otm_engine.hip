@@ -2079,6 +2079,7 @@ struct otm_mma {
   void* small = nullptr;
   MmaHost* mh = nullptr;       // coherent pinned block the finalisers publish to
   MmaHost* mh_dev = nullptr;   // its device address
+  unsigned mh_tag = 0;         // last tag published to it
   float* fx = nullptr;         // design, previous designs, gradients (FP32): (5 + m) n floats
   float* fbounds = nullptr;    // per-element bounds (2n floats), once set
   float* xout = nullptr;       // FP32 result staging for host callers
@@ -2213,7 +2214,7 @@ OTM_API int otm_mma_update(otm_mma* o, int itn, float* x, const float* dfdx, con
     hip_check(hipMemcpyAsync(o->gval, gval, sizeof(double) * o->m, hipMemcpyHostToDevice, o->s), "gval");
     float* xout = where == OTM_DEVICE ? x : o->xout;
     const int rc =
-        mma_update(o->s, o->m, o->A, o->small, o->mh, o->mh_dev, o->gval, itn, o->a0, o->a, o->c, o->d, xout,
+        mma_update(o->s, o->m, o->A, o->small, o->mh, o->mh_dev, o->mh_tag, o->gval, itn, o->a0, o->a, o->c, o->d, xout,
                    &o->prof);
     if (rc == -2) fail(OTM_E_NUMERIC, "MMA subsolver produced non-finite values");
     if (rc < 0) fail(OTM_E_HIP, "MMA update failed");

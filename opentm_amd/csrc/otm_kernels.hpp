@@ -208,18 +208,24 @@ struct MmaProf {
   std::vector<hipEvent_t> pool;
 };
 void mma_prof_release(MmaProf& P);
-// What the host loop of an MMA update needs after each point pass, in
-// coherent pinned host memory: the pass's finaliser writes it and then its
-// tag, and the host polls the tag (no copy, no stream synchronisation).
-struct MmaHost {
-  double residumax, rmaxnew, rmaxnext;
-  int accept, respec, fault;
+// What the host learns of each MMA pass, in coherent pinned host memory: the
+// kernel after the pass writes the slot of its tag and then the tag, and
+// the host polls it (no copy, no stream synchronisation).
+constexpr int kMmaSlots = 4;
+struct MmaHostSlot {
+  int kind;          // class of the pass (as MmaProf), -1: it had nothing to do
+  int done, newton;  // the subproblem is solved; Newton steps so far
+  int fault;
   unsigned seq;
+};
+struct MmaHost {
+  MmaHostSlot slot[kMmaSlots];
 };
 // One MMA update on device arrays; returns Newton steps or a negative code
 // (-1 HIP error, -2 non-finite values, -3 unsupported m). mh is the host
-// block (host address), mh_dev its device address.
-int mma_update(hipStream_t s, int m, MmaArrays& A, void* small_dev, MmaHost* mh, MmaHost* mh_dev,
+// block (host address), mh_dev its device address, tag the last tag used on
+// it.
+int mma_update(hipStream_t s, int m, MmaArrays& A, void* small_dev, MmaHost* mh, MmaHost* mh_dev, unsigned& tag,
                const double* gval_dev, int itn, double a0, double av, double cv, double dv, float* xout,
                MmaProf* prof = nullptr);
 void launch_f2d(hipStream_t s, long long n, const float* in, double* out);

@@ -12,19 +12,17 @@
 // reference casts both to FP64, which is exact) and the FP64 asymptotes, for
 // about 60 FP64 operations per element instead of 8 (4 + 2m) bytes of
 // reads. A pass reads 4 + 16 + 4 (1 + m) + 24 bytes per element (x, low and
-// upp, gradients, the interior point; per-element bounds add 8). Each Newton
-// step is two passes:
-//   dir:   the Newton direction dx from the small system's dlam and the
-//          fraction-to-boundary bound (dx is not stored);
-//   point: the trial point (dx recomputed by the same function as in dir,
-//          so the same bits), its KKT residual norm/max and, speculatively,
-//          the sums that build the Newton system at that point (gvec,
-//          GG.(delx/diagx), GG diag(1/diagx) GG^T). When the line search
-//          accepts the point these are the next step's system; when it
-//          rejects it they are dropped.
-// Each pass is followed by a one-block finaliser for the scalar logic (the
-// (m+1) solve by Gaussian elimination with partial pivoting, step length,
-// line-search bookkeeping) on the device. m is limited to kMmaMaxM.
+// upp, gradients, the interior point; per-element bounds add 8). Each line
+// search trial is one pass: it forms the trial point from the Newton
+// direction (recomputed in registers), its KKT residual norm/max and,
+// speculatively, the sums that build the Newton system at that point (gvec,
+// GG.(delx/diagx), GG diag(1/diagx) GG^T). When the line search accepts the
+// point these are the next step's system; when it rejects it they are
+// dropped.
+// Each pass is followed by a one-block kernel that carries the subsolver on
+// (k_mma_step): line search, barrier levels, and the (m+1) Newton solve of
+// the next pass, all on the device. The host only keeps a pass queued ahead
+// of the one it last saw finish. m is limited to kMmaMaxM.
 #include <math.h>
 
 #include <algorithm>
@@ -34,9 +32,19 @@
 
 namespace otm {
 
+// What the next pass has to do.
+enum MmaMode : int {
+  kMmaPoint = 0,  // residual and Newton sums at the start point of a barrier level
+  kMmaTrial = 1,  // a trial point of the line search
+  kMmaDone = 2    // the subproblem is solved (or has failed): nothing
+};
+
 struct MmaSmall {
   int m, itto;
-  int accept, fault;
+  int mode, par;       // MmaMode; par 1: the current point is in the trial buffers
+  int first, spec;     // first trial of its Newton step; ns_n holds the next level's start
+  int ittt, newton;    // Newton steps of this level, of the update
+  int fault, pad;
   double a0, epsi;
   double a[kMmaMaxM], b[kMmaMaxM], c[kMmaMaxM], d[kMmaMaxM];
   double y[kMmaMaxM], lam[kMmaMaxM], mu[kMmaMaxM], s[kMmaMaxM], z, zet;
@@ -44,7 +52,6 @@ struct MmaSmall {
   double yt[kMmaMaxM], lamt[kMmaMaxM], mut[kMmaMaxM], st[kMmaMaxM], zt, zett;
   double steg, stm_small;
   double lamtr[kMmaMaxM];  // lam + steg dlam of the next trial (uniform for its pass)
-  int respec;              // the last trial's step bound was wrong: run it again at steg
   double residunorm, residumax, resinew, rmaxnew;
   // Newton-system sums at the current point and at the trial point:
   // gvec[m], GG.(delx/diagx)[m], upper triangle of GG diag(1/diagx) GG^T
@@ -88,43 +95,27 @@ __device__ inline void block_sum_max(double (&s)[NS], double (&mx)[NM], double* 
   }
 }
 
-// One-block reduction of the value-major partials of nblocks blocks:
-// out[0..NS) sums (in block order per thread, then a fixed tree), out[NS..)
-// maxima.
-template <int NS, int NM>
-__device__ inline void final_sum_max(const double* partials, int nblocks, double* out) {
-  constexpr int NV = NS + NM;
-  __shared__ double sh[NV * kWaves];
-  double s[NV];
+// One-block reduction (kMmaStepThreads threads) of the value-major partials
+// of nblocks blocks into out: nsum sums, then nmax maxima. A wave takes a
+// value, its lanes a stride of the blocks with all their loads in flight,
+// then a fixed tree.
+constexpr int kMmaStepThreads = 1024;
+constexpr int kMmaValues = 32;  // partial-sum values of a pass, at most
+__device__ inline void mma_reduce(const double* __restrict__ partials, int nblocks, int nsum, int nmax, double* out) {
+  const int lane = threadIdx.x & 63;
+  for (int v = threadIdx.x >> 6; v < nsum + nmax; v += kMmaStepThreads / 64) {
+    const double* __restrict__ pv = partials + (size_t)v * nblocks;
+    const bool sum = v < nsum;
+    double r = sum ? 0.0 : -1e300;
+#pragma unroll 8
+    for (int b = lane; b < nblocks; b += 64) r = sum ? r + pv[b] : fmax(r, pv[b]);
+    if (sum) {
+      r = wave_sum(r);
+    } else {
 #pragma unroll
-  for (int i = 0; i < NS; i++) s[i] = 0.0;
-#pragma unroll
-  for (int i = 0; i < NM; i++) s[NS + i] = -1e300;
-  for (int b = threadIdx.x; b < nblocks; b += blockDim.x) {
-#pragma unroll
-    for (int i = 0; i < NS; i++) s[i] += partials[(size_t)i * nblocks + b];
-#pragma unroll
-    for (int i = 0; i < NM; i++) s[NS + i] = fmax(s[NS + i], partials[(size_t)(NS + i) * nblocks + b]);
-  }
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-  for (int i = 0; i < NS; i++) {
-    const double v = wave_sum(s[i]);
-    if (lane == 0) sh[i * kWaves + wid] = v;
-  }
-#pragma unroll
-  for (int i = NS; i < NV; i++) {
-    double v = s[i];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_down(v, o, 64));
-    if (lane == 0) sh[i * kWaves + wid] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < NV) {
-    const int i = threadIdx.x;
-    double v = i < NS ? 0.0 : -1e300;
-    for (int w = 0; w < kWaves; w++) v = i < NS ? v + sh[i * kWaves + w] : fmax(v, sh[i * kWaves + w]);
-    out[i] = v;
+      for (int o = 32; o > 0; o >>= 1) r = fmax(r, __shfl_xor(r, o, 64));
+    }
+    if (lane == 0) out[v] = r;
   }
   __syncthreads();
 }
@@ -328,10 +319,11 @@ __global__ void __launch_bounds__(kBlock) k_mma_prep(MmaArrays A, int itn) {
 }
 
 template <int M>
-__global__ void __launch_bounds__(kBlock) k_mma_prep_final(MmaArrays A, MmaSmall* S, const double* gval, int nblocks,
-                                                           double a0, double av, double cv, double dv) {
-  __shared__ double out[M + 1];
-  final_sum_max<M, 1>(A.partials, nblocks, out);
+__global__ void __launch_bounds__(kMmaStepThreads) k_mma_prep_final(MmaArrays A, MmaSmall* S, const double* gval,
+                                                                    int nblocks, double a0, double av, double cv,
+                                                                    double dv) {
+  __shared__ double out[kMmaValues];
+  mma_reduce(A.partials, nblocks, M, 0, out);
   if (threadIdx.x != 0) return;
   S->m = M;
   S->a0 = a0;
@@ -348,6 +340,12 @@ __global__ void __launch_bounds__(kBlock) k_mma_prep_final(MmaArrays A, MmaSmall
   }
   S->z = 1.0;
   S->zet = 1.0;
+  S->mode = kMmaPoint;
+  S->par = 0;
+  S->first = 0;
+  S->spec = 0;
+  S->ittt = 0;
+  S->newton = 0;
   S->fault = 0;
 }
 
@@ -386,19 +384,19 @@ struct MmaPointNV {
   static constexpr int NX = 1 + M;
 };
 static_assert(MmaPointNV<kMmaMaxM>::NN <= kMmaMaxNS, "Newton sums exceed their slots");
-static_assert(MmaPointNV<kMmaMaxM>::NS + MmaPointNV<kMmaMaxM>::NX + 2 <= 32, "point pass partials exceed their slots");
+static_assert(MmaPointNV<kMmaMaxM>::NS + MmaPointNV<kMmaMaxM>::NX + 3 <= kMmaValues, "point pass partials exceed their slots");
 
 // TRIAL: the point is the current one + steg * (Newton direction); the
 // direction is recomputed from the current point, the point written to the trial
-// buffers and the small-vector trial values are formed by the finaliser.
-// BOUND (the first trial of a Newton step): the step was taken as
-// 1 / stm_small, the bound of the small variables alone, and the pass also
-// forms the elements' fraction-to-boundary bound (mmaOpt.cu:700-716) as
-// its third maximum; the finaliser redoes the trial if that bound is the
-// larger one.
-template <int M, bool TRIAL, bool BOUND = false>
-__device__ inline void mma_point_body(MmaArrays& A, const MmaSmall* __restrict__ S) {
-  constexpr int NS = MmaPointNV<M>::NS, NX = TRIAL ? MmaPointNV<M>::NX : 0, NM = TRIAL ? (BOUND ? 3 : 2) : 1;
+// buffers and the small-vector trial values are formed by k_mma_step.
+// The first trial of a Newton step is taken at 1 / stm_small, the bound of
+// the small variables alone, and the pass also forms the elements'
+// fraction-to-boundary bound (mmaOpt.cu:700-716) as its third maximum; the
+// trial is redone if that bound is the larger one.
+template <int M, bool TRIAL>
+__device__ __forceinline__ void mma_point_body(MmaArrays& A, const MmaSmall* __restrict__ S) {
+  constexpr int NS = MmaPointNV<M>::NS, NX = TRIAL ? MmaPointNV<M>::NX : 0, NM = TRIAL ? 3 : 1;
+  const bool first = TRIAL && S->first;
   double lam[M], lamc[M], dlam[M];
   const double epsi = S->epsi, steg = S->steg;
   const double epsi2 = epsi * 0.1;  // the next level's, as k_mma_epsi forms it
@@ -414,7 +412,7 @@ __device__ inline void mma_point_body(MmaArrays& A, const MmaSmall* __restrict__
   double mx[NM];
 #pragma unroll
   for (int i = 0; i < NM; i++) mx[i] = 0.0;
-  if (BOUND) mx[NM - 1] = -1e300;
+  if (TRIAL) mx[NM - 1] = -1e300;
   mma_for_each<M>(A, [&](unsigned j, const MmaRaw<M>& r) {
     MmaElem<M> e;
     mma_elem<M>(A, r, e);
@@ -425,7 +423,7 @@ __device__ inline void mma_point_body(MmaArrays& A, const MmaSmall* __restrict__
       const double dx = mma_dx<M>(qc, dlam);
       const double dxsi = -xsi + epsi * qc.rxa - xsi * dx * qc.rxa;
       const double deta = -eta + epsi * qc.rbx + eta * dx * qc.rbx;
-      if (BOUND)
+      if (first)
         mx[NM - 1] = fmax(mx[NM - 1], fmax(fmax(-1.01 * dxsi * rcp64(xsi), -1.01 * deta * rcp64(eta)),
                                            fmax(-1.01 * dx * qc.rxa, 1.01 * dx * qc.rbx)));
       x += steg * dx;
@@ -469,180 +467,96 @@ __device__ inline void mma_point_body(MmaArrays& A, const MmaSmall* __restrict__
   block_sum_max<NS + NX, NM>(sums, mx, A.partials);
 }
 
-// The start-of-level point pass (up to m = 3) asks the compiler for five
-// waves per SIMD. The trial passes do not: in grid-stride order a trial
-// pass with that request (96 VGPRs, 1280 workgroups) took 282 us at 2^24
-// elements, without it (four waves, 1024 workgroups) 262 us; at m = 4 the
-// request would spill.
-template <int M, bool TRIAL, bool BOUND>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8)))
-k_mma_point(MmaArrays A, const MmaSmall* __restrict__ S) {
-  mma_point_body<M, TRIAL, BOUND>(A, S);
-}
-template <int M, bool TRIAL, bool BOUND>
-__global__ void __launch_bounds__(kBlock) k_mma_point_wide(MmaArrays A, const MmaSmall* __restrict__ S) {
-  mma_point_body<M, TRIAL, BOUND>(A, S);
-}
-template <int M, bool TRIAL, bool BOUND = false>
-static constexpr auto mma_point_kernel() {
-  if constexpr (M <= 3 && !BOUND && !TRIAL) return k_mma_point<M, TRIAL, BOUND>;
-  else return k_mma_point_wide<M, TRIAL, BOUND>;
-}
-
-// The host loop's inputs to the host block, then the tag (one thread).
-__device__ inline void mma_publish(const MmaSmall* S, MmaHost* mh, unsigned tag) {
-  mh->residumax = S->residumax;
-  mh->rmaxnew = S->rmaxnew;
-  mh->rmaxnext = S->rmaxn;
-  mh->accept = S->accept;
-  mh->respec = S->respec;
-  mh->fault = S->fault;
-  __hip_atomic_store(&mh->seq, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-template <int M, bool TRIAL, bool BOUND = false>
-__device__ inline void mma_point_final_body(MmaArrays& A, MmaSmall* S, int nblocks) {
-  constexpr int NS = MmaPointNV<M>::NS, NN = MmaPointNV<M>::NN;
-  constexpr int NX = TRIAL ? MmaPointNV<M>::NX : 0, NM = TRIAL ? (BOUND ? 3 : 2) : 1;
-  __shared__ double out[NS + NX + NM];
-  final_sum_max<NS + NX, NM>(A.partials, nblocks, out);
-  if (threadIdx.x != 0) return;
-  S->respec = 0;
-  if (BOUND) {
-    // step = 1 / max(stm_small, element bound) (mmaOpt.cu:700-716): when the
-    // elements bound it, the trial taken at 1 / stm_small is discarded and
-    // the line search starts at the right step
-    const double stm_elem = out[NS + NX + NM - 1];
-    if (stm_elem > S->stm_small) {
-      S->steg = 1.0 / fmax(S->stm_small, stm_elem);
-      for (int i = 0; i < M; i++) S->lamtr[i] = S->lam[i] + S->steg * S->dlam[i];
-      S->accept = 0;
-      S->respec = 1;
-      return;
-    }
-  }
-  double ss = out[0], mx = out[NS + NX];
-  double* ns = TRIAL ? S->ns_t : S->ns;
-  for (int i = 0; i < NN; i++) ns[i] = out[1 + i];
-  if (!TRIAL) {
-    small_residual(S, out + 1, S->y, S->z, S->lam, S->mu, S->zet, S->s, ss, mx, S->epsi);
-    S->residunorm = sqrt(ss);
-    S->residumax = mx;
-    return;
-  }
-  const double steg = S->steg;
-  for (int i = 0; i < M; i++) {
-    S->yt[i] = S->y[i] + steg * S->dy[i];
-    S->lamt[i] = S->lamtr[i];  // the multipliers the pass used
-    S->mut[i] = S->mu[i] + steg * S->dmu[i];
-    S->st[i] = S->s[i] + steg * S->ds[i];
-  }
-  S->zt = S->z + steg * S->dz;
-  S->zett = S->zet + steg * S->dzet;
-  small_residual(S, out + 1, S->yt, S->zt, S->lamt, S->mut, S->zett, S->st, ss, mx, S->epsi);
-  S->resinew = sqrt(ss);
-  S->rmaxnew = mx;
-  // the same point at the next barrier level (used if this trial ends the level)
-  const double epsi2 = S->epsi * 0.1;
-  double ss2 = out[NS], mx2 = out[NS + NX + 1];
-  for (int i = 0; i < NN; i++) S->ns_n[i] = out[1 + i];
-  for (int i = 0; i < M; i++) S->ns_n[M + i] = out[NS + 1 + i];
-  small_residual(S, out + 1, S->yt, S->zt, S->lamt, S->mut, S->zett, S->st, ss2, mx2, epsi2);
-  S->resn = sqrt(ss2);
-  S->rmaxn = mx2;
-  S->itto += 1;
-  // line search rule (mmaOpt.cu:718-805): accept when the norm does not
-  // grow, or after 50 halvings
-  S->accept = (!(S->resinew > S->residunorm) || S->itto >= 50) ? 1 : 0;
-  if (!(S->resinew - S->resinew == 0.0)) S->fault = 1;
-  S->steg = steg / 2;
-  for (int i = 0; i < M; i++) S->lamtr[i] = S->lam[i] + S->steg * S->dlam[i];
-}
-
-template <int M, bool TRIAL, bool BOUND>
-__global__ void __launch_bounds__(kBlock) k_mma_point_final(MmaArrays A, MmaSmall* S, int nblocks, MmaHost* mh,
-                                                            unsigned tag) {
-  mma_point_final_body<M, TRIAL, BOUND>(A, S, nblocks);
-  if (threadIdx.x == 0) mma_publish(S, mh, tag);
-}
-
-// After acceptance the trial becomes the current point, with its Newton
-// sums; done by the kernel that follows the accepted trial (the next Newton
-// system or the next barrier level).
-__device__ inline void mma_commit(MmaSmall* S) {
-  for (int i = 0; i < S->m; i++) {
-    S->y[i] = S->yt[i];
-    S->lam[i] = S->lamt[i];
-    S->mu[i] = S->mut[i];
-    S->s[i] = S->st[i];
-  }
-  for (int i = 0; i < kMmaMaxNS; i++) S->ns[i] = S->ns_t[i];
-  S->z = S->zt;
-  S->zet = S->zett;
-  S->residunorm = S->resinew;
-  S->residumax = S->rmaxnew;
-}
-
-// ---- Newton system ---------------------------------------------------------------
-// Solves [Alam a; a^T -zet/z] [dlam; dz] = [blam; delz] from the point's
-// sums and the small directions (mmaOpt.cu:595-678). One thread.
+// One pass over the design, as S asks. (No waves-per-EU request: in
+// grid-stride order a trial pass held to five waves per SIMD took 282 us at
+// 2^24 elements, with the compiler's four 262 us.)
 template <int M>
-__global__ void k_mma_newton_final(MmaSmall* S, int commit) {
-  if (commit) mma_commit(S);
+__global__ void __launch_bounds__(kBlock) k_mma_pass(MmaArrays A, const MmaSmall* __restrict__ S) {
+  const int mode = S->mode;
+  if (mode == kMmaDone) return;
+  if (S->par) {
+    double* t;
+    t = A.xs, A.xs = A.xs_t, A.xs_t = t;
+    t = A.xsi, A.xsi = A.xsi_t, A.xsi_t = t;
+    t = A.eta, A.eta = A.eta_t, A.eta_t = t;
+  }
+  if (mode == kMmaPoint)
+    mma_point_body<M, false>(A, S);
+  else
+    mma_point_body<M, true>(A, S);
+}
+
+// ---- the subsolver between two passes (one thread, S in LDS) -----------------
+// Newton system at the current point: solves [Alam a; a^T -zet/z] [dlam; dz]
+// = [blam; delz] from the point's sums, and the small directions
+// (mmaOpt.cu:595-678).
+template <int M>
+__device__ inline void mma_newton(MmaSmall* S) {
   const double epsi = S->epsi;
   const double* gvec = S->ns;
   const double* GGdd = S->ns + M;
-  double Alam[M][M];
-  int t = 2 * M;
-  for (int i = 0; i < M; i++)
-    for (int k = i; k < M; k++) {
-      Alam[i][k] = S->ns[t];
-      Alam[k][i] = S->ns[t];
-      t++;
-    }
   constexpr int K = M + 1;
   double AA[K][K], bb[K];
+  int t = 2 * M;
+#pragma unroll
+  for (int i = 0; i < M; i++)
+#pragma unroll
+    for (int k = i; k < M; k++) {
+      AA[i][k] = S->ns[t];
+      AA[k][i] = S->ns[t];
+      t++;
+    }
   double alam = 0.0;
+#pragma unroll
   for (int i = 0; i < M; i++) alam += S->a[i] * S->lam[i];
+#pragma unroll
   for (int i = 0; i < M; i++) {
     const double dely = S->c[i] + S->d[i] * S->y[i] - S->lam[i] - epsi / S->y[i];
     const double dellam = gvec[i] - S->a[i] * S->z - S->y[i] - S->b[i] + epsi / S->lam[i];
     const double diagy = S->d[i] + S->mu[i] / S->y[i];
     const double diaglamyi = S->s[i] / S->lam[i] + 1.0 / diagy;
     bb[i] = dellam + dely / diagy - GGdd[i];
-    for (int k = 0; k < M; k++) AA[i][k] = Alam[i][k] + (i == k ? diaglamyi : 0.0);
+    AA[i][i] += diaglamyi;
     AA[i][M] = S->a[i];
     AA[M][i] = S->a[i];
   }
   AA[M][M] = -S->zet / S->z;
   bb[M] = S->a0 - alam - epsi / S->z;
-  // Gaussian elimination with partial pivoting
+  // Gaussian elimination with partial pivoting; the pivot row is brought up
+  // by conditional exchanges, so every index is static and the system stays
+  // in registers
+#pragma unroll
   for (int c = 0; c < K; c++) {
-    int p = c;
-    for (int r = c + 1; r < K; r++)
-      if (fabs(AA[r][c]) > fabs(AA[p][c])) p = r;
-    if (p != c) {
+#pragma unroll
+    for (int r = c + 1; r < K; r++) {
+      const bool sw = fabs(AA[r][c]) > fabs(AA[c][c]);
+#pragma unroll
       for (int j = 0; j < K; j++) {
-        const double tmp = AA[c][j];
-        AA[c][j] = AA[p][j];
-        AA[p][j] = tmp;
+        const double u = AA[c][j], v = AA[r][j];
+        AA[c][j] = sw ? v : u;
+        AA[r][j] = sw ? u : v;
       }
-      const double tmp = bb[c];
-      bb[c] = bb[p];
-      bb[p] = tmp;
+      const double u = bb[c], v = bb[r];
+      bb[c] = sw ? v : u;
+      bb[r] = sw ? u : v;
     }
+#pragma unroll
     for (int r = c + 1; r < K; r++) {
       const double f = AA[r][c] / AA[c][c];
+#pragma unroll
       for (int j = c; j < K; j++) AA[r][j] -= f * AA[c][j];
       bb[r] -= f * bb[c];
     }
   }
+#pragma unroll
   for (int r = K - 1; r >= 0; r--) {
     double sacc = bb[r];
+#pragma unroll
     for (int j = r + 1; j < K; j++) sacc -= AA[r][j] * bb[j];
     bb[r] = sacc / AA[r][r];
   }
   double stm = 1.0;
+#pragma unroll
   for (int i = 0; i < M; i++) {
     const double dlam = bb[i];
     const double dely = S->c[i] + S->d[i] * S->y[i] - S->lam[i] - epsi / S->y[i];
@@ -665,31 +579,171 @@ __global__ void k_mma_newton_final(MmaSmall* S, int commit) {
   S->stm_small = stm;
   if (!(stm - stm == 0.0)) S->fault = 1;
   // the first trial takes the small variables' step; its pass forms the
-  // elements' bound and the finaliser redoes it if that one is larger
+  // elements' bound and the trial is redone if that one is larger
   S->steg = 1.0 / stm;
+#pragma unroll
   for (int i = 0; i < M; i++) S->lamtr[i] = S->lam[i] + S->steg * S->dlam[i];
   S->itto = 0;
-  S->accept = 0;
 }
 
-__global__ void k_mma_epsi(MmaSmall* S, int commit, int spec) {
-  if (commit) mma_commit(S);
-  S->epsi *= 0.1;
-  if (spec) {
-    for (int i = 0; i < kMmaMaxNS; i++) S->ns[i] = S->ns_n[i];
+// A start-of-level pass: the residual at the current point.
+template <int M>
+__device__ inline void mma_take_point(MmaSmall* S, const double* out) {
+  constexpr int NS = MmaPointNV<M>::NS, NN = MmaPointNV<M>::NN;
+  double ss = out[0], mx = out[NS];
+  for (int i = 0; i < NN; i++) S->ns[i] = out[1 + i];
+  small_residual(S, out + 1, S->y, S->z, S->lam, S->mu, S->zet, S->s, ss, mx, S->epsi);
+  S->residunorm = sqrt(ss);
+  S->residumax = mx;
+}
+
+// A trial pass: returns whether the line search accepts it. If not, the next
+// trial's step is set.
+template <int M>
+__device__ inline bool mma_take_trial(MmaSmall* S, const double* out) {
+  constexpr int NS = MmaPointNV<M>::NS, NN = MmaPointNV<M>::NN, NX = MmaPointNV<M>::NX;
+  if (S->first) {
+    S->first = 0;
+    // step = 1 / max(stm_small, element bound) (mmaOpt.cu:700-716): when the
+    // elements bound it, the trial taken at 1 / stm_small is discarded and
+    // the line search starts at the right step
+    const double stm_elem = out[NS + NX + 2];
+    if (stm_elem > S->stm_small) {
+      S->steg = 1.0 / fmax(S->stm_small, stm_elem);
+      for (int i = 0; i < M; i++) S->lamtr[i] = S->lam[i] + S->steg * S->dlam[i];
+      return false;
+    }
+  }
+  double ss = out[0], mx = out[NS + NX];
+  const double steg = S->steg;
+  for (int i = 0; i < M; i++) {
+    S->yt[i] = S->y[i] + steg * S->dy[i];
+    S->lamt[i] = S->lamtr[i];  // the multipliers the pass used
+    S->mut[i] = S->mu[i] + steg * S->dmu[i];
+    S->st[i] = S->s[i] + steg * S->ds[i];
+  }
+  S->zt = S->z + steg * S->dz;
+  S->zett = S->zet + steg * S->dzet;
+  small_residual(S, out + 1, S->yt, S->zt, S->lamt, S->mut, S->zett, S->st, ss, mx, S->epsi);
+  const double resinew = sqrt(ss);
+  S->itto += 1;
+  if (!(resinew - resinew == 0.0)) S->fault = 1;
+  // line search rule (mmaOpt.cu:718-805): accept when the norm does not
+  // grow, or after 50 halvings
+  if (resinew > S->residunorm && S->itto < 50) {
+    S->steg = steg / 2;
+    for (int i = 0; i < M; i++) S->lamtr[i] = S->lam[i] + S->steg * S->dlam[i];
+    return false;
+  }
+  // the trial is the current point, with its Newton sums here and at the
+  // next barrier level
+  const double epsi2 = S->epsi * 0.1;
+  double ss2 = out[NS], mx2 = out[NS + NX + 1];
+  for (int i = 0; i < NN; i++) S->ns[i] = S->ns_n[i] = out[1 + i];
+  for (int i = 0; i < M; i++) S->ns_n[M + i] = out[NS + 1 + i];
+  small_residual(S, out + 1, S->yt, S->zt, S->lamt, S->mut, S->zett, S->st, ss2, mx2, epsi2);
+  S->resn = sqrt(ss2);
+  S->rmaxn = mx2;
+  S->spec = 1;
+  for (int i = 0; i < M; i++) {
+    S->y[i] = S->yt[i];
+    S->lam[i] = S->lamt[i];
+    S->mu[i] = S->mut[i];
+    S->s[i] = S->st[i];
+  }
+  S->z = S->zt;
+  S->zet = S->zett;
+  S->residunorm = resinew;
+  S->residumax = mx;
+  S->par ^= 1;
+  return true;
+}
+
+// From the current point to the next pass: a Newton step of this barrier
+// level, or the next level (whose start an accepted trial has already
+// summed; otherwise a point pass), or the end.
+template <int M>
+__device__ inline void mma_advance(MmaSmall* S, double epsimin) {
+  while (true) {
+    if (S->residumax > 0.9 * S->epsi && S->ittt < 200) {
+      S->ittt++;
+      S->newton++;
+      mma_newton<M>(S);
+      S->mode = kMmaTrial;
+      S->first = 1;
+      return;
+    }
+    S->epsi *= 0.1;
+    S->ittt = 0;
+    if (!(S->epsi > epsimin)) {
+      S->mode = kMmaDone;
+      return;
+    }
+    if (!S->spec) {
+      S->mode = kMmaPoint;
+      return;
+    }
+    S->spec = 0;
+    for (int i = 0; i < MmaPointNV<M>::NN; i++) S->ns[i] = S->ns_n[i];
     S->residunorm = S->resn;
     S->residumax = S->rmaxn;
   }
 }
 
+// After each pass: its sums, the subsolver's logic, and the host's slot.
+// Bound by latency (one block): the partials are summed a wave per value and
+// the state lives in LDS. 4.4 us at m = 1 with 128 blocks, 8.1 us at m = 2
+// with 1024, where a finaliser (4.9 and 8.1), a Newton kernel (2.3 and 3.9)
+// and a host round trip with its launches (about 18) stood between two
+// passes before.
+template <int M>
+__global__ void __launch_bounds__(kMmaStepThreads) k_mma_step(const double* __restrict__ partials, int nblocks,
+                                                              MmaSmall* Sg, double epsimin, MmaHost* mh,
+                                                              unsigned tag) {
+  __shared__ MmaSmall S;
+  __shared__ double out[kMmaValues];
+  constexpr int kWords = sizeof(MmaSmall) / sizeof(unsigned);
+  static_assert(kWords <= kMmaStepThreads, "state copied in one go");
+  if (threadIdx.x < kWords) ((unsigned*)&S)[threadIdx.x] = ((const unsigned*)Sg)[threadIdx.x];
+  __syncthreads();
+  const int mode = S.mode;
+  const bool first = S.first;
+  if (mode != kMmaDone) {
+    constexpr int NS = MmaPointNV<M>::NS, NX = MmaPointNV<M>::NX;
+    if (mode == kMmaPoint)
+      mma_reduce(partials, nblocks, NS, 1, out);
+    else
+      mma_reduce(partials, nblocks, NS + NX, 3, out);
+    if (threadIdx.x == 0) {
+      bool next = true;
+      if (mode == kMmaPoint)
+        mma_take_point<M>(&S, out);
+      else
+        next = mma_take_trial<M>(&S, out);
+      if (next && !S.fault) mma_advance<M>(&S, epsimin);
+      if (S.fault) S.mode = kMmaDone;
+    }
+    __syncthreads();
+    if (threadIdx.x < kWords) ((unsigned*)Sg)[threadIdx.x] = ((const unsigned*)&S)[threadIdx.x];
+  }
+  if (threadIdx.x == 0) {
+    MmaHostSlot* slot = &mh->slot[tag % kMmaSlots];
+    slot->kind = mode == kMmaDone ? -1 : (mode == kMmaPoint ? 2 : (first ? 1 : 0));
+    slot->done = S.mode == kMmaDone;
+    slot->newton = S.newton;
+    slot->fault = S.fault;
+    __hip_atomic_store(&slot->seq, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 // xold2 = xold1, xold1 = x (mmaOpt.cu:1055-1057); the subsolver solution
 // goes to the caller's FP32 design
-__global__ void __launch_bounds__(kBlock) k_mma_finish(MmaArrays A, float* xout) {
+__global__ void __launch_bounds__(kBlock) k_mma_finish(MmaArrays A, const MmaSmall* __restrict__ S, float* xout) {
   const long long j = stid();
   if (j >= A.n) return;
   A.xold2[j] = A.xold1[j];
   A.xold1[j] = A.xvar[j];
-  xout[j] = (float)A.xs[j];
+  xout[j] = (float)(S->par ? A.xs_t[j] : A.xs[j]);
 }
 
 // ---- host driver ---------------------------------------------------------------
@@ -703,20 +757,22 @@ static hipEvent_t prof_event(MmaProf& P) {
   if (hipEventCreate(&e) != hipSuccess) return nullptr;
   return e;
 }
-// events of finished launches -> per-class time (after a stream sync)
-static void prof_collect(MmaProf& P) {
-  for (const auto& q : P.pending) {
-    float ms = 0.f;
-    if (hipEventSynchronize(q.b) == hipSuccess && hipEventElapsedTime(&ms, q.a, q.b) == hipSuccess) P.ms[q.cls] += ms;
-    P.pool.push_back(q.a);
-    P.pool.push_back(q.b);
+// a finished pass's events -> its class's time
+static void prof_take(MmaProf& P, const MmaProf::Pending& q, int cls, const double* bytes_of) {
+  float ms = 0.f;
+  if (cls >= 0 && q.a && q.b && hipEventSynchronize(q.b) == hipSuccess &&
+      hipEventElapsedTime(&ms, q.a, q.b) == hipSuccess) {
+    P.launches[cls]++;
+    P.bytes[cls] += bytes_of[cls];
+    P.ms[cls] += ms;
   }
-  P.pending.clear();
+  if (q.a) P.pool.push_back(q.a);
+  if (q.b) P.pool.push_back(q.b);
 }
 void mma_prof_release(MmaProf& P) {
   for (const auto& q : P.pending) {
-    P.pool.push_back(q.a);
-    P.pool.push_back(q.b);
+    if (q.a) P.pool.push_back(q.a);
+    if (q.b) P.pool.push_back(q.b);
   }
   P.pending.clear();
   for (hipEvent_t e : P.pool) (void)hipEventDestroy(e);
@@ -741,14 +797,14 @@ static unsigned mma_grid(K kernel, long long n) {
   return (unsigned)std::max<long long>(b, 1);
 }
 
-// Polls the host block for a tag; -1 when the stream finished without it
-// or failed.
-static int mma_wait(hipStream_t s, const MmaHost* mh, unsigned tag) {
+// Polls a host slot for a tag; -1 when the stream finished without it or
+// failed.
+static int mma_wait(hipStream_t s, const MmaHostSlot* slot, unsigned tag) {
   unsigned spins = 0;
-  while (__atomic_load_n(&mh->seq, __ATOMIC_ACQUIRE) != tag) {
+  while (__atomic_load_n(&slot->seq, __ATOMIC_ACQUIRE) != tag) {
     if ((++spins & 255u) == 0) {
       const hipError_t e = hipStreamQuery(s);
-      if (e == hipSuccess) return __atomic_load_n(&mh->seq, __ATOMIC_ACQUIRE) == tag ? 0 : -1;
+      if (e == hipSuccess) return __atomic_load_n(&slot->seq, __ATOMIC_ACQUIRE) == tag ? 0 : -1;
       if (e != hipErrorNotReady) return -1;
     }
     __builtin_ia32_pause();
@@ -756,130 +812,77 @@ static int mma_wait(hipStream_t s, const MmaHost* mh, unsigned tag) {
   return 0;
 }
 
+// Passes queued beyond the last one the host saw finish: one runs while the
+// host queues the next, so the device never waits for the host, and at most
+// one finds nothing left to do.
+constexpr int kMmaAhead = 2;
+static_assert(kMmaAhead < kMmaSlots, "a slot is read before it is written again");
+
 template <int M>
-static int mma_run(hipStream_t s, MmaArrays A, MmaSmall* S, MmaHost* mh, MmaHost* mh_dev, const double* gval_dev,
-                   int itn, double a0, double av, double cv, double dv, float* xout, double epsimin, MmaProf* prof) {
+static int mma_run(hipStream_t s, MmaArrays A, MmaSmall* S, MmaHost* mh, MmaHost* mh_dev, unsigned& tag,
+                   const double* gval_dev, int itn, double a0, double av, double cv, double dv, float* xout,
+                   double epsimin, MmaProf* prof) {
   const unsigned nb_prep = mma_grid(k_mma_prep<M>, A.n);
-  const unsigned nb_point = mma_grid(mma_point_kernel<M, false>(), A.n);
-  const unsigned nb_trial = mma_grid(mma_point_kernel<M, true>(), A.n);
-  const unsigned nb_bound = mma_grid(mma_point_kernel<M, true, true>(), A.n);
-  // no kernel of this optimiser is in flight: the block holds the last tag
-  unsigned tag = __atomic_load_n(&mh->seq, __ATOMIC_ACQUIRE);
-  auto read = [&]() -> int {
-    if (mma_wait(s, mh, tag) != 0) return -1;
-    if (prof && prof->on) prof_collect(*prof);
-    return mh->fault ? -2 : 0;
-  };
+  const unsigned nb = mma_grid(k_mma_pass<M>, A.n);
   // algorithmic bytes per element: x, low/upp, gradients, interior point
   // (+ per-element bounds), and the trial point written
   const double rd = 4.0 + 16.0 + 4.0 * (1 + M) + 24.0 + (A.xmin ? 8.0 : 0.0);
   const double bytes_of[3] = {(rd + 24.0) * (double)A.n, (rd + 24.0) * (double)A.n, rd * (double)A.n};
-  struct Timed {
-    MmaProf* P;
-    int cls;
-    hipStream_t s;
-    hipEvent_t a = nullptr;
-    Timed(MmaProf* P_, int cls_, hipStream_t s_, const double* by) : P(P_), cls(cls_), s(s_) {
-      if (!P || !P->on) return;
-      a = prof_event(*P);
-      if (a && hipEventRecord(a, s) != hipSuccess) a = nullptr;
-      if (a) {
-        P->launches[cls]++;
-        P->bytes[cls] += by[cls];
-      }
-    }
-    ~Timed() {
-      if (!a) return;
-      hipEvent_t b = prof_event(*P);
-      if (b && hipEventRecord(b, s) == hipSuccess)
-        P->pending.push_back({cls, a, b});
-      else
-        P->pool.push_back(a);
-    }
-  };
+  const bool timed = prof && prof->on;
   hipLaunchKernelGGL(k_mma_prep<M>, dim3(nb_prep), dim3(kBlock), 0, s, A, itn);
-  hipLaunchKernelGGL(k_mma_prep_final<M>, dim3(1), dim3(kBlock), 0, s, A, S, gval_dev, (int)nb_prep, a0, av, cv,
-                     dv);
-  int newton = 0;
-  double epsi = 1.0;
-  int commit = 0;   // an accepted trial waits to become the current point
-  bool spec = false;  // that trial's sums at this level are known (its pass formed them)
-  double residumax_next = 0.0;
-  while (epsi > epsimin) {
-    double residumax;
-    if (spec) {
-      residumax = residumax_next;
-    } else {
-      // residual and Newton system at the start point of this epsi level
-      {
-        Timed t(prof, 2, s, bytes_of);
-        hipLaunchKernelGGL((mma_point_kernel<M, false>()), dim3(nb_point), dim3(kBlock), 0, s, A, S);
-      }
-      hipLaunchKernelGGL((k_mma_point_final<M, false, false>), dim3(1), dim3(kBlock), 0, s, A, S, (int)nb_point,
-                         mh_dev, ++tag);
-      const int rc = read();
-      if (rc) return rc;
-      residumax = mh->residumax;
+  hipLaunchKernelGGL(k_mma_prep_final<M>, dim3(1), dim3(kMmaStepThreads), 0, s, A, S, gval_dev, (int)nb_prep, a0, av,
+                     cv, dv);
+  auto queue = [&] {
+    MmaProf::Pending q{0, nullptr, nullptr};
+    if (timed && (q.a = prof_event(*prof))) (void)hipEventRecord(q.a, s);
+    hipLaunchKernelGGL(k_mma_pass<M>, dim3(nb), dim3(kBlock), 0, s, A, S);
+    if (timed && (q.b = prof_event(*prof))) (void)hipEventRecord(q.b, s);
+    if (timed) prof->pending.push_back(q);
+    hipLaunchKernelGGL(k_mma_step<M>, dim3(1), dim3(kMmaStepThreads), 0, s, A.partials, (int)nb, S, epsimin, mh_dev,
+                       ++tag);
+  };
+  unsigned seen = tag;  // last pass whose slot was read
+  int rc = 0;
+  while (true) {
+    while ((int)(tag - seen) < kMmaAhead) queue();
+    const MmaHostSlot* slot = &mh->slot[++seen % kMmaSlots];
+    if (mma_wait(s, slot, seen) != 0) {
+      rc = -1;
+      break;
     }
-    spec = false;
-    int rc = 0;
-    int ittt = 0;
-    while (residumax > 0.9 * epsi && ittt < 200) {
-      ittt++;
-      newton++;
-      hipLaunchKernelGGL(k_mma_newton_final<M>, dim3(1), dim3(1), 0, s, S, commit);
-      commit = 0;
-      // line search; the first trial also checks the step it was given
-      bool first = true;
-      do {
-        {
-          Timed t(prof, first ? 1 : 0, s, bytes_of);
-          if (first)
-            hipLaunchKernelGGL((mma_point_kernel<M, true, true>()), dim3(nb_bound), dim3(kBlock), 0, s, A, S);
-          else
-            hipLaunchKernelGGL((mma_point_kernel<M, true>()), dim3(nb_trial), dim3(kBlock), 0, s, A, S);
-        }
-        if (first)
-          hipLaunchKernelGGL((k_mma_point_final<M, true, true>), dim3(1), dim3(kBlock), 0, s, A, S, (int)nb_bound,
-                             mh_dev, ++tag);
-        else
-          hipLaunchKernelGGL((k_mma_point_final<M, true, false>), dim3(1), dim3(kBlock), 0, s, A, S, (int)nb_trial,
-                             mh_dev, ++tag);
-        first = false;
-        rc = read();
-        if (rc) return rc;
-      } while (!mh->accept);
-      commit = 1;
-      std::swap(A.xs, A.xs_t);
-      std::swap(A.xsi, A.xsi_t);
-      std::swap(A.eta, A.eta_t);
-      residumax = mh->rmaxnew;
-      residumax_next = mh->rmaxnext;
-      spec = true;
+    if (timed) {
+      prof_take(*prof, prof->pending.front(), slot->kind, bytes_of);
+      prof->pending.erase(prof->pending.begin());
     }
-    hipLaunchKernelGGL(k_mma_epsi, dim3(1), dim3(1), 0, s, S, commit, spec ? 1 : 0);
-    commit = 0;
-    epsi *= 0.1;
+    if (slot->done) {
+      rc = slot->fault ? -2 : slot->newton;
+      break;
+    }
   }
-  hipLaunchKernelGGL(k_mma_finish, dim3(nblk(A.n)), dim3(kBlock), 0, s, A, xout);
+  if (timed) {  // what was queued past the end
+    for (const auto& q : prof->pending) prof_take(*prof, q, -1, bytes_of);
+    prof->pending.clear();
+  }
+  if (rc < 0) {
+    (void)hipStreamSynchronize(s);
+    return rc;
+  }
+  hipLaunchKernelGGL(k_mma_finish, dim3(nblk(A.n)), dim3(kBlock), 0, s, A, S, xout);
   if (hipGetLastError() != hipSuccess) return -1;
-  return newton;
+  return rc;
 }
 
-int mma_update(hipStream_t s, int m, MmaArrays& A, void* small_dev, MmaHost* mh, MmaHost* mh_dev,
+int mma_update(hipStream_t s, int m, MmaArrays& A, void* small_dev, MmaHost* mh, MmaHost* mh_dev, unsigned& tag,
                const double* gval_dev, int itn, double a0, double av, double cv, double dv, float* xout,
                MmaProf* prof) {
   MmaSmall* S = (MmaSmall*)small_dev;
-  MmaArrays B = A;  // the driver swaps the subsolver buffers locally
-  int rc;
   switch (m) {
-    case 1: rc = mma_run<1>(s, B, S, mh, mh_dev, gval_dev, itn, a0, av, cv, dv, xout, 1e-7, prof); break;
-    case 2: rc = mma_run<2>(s, B, S, mh, mh_dev, gval_dev, itn, a0, av, cv, dv, xout, 1e-7, prof); break;
-    case 3: rc = mma_run<3>(s, B, S, mh, mh_dev, gval_dev, itn, a0, av, cv, dv, xout, 1e-7, prof); break;
-    case 4: rc = mma_run<4>(s, B, S, mh, mh_dev, gval_dev, itn, a0, av, cv, dv, xout, 1e-7, prof); break;
-    default: rc = -3;
+    case 1: return mma_run<1>(s, A, S, mh, mh_dev, tag, gval_dev, itn, a0, av, cv, dv, xout, 1e-7, prof);
+    case 2: return mma_run<2>(s, A, S, mh, mh_dev, tag, gval_dev, itn, a0, av, cv, dv, xout, 1e-7, prof);
+    case 3: return mma_run<3>(s, A, S, mh, mh_dev, tag, gval_dev, itn, a0, av, cv, dv, xout, 1e-7, prof);
+    case 4: return mma_run<4>(s, A, S, mh, mh_dev, tag, gval_dev, itn, a0, av, cv, dv, xout, 1e-7, prof);
+    default: return -3;
   }
-  return rc;
 }
 
 size_t mma_small_bytes() { return sizeof(MmaSmall); }
