@@ -145,16 +145,16 @@ kb_fine_brick(const Ent* __restrict__ ents, int nents, const CellDev* __restrict
 }
 
 // ---- operations (one functor per batched launch) ---------------------------
+template <int FORM, int NR>
 struct OpStBrick {
-  static constexpr int kThreads = kBrickThreads;
+  static constexpr int kThreads = kStBrickThreads;
+  static constexpr int kParts = OTM_NRHS / NR;  // workgroups of a brick
   int l, post;
   __device__ void operator()(const CellDev& C, const Ent& e, int lb, int) const {
     const float* uin = post ? ucur(C, e.par, l) : nullptr;
     float* uout = post ? uoth(C, e.par, l) : ucur(C, e.par, l);
-    if (C.st[l].f16)
-      st_brick_body<true>(C.g[l], C.st[l], C.f[l], uin, uout, C.sweeps_coarse, post ? 0 : 1, post ? 0 : 1, lb);
-    else
-      st_brick_body<false>(C.g[l], C.st[l], C.f[l], uin, uout, C.sweeps_coarse, post ? 0 : 1, post ? 0 : 1, lb);
+    st_brick_body<FORM, NR>(C.g[l], C.st[l], C.f[l], uin, uout, C.sweeps_coarse, post ? 0 : 1, post ? 0 : 1,
+                            lb / kParts, (lb % kParts) * NR);
   }
 };
 
@@ -666,6 +666,27 @@ long long residb(const Member& m) {
 }
 long long one(const Member&) { return 1; }
 
+// Brick smoothing of level l, the cells with FP32 and with FP16 stencils
+// apart (each form has its own registers), split by load case up to
+// kStOneMax bricks in the launch.
+template <int FORM>
+void add_st_brick(otm_batch* b, const std::vector<Member*>& set, int l, int post) {
+  long long bricks = 0;
+  for (Member* m : set) bricks += brick_count(m->c->lv[l].g);
+  if (bricks <= kStOneMax)
+    add_op(b, set, OpStBrick<FORM == kStPacked ? kStWide : FORM, 1>{l, post},
+           [l](const Member& m) { return (long long)OTM_NRHS * brick_count(m.c->lv[l].g); });
+  else
+    add_op(b, set, OpStBrick<FORM, OTM_NRHS>{l, post},
+           [l](const Member& m) { return (long long)brick_count(m.c->lv[l].g); });
+}
+void plan_st_brick(otm_batch* b, const std::vector<Member*>& set, int l, int post) {
+  std::vector<Member*> f32, f16;
+  for (Member* m : set) (m->c->lv[l].st16 ? f16 : f32).push_back(m);
+  add_st_brick<kStFp32>(b, f32, l, post);
+  add_st_brick<kStPacked>(b, f16, l, post);
+}
+
 // V-cycle for the member set V (all levels, every member at its own depth).
 void plan_vcycle(otm_batch* b, std::vector<Member*>& V) {
   // levels above each member's tail run as separate launches (all members
@@ -708,7 +729,7 @@ void plan_vcycle(otm_batch* b, std::vector<Member*>& V) {
       }
       add_op(b, S, OpFineResid{}, residb);
     } else {
-      add_op(b, S, OpStBrick{l, 0}, [l](const Member& m) { return (long long)brick_count(m.c->lv[l].g); });
+      plan_st_brick(b, S, l, 0);
       add_op(b, S, OpStResid{l}, [l](const Member& m) {
         const Level& L = m.c->lv[l];
         return (long long)nblk(st_resid8(L.g, L.st16 != nullptr) ? 8 * L.g.nn : L.g.nn);
@@ -754,7 +775,7 @@ void plan_vcycle(otm_batch* b, std::vector<Member*>& V) {
             add_op(b, col, OpFineGsColor{cc & 1, cc >> 1},
                    [](const Member& m) { return (long long)nblk(m.c->g0.nx * (m.c->g0.ny / 2) * (m.c->g0.nz / 2)); });
     } else {
-      add_op(b, S, OpStBrick{l, 1}, [l](const Member& m) { return (long long)brick_count(m.c->lv[l].g); });
+      plan_st_brick(b, S, l, 1);
       for (Member* m : S) m->par ^= (1 << l);
     }
   }

@@ -107,12 +107,17 @@ __global__ void __launch_bounds__(kBlock) k_coarsest_rows(Geom g, const double* 
   coarsest_rows_body(g, Binv, f, u, blockIdx.x);
 }
 
-template <bool HALF>
-__global__ void __launch_bounds__(kBrickThreads) k_st_smooth_brick(Geom g, StRef S, const float* __restrict__ f,
-                                                                   const float* __restrict__ uin,
-                                                                   float* __restrict__ uout, int sweeps,
-                                                                   int forward, int zero_in) {
-  st_brick_body<HALF>(g, S, f, uin, uout, sweeps, forward, zero_in, xcd_block());
+// One brick and NR load cases per workgroup. The waves-per-EU requests are
+// what each form's registers allow without scratch memory (FP32 couplings
+// held to four waves spill: 13.1 -> 20.3 us at 64^3).
+template <int FORM, int NR>
+__global__ void __launch_bounds__(kStBrickThreads)
+    __attribute__((amdgpu_waves_per_eu(NR == OTM_NRHS && FORM != kStPacked ? 3 : 5, 8)))
+k_st_smooth_brick(Geom g, StRef S, const float* __restrict__ f, const float* __restrict__ uin,
+                  float* __restrict__ uout, int sweeps, int forward, int zero_in) {
+  constexpr int kParts = OTM_NRHS / NR;
+  const int b = xcd_block();
+  st_brick_body<FORM, NR>(g, S, f, uin, uout, sweeps, forward, zero_in, b / kParts, (b % kParts) * NR);
 }
 
 __global__ void __launch_bounds__(kTailThreads) k_tail_vcycle(TailLevels T) { tail_vcycle_body(T); }
@@ -178,12 +183,11 @@ bool brick_ok(const Geom& g) { return g.nx >= 2 && g.ny >= 2 && g.nz >= 2; }
 void launch_st_smooth_brick(hipStream_t s, const Geom& g, const StRef& S, const float* f, const float* uin,
                             float* uout, int sweeps, bool forward, bool zero_in) {
   const unsigned nb = (unsigned)brick_count(g);
-  if (S.f16)
-    hipLaunchKernelGGL(k_st_smooth_brick<true>, dim3(nb), dim3(kBrickThreads), 0, s, g, S, f, uin, uout, sweeps,
-                       forward ? 1 : 0, zero_in ? 1 : 0);
-  else
-    hipLaunchKernelGGL(k_st_smooth_brick<false>, dim3(nb), dim3(kBrickThreads), 0, s, g, S, f, uin, uout, sweeps,
-                       forward ? 1 : 0, zero_in ? 1 : 0);
+  const bool one = nb <= (unsigned)kStOneMax;
+  const auto k = S.f16 ? (one ? k_st_smooth_brick<kStWide, 1> : k_st_smooth_brick<kStPacked, OTM_NRHS>)
+                       : (one ? k_st_smooth_brick<kStFp32, 1> : k_st_smooth_brick<kStFp32, OTM_NRHS>);
+  hipLaunchKernelGGL(k, dim3(one ? OTM_NRHS * nb : nb), dim3(kStBrickThreads), 0, s, g, S, f, uin, uout, sweeps,
+                     forward ? 1 : 0, zero_in ? 1 : 0);
 }
 void launch_coarsest_solve(hipStream_t s, const Geom& g, const double* Binv, const float* f, float* u) {
   hipLaunchKernelGGL(k_coarsest_rows, dim3((unsigned)coarsest_row_blocks(g)), dim3(kBlock), 0, s, g, Binv, f, u);

@@ -383,174 +383,293 @@ __device__ inline void coarsest_rows_body(const Geom& g, const double* __restric
   }
 }
 
-// Brick smoother for stored-stencil levels. One 512-thread workgroup owns an
-// 8^3 brick (cut at the level's edge when an edge is not a multiple of 8):
-// its nodes' stencils sit in registers, u of the brick plus a one-node halo
-// sits in LDS. All colours of `sweeps` Gauss-Seidel sweeps run inside the
-// brick with workgroup barriers; halo values stay frozen at their values on
-// entry (block Gauss-Seidel across bricks, exact multicolour Gauss-Seidel
-// inside; a level smaller than a brick is smoothed exactly except across
-// its periodic seam). The result goes to a second buffer so bricks never
-// read a neighbour's new values. The post-smoother runs the colours in
-// reverse order, which is the adjoint of the pre-smoother: the V-cycle
-// stays symmetric.
+// Brick smoother for stored-stencil levels. One workgroup owns an 8^3 brick
+// (cut at the level's edge when an edge is not a multiple of 8): u of the
+// brick plus a one-node halo sits in LDS. All colours of `sweeps`
+// Gauss-Seidel sweeps run inside the brick with workgroup barriers; halo
+// values stay frozen at their values on entry (block Gauss-Seidel across
+// bricks, exact multicolour Gauss-Seidel inside; a level smaller than a
+// brick is smoothed exactly except across its periodic seam). The result
+// goes to a second buffer so bricks never read a neighbour's new values. The
+// post-smoother runs the colours in reverse order, which is the adjoint of
+// the pre-smoother: the V-cycle stays symmetric.
+//
+// Work split: wave w owns the rows of one (y, z) parity, w = (y%2) + 2(z%2),
+// and each of its 64 lanes the node pair (2m, 2m + 1) of one such row, whose
+// 2 x 26 couplings it holds in registers (FP16 couplings as loaded, widened
+// inside the multiply-adds). The pair's two colours are consecutive in the
+// colour order, so one wave does both in a step with no barrier between: the
+// eight other rows' values (two 8-byte LDS reads per row and load case) serve
+// both nodes, the partner's new value is in a register and the neighbouring
+// pair's comes by DPP. A sweep is four steps with one barrier each.
+// With a node spread over 8 lanes (each 2 to 4 couplings, partial sums
+// added by DPP, 8 steps a sweep) the kernel issued three times the
+// instructions and was bound by them: two sweeps at 128^3 (FP16) 97 us, now
+// 59; 64^3 (FP16 / FP32) 17 / 13.6, now 14.8 / 13.1.
+// Small levels are bound by the latency of the eight steps. There each
+// workgroup takes one load case (NR = 1; the couplings are then read three
+// times, from L2): a step waits for a third of the reads and multiply-adds.
+// 16^3 and 32^3: 9.2 -> 5.4 and 6.1 us, where all three load cases together
+// (NR = 3) take 8.3; at 512 bricks 18.5 against 13.1 us. The results have
+// the same bits either way.
 constexpr int kBrick = 8;
-constexpr int kBrickThreads = kBrick * kBrick * kBrick;
+constexpr int kStBrickThreads = 256;
 constexpr int kHalo = kBrick + 2;
+// LDS pitches of a row and a plane: the 8-byte reads of half a wave (rows
+// two apart, planes two apart) then fall on different banks
+constexpr int kStPitch = 12, kStPlane = 144;
+constexpr int kStOneMax = 256;  // bricks of a launch up to which NR = 1
 __host__ __device__ inline int brick_count(const Geom& g) {
   return ((g.nx + kBrick - 1) / kBrick) * ((g.ny + kBrick - 1) / kBrick) * ((g.nz + kBrick - 1) / kBrick);
 }
-__device__ inline int wrap_any(int a, int n) {
-  a %= n;
-  return a < 0 ? a + n : a;
-}
-// Coupling o of the stored stencil at node v (FP16: scaled back to FP32).
-template <bool HALF>
-__device__ inline float stencil_coef(const StRef& S, long long nn, long long v, int o) {
-  if constexpr (HALF)
-    return (float)S.f16[o * nn + v] * *S.scale;
-  else
-    return S.f32[o * nn + v];
-}
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
-// Work split of a colour step: the 64 nodes of one colour in a brick are
-// updated by 64 groups of 8 lanes. Lane j of a group holds the couplings
-// o = j, j + 8, j + 16, j + 24 (o != 13, o < 27: 2 to 4 of the 26) of its
-// node for every colour, forms their products with the three load cases'
-// values, and the group adds its eight partial sums (group8_sum); lanes
-// 0-2 then write load cases 0-2. With one node per thread
-// only 16 lanes of half the waves worked in a colour step, each through 78
-// dependent multiply-adds.
 // LDS of the brick smoother, one allocation for both stencil precisions
 // (a batched launch instantiates both bodies in one kernel).
-struct StBrickLds {
-  float su[OTM_NRHS][kHalo * kHalo * kHalo];  // u of the brick and its halo
-  float scf[kBrickThreads * 27];              // stencils, colour-major node order
+struct alignas(16) StBrickLds {
+  float su[OTM_NRHS][kHalo * kStPlane];  // u of the brick and its halo
 };
 __device__ inline StBrickLds& st_brick_lds() {
   __shared__ StBrickLds lds;
   return lds;
 }
 
-template <bool HALF>
-__device__ inline void st_brick_body(const Geom& g, const StRef& S, const float* __restrict__ f,
-                                     const float* __restrict__ uin, float* __restrict__ uout, int sweeps, int forward,
-                                     int zero_in, int b) {
-  auto& su = st_brick_lds().su;
-  float* scf = st_brick_lds().scf;
+// The brick of block b, its size, and this lane's node pair.
+struct StPair {
+  int ox, oy, oz, wx, wy, wz;  // first node, edges
+  int lx, ly, lz;              // the pair's first node in the brick
+  bool act;                    // inside the brick
+  unsigned v;                  // its index (of a node of the brick when not)
+};
+__device__ __forceinline__ StPair st_pair(const Geom& g, int b) {
+  StPair P;
   const int bx = (g.nx + kBrick - 1) / kBrick, by = (g.ny + kBrick - 1) / kBrick;
-  const int ox = (b % bx) * kBrick, oy = ((b / bx) % by) * kBrick, oz = (b / (bx * by)) * kBrick;
+  P.ox = (b % bx) * kBrick;
+  P.oy = ((b / bx) % by) * kBrick;
+  P.oz = (b / (bx * by)) * kBrick;
+  P.wx = min(kBrick, g.nx - P.ox);
+  P.wy = min(kBrick, g.ny - P.oy);
+  P.wz = min(kBrick, g.nz - P.oz);
+  const int m = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
+  P.lx = 2 * (m & 3);
+  P.ly = 2 * ((m >> 2) & 3) + (w & 1);
+  P.lz = 2 * (m >> 4) + (w >> 1);
+  P.act = P.lx < P.wx && P.ly < P.wy && P.lz < P.wz;
+  const int ax = P.act ? P.lx : 0, ay = P.act ? P.ly : 0, az = P.act ? P.lz : 0;
+  P.v = (unsigned)(P.ox + ax) + (unsigned)g.nx * ((unsigned)(P.oy + ay) + (unsigned)g.ny * (unsigned)(P.oz + az));
+  return P;
+}
+
+// u of the brick and its halo into LDS (zero without uin). Positions past a
+// cut brick's halo are not written: no active pair reads them.
+template <int NR>
+__device__ __forceinline__ void st_stage_u(const Geom& g, const StPair& P, const float* __restrict__ uin,
+                                           float (*su)[kHalo * kStPlane]) {
+  constexpr int kH3 = kHalo * kHalo * kHalo;
+  constexpr int kTrips = (kH3 + kStBrickThreads - 1) / kStBrickThreads;
   const int t = threadIdx.x;
-  const long long nn = g.nn;
-  // halo load (or zero initial guess): loads first, then the LDS stores
-  {
-    constexpr int kH3 = kHalo * kHalo * kHalo;
-    constexpr int kTrips = (kH3 + kBrickThreads - 1) / kBrickThreads;
-    float hv[kTrips][OTM_NRHS];
+  if (!uin) {
+    float* z = su[0];
+    for (int i = t; i < NR * kHalo * kStPlane; i += kStBrickThreads) z[i] = 0.f;
+    return;
+  }
+  float hv[kTrips][NR];
 #pragma unroll
-    for (int r = 0; r < kTrips; r++) {
-      const int i = t + kBrickThreads * r;
+  for (int r = 0; r < kTrips; r++) {
+    const int i = min(t + kStBrickThreads * r, kH3 - 1);
+    const int hx = min(i % kHalo, P.wx + 1), hy = min((i / kHalo) % kHalo, P.wy + 1),
+              hz = min(i / (kHalo * kHalo), P.wz + 1);
+    const unsigned w = (unsigned)wrapm(P.ox + hx - 1, g.nx) +
+                       (unsigned)g.nx * ((unsigned)wrapm(P.oy + hy - 1, g.ny) +
+                                         (unsigned)g.ny * (unsigned)wrapm(P.oz + hz - 1, g.nz));
 #pragma unroll
-      for (int k = 0; k < OTM_NRHS; k++) hv[r][k] = 0.f;
-      if (i < kH3 && !zero_in) {
-        const int hx = i % kHalo, hy = (i / kHalo) % kHalo, hz = i / (kHalo * kHalo);
-        const int X = wrap_any(ox + hx - 1, g.nx), Y = wrap_any(oy + hy - 1, g.ny), Z = wrap_any(oz + hz - 1, g.nz);
-        const long long w = (long long)X + (long long)g.nx * ((long long)Y + (long long)g.ny * Z);
+    for (int k = 0; k < NR; k++) hv[r][k] = ld_off(uin + (size_t)k * (size_t)g.nn, 4u * w);
+  }
 #pragma unroll
-        for (int k = 0; k < OTM_NRHS; k++) hv[r][k] = uin[k * nn + w];
-      }
-    }
+  for (int r = 0; r < kTrips; r++) {
+    const int i = t + kStBrickThreads * r;
+    const int hx = i % kHalo, hy = (i / kHalo) % kHalo, hz = i / (kHalo * kHalo);
+    if (i < kH3) {
 #pragma unroll
-    for (int r = 0; r < kTrips; r++) {
-      const int i = t + kBrickThreads * r;
-      if (i < kH3) {
-#pragma unroll
-        for (int k = 0; k < OTM_NRHS; k++) su[k][i] = hv[r][k];
-      }
+      for (int k = 0; k < NR; k++) su[k][hx + kStPitch * hy + kStPlane * hz] = hv[r][k];
     }
   }
-  const int m = t >> 3, j = t & 7;
-  int doff[4];
-  bool slot[4];
+}
+
+// A pair's couplings (first node a, second b) and diagonals. FP16 couplings
+// stay divided by the level's scale, which the sums are multiplied with;
+// they are held packed (kStPacked), half the registers for multiply-adds at
+// half the rate, or widened (kStWide): the same values and bits.
+enum StForm : int { kStFp32 = 0, kStPacked = 1, kStWide = 2 };
+template <int FORM>
+struct StCoef {
+  f32x2 c[27];
+  float scale;
+  __device__ __forceinline__ void load(const StRef& S, size_t nn, unsigned v) {
+    if constexpr (FORM == kStFp32) {
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const int o = j + 8 * q;
-    slot[q] = o < 27 && o != 13;
-    doff[q] = slot[q] ? (o % 3 - 1) + kHalo * (((o / 3) % 3 - 1) + kHalo * (o / 9 - 1)) : 0;
-  }
-  // Stencils: each thread loads its own node's 27 entries (neighbouring
-  // threads read neighbouring entries; load_stencil's values, FP16 diagonal
-  // included) into LDS in colour-major node order, from where each lane
-  // takes its slots for every colour. (Loaded straight into the slots, a
-  // wave's 64 loads touched 8 stencil arrays at stride-2 nodes.)
-  float cf[8][4], inv[8], fv[8];
-  {
-    const int lx = t & 7, ly = (t >> 3) & 7, lz = t >> 6;
-    const int x = ox + lx, y = oy + ly, z = oz + lz;
-    const bool act = x < g.nx && y < g.ny && z < g.nz;
-    float a[27];
-    if (act) {
-      load_stencil<HALF>(S, nn, (long long)x + (long long)g.nx * ((long long)y + (long long)g.ny * z), a);
+      for (int o = 0; o < 27; o++) c[o] = *(const f32x2*)((const char*)(S.f32 + o * nn) + 4u * v);
     } else {
+      scale = *S.scale;
+      f32x2 off = {0.f, 0.f};
 #pragma unroll
-      for (int o = 0; o < 27; o++) a[o] = 0.f;
+      for (int o = 0; o < 27; o++) {
+        if (o == 13) continue;
+        const f16x2 h = *(const f16x2*)((const char*)(S.f16 + o * nn) + 2u * v);
+        c[o] = f32x2{(float)h.x, (float)h.y};
+        off.x += c[o].x;
+        off.y += c[o].y;
+      }
+      c[13] = f32x2{-off.x * scale, -off.y * scale};  // minus the sum of the couplings
     }
-    const int c = (lx & 1) + 2 * (ly & 1) + 4 * (lz & 1), mm = (lx >> 1) + 4 * (ly >> 1) + 16 * (lz >> 1);
-    float* d = scf + (c * 64 + mm) * 27;
-#pragma unroll
-    for (int o = 0; o < 27; o++) d[o] = a[o];
   }
+  __device__ __forceinline__ f32x2 diag() const { return c[13]; }
+  __device__ __forceinline__ float scaled(float s) const { return FORM == kStFp32 ? s : s * scale; }
+  __device__ __forceinline__ float fma_a(int o, float w, float s) const { return fmaf(c[o].x, w, s); }
+  __device__ __forceinline__ float fma_b(int o, float w, float s) const { return fmaf(c[o].y, w, s); }
+};
+template <>
+struct StCoef<kStPacked> {
+  f16x2 c[27];
+  float scale;
+  __device__ __forceinline__ void load(const StRef& S, size_t nn, unsigned v) {
+    scale = *S.scale;
 #pragma unroll
-  for (int c = 0; c < 8; c++) {
-    const int x = ox + 2 * (m & 3) + (c & 1), y = oy + 2 * ((m >> 2) & 3) + ((c >> 1) & 1),
-              z = oz + 2 * (m >> 4) + (c >> 2);
-    const bool act = x < g.nx && y < g.ny && z < g.nz;
-    const long long v = act ? (long long)x + (long long)g.nx * ((long long)y + (long long)g.ny * z) : 0;
-    fv[c] = act && j < OTM_NRHS ? f[j * nn + v] : 0.f;
+    for (int o = 0; o < 27; o++)
+      if (o != 13) c[o] = *(const f16x2*)((const char*)(S.f16 + o * nn) + 2u * v);
   }
-  __syncthreads();
+  __device__ __forceinline__ f32x2 diag() const {
+    f32x2 off = {0.f, 0.f};
 #pragma unroll
-  for (int c = 0; c < 8; c++) {
-    const float* d = scf + (c * 64 + m) * 27;
-#pragma unroll
-    for (int q = 0; q < 4; q++) cf[c][q] = slot[q] ? d[j + 8 * q] : 0.f;
-    const float dg = d[13];
-    inv[c] = dg != 0.f ? 1.f / dg : 0.f;  // zero for nodes past the level's edge
+    for (int o = 0; o < 27; o++)
+      if (o != 13) {
+        off.x += (float)c[o].x;
+        off.y += (float)c[o].y;
+      }
+    return f32x2{-off.x * scale, -off.y * scale};
   }
-  auto step = [&](const int c) {
-    const int c0 = (2 * (m & 3) + (c & 1) + 1) + kHalo * ((2 * ((m >> 2) & 3) + ((c >> 1) & 1) + 1) +
-                                                          kHalo * (2 * (m >> 4) + (c >> 2) + 1));
-    float a[OTM_NRHS] = {0.f, 0.f, 0.f};
+  __device__ __forceinline__ float scaled(float s) const { return s * scale; }
+  // Takes either half of the packed register as it is. (Written as fmaf of
+  // a widened value, the compiler widens all couplings ahead of the sweeps.)
+  __device__ __forceinline__ float fma_a(int o, float w, float s) const {
+    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel_hi:[1,0,0]" : "+v"(s) : "v"(c[o]), "v"(w));
+    return s;
+  }
+  __device__ __forceinline__ float fma_b(int o, float w, float s) const {
+    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(s) : "v"(c[o]), "v"(w));
+    return s;
+  }
+};
+
+// Sums of the pair's couplings to the eight rows other than its own, with
+// the reads of two rows in flight (left to itself the compiler issues all of
+// them first, for 150 registers and a third of the resident workgroups).
+template <int NR, class Coef>
+__device__ __forceinline__ void st_other_rows(const Coef& C, const float (*su)[kHalo * kStPlane], int base,
+                                              float (&sa)[NR], float (&sb)[NR]) {
+  f32x2 w[3][NR][2];
+  auto fetch = [&](int i) {
+    const int r = i < 4 ? i : i + 1, off = base + kStPitch * (r % 3 - 1) + kStPlane * (r / 3 - 1);
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int p = c0 + doff[q];
-#pragma unroll
-      for (int k = 0; k < OTM_NRHS; k++) a[k] += cf[c][q] * su[k][p];
+    for (int k = 0; k < NR; k++) {
+      w[i % 3][k][0] = *(const f32x2*)&su[k][off];
+      w[i % 3][k][1] = *(const f32x2*)&su[k][off + 2];
     }
+  };
 #pragma unroll
-    for (int k = 0; k < OTM_NRHS; k++) a[k] = group8_sum(a[k]);
-    if (j < OTM_NRHS && inv[c] != 0.f) {
-      const float acc = j == 0 ? a[0] : (j == 1 ? a[1] : a[2]);
-      su[j][c0] = (fv[c] - acc) * inv[c];
+  for (int k = 0; k < NR; k++) sa[k] = sb[k] = 0.f;
+  fetch(0);
+  fetch(1);
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const int r = i < 4 ? i : i + 1;
+    if (i + 2 < 8) fetch(i + 2);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < NR; k++) {
+      const f32x2 w01 = w[i % 3][k][0], w23 = w[i % 3][k][1];
+      sa[k] = C.fma_a(3 * r, w01.x, sa[k]);
+      sb[k] = C.fma_b(3 * r, w01.y, sb[k]);
+      sa[k] = C.fma_a(3 * r + 1, w01.y, sa[k]);
+      sb[k] = C.fma_b(3 * r + 1, w23.x, sb[k]);
+      sa[k] = C.fma_a(3 * r + 2, w23.x, sa[k]);
+      sb[k] = C.fma_b(3 * r + 2, w23.y, sb[k]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// Value of the next / previous lane of a row of 16.
+__device__ __forceinline__ float row_next(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x101, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float row_prev(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x111, 0xF, 0xF, true));
+}
+
+template <bool FORWARD, int NR, class Coef>
+__device__ __forceinline__ void st_brick_sweeps(const StPair& P, const Coef& C, float (*su)[kHalo * kStPlane],
+                                                const f32x2 (&fv)[NR], f32x2 inv, int sweeps,
+                                                f32x2 (&u)[NR]) {
+  const int w = (int)threadIdx.x >> 6;
+  const int base = P.lx + kStPitch * (P.ly + 1) + kStPlane * (P.lz + 1);  // the node before the pair
+  const bool has_prev = P.lx > 0, has_next = P.lx + 2 < P.wx;
+#pragma unroll 1
+  for (int s = 0; s < 4 * sweeps; s++) {
+    const int p = FORWARD ? (s & 3) : 3 - (s & 3);
+    if (w == p) {
+      float sa[NR], sb[NR];
+      st_other_rows<NR>(C, su, base, sa, sb);
+#pragma unroll
+      for (int k = 0; k < NR; k++) {
+        const f32x2 w01 = *(const f32x2*)&su[k][base], w23 = *(const f32x2*)&su[k][base + 2];
+        if (FORWARD) {
+          sa[k] = C.fma_a(12, w01.x, C.fma_a(14, w23.x, sa[k]));
+          u[k].x = (fv[k].x - C.scaled(sa[k])) * inv.x;
+          const float nx = row_next(u[k].x);
+          sb[k] = C.fma_b(12, u[k].x, C.fma_b(14, has_next ? nx : w23.y, sb[k]));
+          u[k].y = (fv[k].y - C.scaled(sb[k])) * inv.y;
+        } else {
+          sb[k] = C.fma_b(12, w01.y, C.fma_b(14, w23.y, sb[k]));
+          u[k].y = (fv[k].y - C.scaled(sb[k])) * inv.y;
+          const float pv = row_prev(u[k].y);
+          sa[k] = C.fma_a(12, has_prev ? pv : w01.x, C.fma_a(14, u[k].y, sa[k]));
+          u[k].x = (fv[k].x - C.scaled(sa[k])) * inv.x;
+        }
+        if (P.act) {
+          su[k][base + 1] = u[k].x;
+          su[k][base + 2] = u[k].y;
+        }
+      }
     }
     __syncthreads();
-  };
-  for (int s = 0; s < sweeps; s++) {
-    if (forward) {
-#pragma unroll
-      for (int c = 0; c < 8; c++) step(c);
-    } else {
-#pragma unroll
-      for (int c = 7; c >= 0; c--) step(c);
-    }
   }
-  const int lx = t & 7, ly = (t >> 3) & 7, lz = t >> 6;
-  const int x = ox + lx, y = oy + ly, z = oz + lz;
-  if (x < g.nx && y < g.ny && z < g.nz) {
-    const long long v = (long long)x + (long long)g.nx * ((long long)y + (long long)g.ny * z);
-    const int c0 = (lx + 1) + kHalo * ((ly + 1) + kHalo * (lz + 1));
+}
+
+// NR load cases from k0 on of block b's brick.
+template <int FORM, int NR>
+__device__ inline void st_brick_body(const Geom& g, const StRef& S, const float* __restrict__ f,
+                                     const float* __restrict__ uin, float* __restrict__ uout, int sweeps, int forward,
+                                     int zero_in, int b, int k0) {
+  auto& su = st_brick_lds().su;
+  const StPair P = st_pair(g, b);
+  const size_t nn = (size_t)g.nn;
+  StCoef<FORM> C;
+  C.load(S, nn, P.v);
+  f32x2 fv[NR], u[NR];
 #pragma unroll
-    for (int k = 0; k < OTM_NRHS; k++) uout[k * nn + v] = su[k][c0];
+  for (int k = 0; k < NR; k++) fv[k] = *(const f32x2*)((const char*)(f + (k0 + k) * nn) + 4u * P.v);
+  st_stage_u<NR>(g, P, zero_in ? nullptr : uin + k0 * nn, su);
+  const f32x2 dg = C.diag(), inv = {1.f / dg.x, 1.f / dg.y};
+  __syncthreads();
+  if (forward)
+    st_brick_sweeps<true, NR>(P, C, su, fv, inv, sweeps, u);
+  else
+    st_brick_sweeps<false, NR>(P, C, su, fv, inv, sweeps, u);
+  if (P.act) {
+#pragma unroll
+    for (int k = 0; k < NR; k++) *(f32x2*)((char*)(uout + (k0 + k) * nn) + 4u * P.v) = u[k];
   }
 }
 
