@@ -225,23 +225,8 @@ struct OpProlong {
 struct OpTail {  // one workgroup per cell: the tail V-cycle from level C.tail down
   static constexpr int kThreads = kTailThreads;
   __device__ void operator()(const CellDev& C, const Ent& e, int, int) const {
-    __shared__ TailLevels T;
-    if (threadIdx.x == 0) {
-      T.n = C.nlev - C.tail;
-      T.sweeps = C.sweeps_coarse;
-      for (int i = 0; i < T.n; i++) {
-        const int l = C.tail + i;
-        T.g[i] = C.g[l];
-        T.f[i] = C.f[l];
-        T.res[i] = C.res[l];
-        T.st[i] = C.st[l];
-      }
-      T.f0 = C.f[C.tail];
-      T.Binv = C.Binv;
-      T.uout = ucur(C, e.par, C.tail);
-    }
-    __syncthreads();
-    tail_vcycle_body(T);
+    const int l = C.tail;
+    tail_vcycle_body(TailLevels{C.sweeps_coarse, C.g[l], C.g[l + 1], C.st[l], C.f[l], C.Binv, ucur(C, e.par, l)});
   }
 };
 

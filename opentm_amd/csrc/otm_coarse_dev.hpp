@@ -1230,210 +1230,258 @@ __device__ inline void gj_symmetrise_body(const Geom& g, const double* __restric
 }
 
 // ---- one-workgroup tail V-cycle ---------------------------------------------
-// The last levels of a hierarchy (from the first coarse level with at most
-// kTailStartNodes nodes down to the coarsest) hold a few hundred nodes: as
-// separate launches their smoothers, residuals and transfers are pure
-// launch and memory latency. One workgroup runs the whole tail V-cycle
-// instead. The stencils of its non-coarsest levels are staged into LDS once
-// (kTailStNodes nodes at most) and the corrections of every tail level stay
-// in LDS, with their right-hand sides and the residual being restricted;
-// smoothing is exact 8-colour Gauss-Seidel (forward before restriction,
-// reverse after prolongation, so the V-cycle stays symmetric), and the
-// coarsest level is solved with its explicit inverse. A hierarchy whose
-// coarse levels are all larger has no tail: its coarsest level is solved by
-// coarsest_rows_body.
-constexpr int kTailMaxLevels = 6;
-constexpr int kTailStartNodes = 512;                 // largest first tail level (8^3)
-constexpr int kTailStNodes = 512 + 64 + 8 + 1;       // stencil nodes held in LDS
-constexpr int kTailThreads = 512;  // (1024 would cap registers at 128 and spill)
-constexpr int kCoarsestMax = 4096;                   // largest coarsest level
-constexpr int kTailBinvNodes = 64;                   // coarsest inverse held in LDS up to this size
-static_assert(kTailStartNodes / 8 <= kTailThreads / 8, "a tail colour step has one node per group of 8 lanes");
+// The last two levels of a hierarchy, when the first of them has at most
+// kTailStartNodes nodes (8^3 and 4^3 for edges that are powers of two), are
+// a few hundred nodes: as separate launches their smoothers, residual,
+// transfers and coarsest product are pure launch and memory latency. One
+// workgroup runs the whole V-cycle of the two: exact 8-colour Gauss-Seidel
+// from zero (forward before restriction, reverse after prolongation, so the
+// V-cycle stays symmetric), residual, restriction, product with the coarsest
+// inverse, prolongation. A hierarchy whose coarse levels are larger has no
+// tail: its coarsest level is solved by coarsest_rows_body.
+//
+// Bound by latency: a chain of 16 Gauss-Seidel steps at two sweeps. The work
+// split is the brick smoother's for small levels (a lane owns a node pair of
+// one row parity, its couplings in registers, both colours in one step),
+// here one wave per row parity and load case, with the periodic neighbours
+// exact: rows wrap by their offsets, an x-halo column on either side is
+// written with the edge nodes. The coarsest inverse's entries are loaded
+// into registers at the start, four lanes to a result. 16.4 us at 8^3 (28 us
+// with 8 lanes per node, all stencils staged through LDS and 32 steps).
+constexpr int kTailStartNodes = 512;  // largest first tail level (8^3)
+constexpr int kTailCoarseNodes = kTailStartNodes / 8;
+constexpr int kTailThreads = 64 * 4 * OTM_NRHS;
+constexpr int kTailTerms = kTailCoarseNodes / 4;  // coarsest product, terms of a lane
+constexpr int kCoarsestMax = 4096;    // largest coarsest level
+// u of one load case: rows of nx + 4, planes padded to an odd multiple of 16
+// so that the reads of half a wave fall on different banks (an edge is at
+// least 6, so the largest is 6 x 6 x 14)
+constexpr int kTailU = 1280;
+static_assert(OTM_NRHS * kTailCoarseNodes * 4 <= kTailThreads, "four lanes per coarse result");
 
 struct TailLevels {
-  int n;  // levels in the tail; the last is the coarsest
   int sweeps;
-  Geom g[kTailMaxLevels];
-  const float* f0;                // right-hand side of the first tail level
-  float* f[kTailMaxLevels];       // right-hand sides of the deeper levels (written here)
-  float* res[kTailMaxLevels];     // residual scratch of the non-coarsest levels
-  StRef st[kTailMaxLevels];
-  const double* Binv;             // inverse of the coarsest level
-  float* uout;                    // correction of the first tail level (output)
+  Geom g, gc;          // the two levels
+  StRef st;            // stencil of the first
+  const float* f0;     // its right-hand side
+  const double* Binv;  // inverse of the coarsest
+  float* uout;         // correction of the first (output)
 };
 
 void launch_tail_vcycle(hipStream_t s, const TailLevels& T);
 
-__device__ inline void tail_stencil(const StRef& S, long long nn, long long v, float a[27]) {
-  if (S.f16)
-    load_stencil<true>(S, nn, v, a);
+// This lane's pair of the tail's first level.
+struct TailPair {
+  int k, p;            // load case, row parity
+  bool act;
+  unsigned v;          // first node
+  int off[9];          // LDS position of the node before the pair, per row
+  int next, prev;      // lanes of the neighbouring pairs in the row
+  bool first, last;    // pair at the row's begin / end
+  int nx;
+};
+
+// The next / previous pair's value in the row: in a cube of 8 a row's four
+// pairs are a quad of lanes.
+template <bool CUBE>
+__device__ __forceinline__ float tail_next(const TailPair& P, float v) {
+  if constexpr (CUBE)
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x39, 0xF, 0xF, true));
   else
-    load_stencil<false>(S, nn, v, a);
+    return __shfl(v, P.next, 64);
+}
+template <bool CUBE>
+__device__ __forceinline__ float tail_prev(const TailPair& P, float v) {
+  if constexpr (CUBE)
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x93, 0xF, 0xF, true));
+  else
+    return __shfl(v, P.prev, 64);
 }
 
-// `sweeps` exact 8-colour Gauss-Seidel sweeps on u of one tail level with
-// its stencil sa[o*nn + v] and right-hand side f (all in LDS). A node of
-// the active colour is updated by a group of 8 lanes as in the coarse brick
-// smoother (lane j takes the couplings o = j + 8q, the group adds with
-// group8_sum, lanes 0-2 write the three load cases). A tail level has at
-// most kTailStartNodes nodes, so each group owns one node position per
-// colour: its coordinates are decoded once per call, not per colour step
-// (the runtime divisions and the FP32 division per step made a step 2700
-// cycles long).
-template <bool FORWARD>
-__device__ inline void tail_smooth(const Geom& g, const float* sa, const float* f, float* u, int sweeps) {
-  const int hx = g.nx >> 1, hy = g.ny >> 1, hz = g.nz >> 1;
-  const int cnt = hx * hy * hz;  // nodes per colour, at most blockDim.x / 8
-  const int nn = (int)g.nn;
-  const int grp = (int)threadIdx.x >> 3, j = (int)threadIdx.x & 7;
-  const bool act = grp < cnt;
-  const int tx = act ? grp % hx : 0, tr = act ? grp / hx : 0;
-  const int ty = tr % hy, tz = tr / hy;
-  for (int s = 0; s < sweeps; s++)
+template <bool FORWARD, int FORM, bool CUBE>
+__device__ __forceinline__ void tail_sweeps(const TailPair& P, const StCoef<FORM>& C, float* su, f32x2 fv, f32x2 inv,
+                                            int sweeps, f32x2& u) {
+#pragma unroll 1
+  for (int s = 0; s < 4 * sweeps; s++) {
+    const int p = FORWARD ? (s & 3) : 3 - (s & 3);
+    if (P.p == p) {
+      float* own = su + P.off[4];
+      const float o0 = own[0], o3 = own[3];
+      float ra[2] = {0.f, 0.f}, rb[2] = {0.f, 0.f};  // two chains per node
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int col = FORWARD ? i : 7 - i;
-      if (act) {
-        const int x = 2 * tx + (col & 1), y = 2 * ty + ((col >> 1) & 1), z = 2 * tz + (col >> 2);
-        const int v = x + g.nx * (y + g.ny * z);
-        float a[OTM_NRHS] = {0.f, 0.f, 0.f};
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          const int o = j + 8 * q;
-          if (o < 27 && o != 13) {
-            const int X = wrapm(x + o % 3 - 1, g.nx), Y = wrapm(y + (o / 3) % 3 - 1, g.ny),
-                      Z = wrapm(z + o / 9 - 1, g.nz);
-            const int w = X + g.nx * (Y + g.ny * Z);
-            const float c = sa[o * nn + v];
-#pragma unroll
-            for (int k = 0; k < OTM_NRHS; k++) a[k] += c * u[k * nn + w];
-          }
-        }
-#pragma unroll
-        for (int k = 0; k < OTM_NRHS; k++) a[k] = group8_sum(a[k]);
-        if (j < OTM_NRHS) {
-          const float acc = j == 0 ? a[0] : (j == 1 ? a[1] : a[2]);
-          u[j * nn + v] = (f[j * nn + v] - acc) * __builtin_amdgcn_rcpf(sa[13 * nn + v]);
-        }
+      for (int r = 0; r < 9; r++) {
+        if (r == 4) continue;
+        const f32x2 w01 = *(const f32x2*)&su[P.off[r]], w23 = *(const f32x2*)&su[P.off[r] + 2];
+        float &sa = ra[(r < 4 ? r : r - 1) & 1], &sb = rb[(r < 4 ? r : r - 1) & 1];
+        sa = C.fma_a(3 * r, w01.x, sa);
+        sb = C.fma_b(3 * r, w01.y, sb);
+        sa = C.fma_a(3 * r + 1, w01.y, sa);
+        sb = C.fma_b(3 * r + 1, w23.x, sb);
+        sa = C.fma_a(3 * r + 2, w23.x, sa);
+        sb = C.fma_b(3 * r + 2, w23.y, sb);
       }
-      __syncthreads();
+      float sa = ra[0] + ra[1], sb = rb[0] + rb[1];
+      if (FORWARD) {
+        sa = C.fma_a(12, o0, C.fma_a(14, u.y, sa));
+        u.x = (fv.x - C.scaled(sa)) * inv.x;
+        sb = C.fma_b(12, u.x, C.fma_b(14, tail_next<CUBE>(P, u.x), sb));
+        u.y = (fv.y - C.scaled(sb)) * inv.y;
+      } else {
+        sb = C.fma_b(12, u.x, C.fma_b(14, o3, sb));
+        u.y = (fv.y - C.scaled(sb)) * inv.y;
+        sa = C.fma_a(12, tail_prev<CUBE>(P, u.y), C.fma_a(14, u.y, sa));
+        u.x = (fv.x - C.scaled(sa)) * inv.x;
+      }
+      if (P.act) {
+        own[1] = u.x;
+        own[2] = u.y;
+        if (P.first) own[P.nx + 1] = u.x;
+        if (P.last) own[2 - P.nx] = u.y;
+      }
     }
-}
-
-// res = f - A u at node t of a tail level (st_resid_node's arithmetic with
-// the stencil from LDS).
-__device__ inline void tail_resid_node(const Geom& g, const float* sa, const float* __restrict__ f, const float* u,
-                                       float* res, int t) {
-  const int nn = (int)g.nn;
-  int x, y, z;
-  split_node(g.nx, g.ny, t, x, y, z);
-  const int xs[3] = {x == 0 ? g.nx - 1 : x - 1, x, x == g.nx - 1 ? 0 : x + 1};
-  const int ys[3] = {y == 0 ? g.ny - 1 : y - 1, y, y == g.ny - 1 ? 0 : y + 1};
-  const int zs[3] = {z == 0 ? g.nz - 1 : z - 1, z, z == g.nz - 1 ? 0 : z + 1};
-  float a[27];
-#pragma unroll
-  for (int o = 0; o < 27; o++) a[o] = sa[o * nn + t];
-#pragma unroll
-  for (int k = 0; k < OTM_NRHS; k++) {
-    const float* uk = u + k * nn;
-    float s = 0.f;
-#pragma unroll
-    for (int o = 0; o < 27; o++) s += a[o] * uk[xs[o % 3] + g.nx * (ys[(o / 3) % 3] + g.ny * zs[o / 9])];
-    res[k * nn + t] = f[k * nn + t] - s;
+    __syncthreads();
   }
 }
 
-// Offsets of tail level l in the LDS corrections and in the LDS stencils
-// (every level before it stores OTM_NRHS, resp. 27, values per node).
-__device__ inline int tail_nodes_before(const TailLevels& T, int l) {
-  int o = 0;
-  for (int m = 0; m < l; m++) o += (int)T.g[m].nn;
-  return o;
+// Sum over the four lanes of a quad.
+__device__ __forceinline__ float quad_sum(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, false));
+  return v;
+}
+
+struct alignas(16) TailLds {
+  float u[OTM_NRHS][kTailU];
+  float res[OTM_NRHS][kTailStartNodes];
+  float fc[OTM_NRHS * kTailCoarseNodes], uc[OTM_NRHS * kTailCoarseNodes];
+};
+__device__ inline TailLds& tail_lds() {
+  __shared__ TailLds lds;
+  return lds;
+}
+
+// CUBE: 8^3 and 4^3, all index arithmetic on constants (the divisions by
+// runtime edges cost 2 us).
+template <int FORM, bool CUBE>
+__device__ __forceinline__ void tail_form_body(const TailLevels& T) {
+  TailLds& S = tail_lds();
+  const Geom g = CUBE ? Geom{8, 8, 8, 512} : T.g, gc = CUBE ? Geom{4, 4, 4, 64} : T.gc;
+  const int tid = threadIdx.x, m = tid & 63, w = tid >> 6;
+  const int hx = g.nx >> 1, hy = g.ny >> 1, hz = g.nz >> 1, nc = (int)gc.nn;
+  const int pitch = g.nx + 4, plane = ((pitch * g.ny + 15) & ~31) + 16;
+  TailPair P;
+  // the three waves of a parity are neighbours, so they run on three SIMDs
+  P.k = w % OTM_NRHS;
+  P.p = w / OTM_NRHS;
+  P.act = m < hx * hy * hz;
+  P.nx = g.nx;
+  const int mm = P.act ? m : 0, mx = mm % hx, mr = mm / hx, my = mr % hy, mz = mr / hy;
+  const int x = 2 * mx, y = 2 * my + (P.p & 1), z = 2 * mz + (P.p >> 1);
+  P.v = (unsigned)(x + g.nx * (y + g.ny * z));
+  P.first = mx == 0;
+  P.last = mx == hx - 1;
+  P.next = mm - mx + (P.last ? 0 : mx + 1);
+  P.prev = mm - mx + (P.first ? hx - 1 : mx - 1);
+#pragma unroll
+  for (int r = 0; r < 9; r++)
+    P.off[r] = x + pitch * wrapm(y + r % 3 - 1, g.ny) + plane * wrapm(z + r / 3 - 1, g.nz);
+  const size_t nn = (size_t)g.nn;
+  StCoef<FORM> C;
+  C.load(T.st, nn, P.v);
+  const f32x2 fv = *(const f32x2*)(T.f0 + P.k * nn + P.v);
+  // coarse results: lane quad o = load case, node; its lanes' terms 4t + part
+  const int o = tid >> 2, part = tid & 3;
+  const bool has = o < OTM_NRHS * nc;
+  const int ck = has ? o / nc : 0, ci = has ? o - ck * nc : 0;
+  double bv[kTailTerms];
+#pragma unroll
+  for (int t = 0; t < kTailTerms; t++) {
+    const int j = 4 * t + part;
+    const double b = T.Binv[min(j, nc - 1) * nc + ci];  // symmetric
+    bv[t] = j < nc ? b : 0.0;
+  }
+  float* su = S.u[P.k];
+  for (int i = tid; i < OTM_NRHS * kTailU; i += kTailThreads) S.u[0][i] = 0.f;
+  const f32x2 dg = C.diag(), inv = {1.f / dg.x, 1.f / dg.y};
+  f32x2 u = {0.f, 0.f};
+  __syncthreads();
+  tail_sweeps<true, FORM, CUBE>(P, C, su, fv, inv, T.sweeps, u);
+  {  // residual
+    float sa = 0.f, sb = 0.f;
+#pragma unroll
+    for (int r = 0; r < 9; r++) {
+      const f32x2 w01 = *(const f32x2*)&su[P.off[r]], w23 = *(const f32x2*)&su[P.off[r] + 2];
+      sa = C.fma_a(3 * r, w01.x, sa);
+      sb = C.fma_b(3 * r, w01.y, sb);
+      if (r != 4) {
+        sa = C.fma_a(3 * r + 1, w01.y, sa);
+        sb = C.fma_b(3 * r + 1, w23.x, sb);
+      }
+      sa = C.fma_a(3 * r + 2, w23.x, sa);
+      sb = C.fma_b(3 * r + 2, w23.y, sb);
+    }
+    if (P.act)
+      *(f32x2*)&S.res[P.k][P.v] = f32x2{fv.x - fmaf(dg.x, u.x, C.scaled(sa)), fv.y - fmaf(dg.y, u.y, C.scaled(sb))};
+  }
+  __syncthreads();
+  int cx, cy, cz;
+  split_node(gc.nx, gc.ny, ci, cx, cy, cz);
+  {  // restriction
+    float s = 0.f;
+#pragma unroll
+    for (int t = 0; t < 7; t++) {
+      const int q = min(4 * t + part, 26), dx = q % 3 - 1, dy = (q / 3) % 3 - 1, dz = q / 9 - 1;
+      const float wt = (4 * t + part < 27 ? 1.f : 0.f) * (dx ? 0.5f : 1.f) * (dy ? 0.5f : 1.f) * (dz ? 0.5f : 1.f);
+      s += wt * S.res[ck][wrapm(2 * cx + dx, g.nx) +
+                          g.nx * (wrapm(2 * cy + dy, g.ny) + g.ny * wrapm(2 * cz + dz, g.nz))];
+    }
+    s = quad_sum(s);
+    if (has && part == 0) S.fc[o] = s;
+  }
+  __syncthreads();
+  {  // coarsest: u = Binv f, FP64 accumulation
+    double s = 0.0;
+#pragma unroll
+    for (int t = 0; t < kTailTerms; t++) s += bv[t] * (double)S.fc[ck * nc + min(4 * t + part, nc - 1)];
+    s += dpp_f64<0xB1>(s);
+    s += dpp_f64<0x4E>(s);
+    if (has && part == 0) S.uc[o] = (float)s;
+  }
+  __syncthreads();
+  {  // prolongation
+    const float* uc = S.uc + P.k * nc;
+    const int Y1 = (y & 1) ? (my + 1 == gc.ny ? 0 : my + 1) : my, Z1 = (z & 1) ? (mz + 1 == gc.nz ? 0 : mz + 1) : mz;
+    const int X1 = mx + 1 == gc.nx ? 0 : mx + 1;
+    const int r00 = gc.nx * (my + gc.ny * mz), r10 = gc.nx * (Y1 + gc.ny * mz), r01 = gc.nx * (my + gc.ny * Z1),
+              r11 = gc.nx * (Y1 + gc.ny * Z1);
+    const float c0 = 0.25f * ((uc[r00 + mx] + uc[r10 + mx]) + (uc[r01 + mx] + uc[r11 + mx]));
+    const float c1 = 0.25f * ((uc[r00 + X1] + uc[r10 + X1]) + (uc[r01 + X1] + uc[r11 + X1]));
+    u.x += c0;
+    u.y += 0.5f * (c0 + c1);
+    if (P.act) {
+      float* own = su + P.off[4];
+      own[1] = u.x;
+      own[2] = u.y;
+      if (P.first) own[P.nx + 1] = u.x;
+      if (P.last) own[2 - P.nx] = u.y;
+    }
+  }
+  __syncthreads();
+  tail_sweeps<false, FORM, CUBE>(P, C, su, fv, inv, T.sweeps, u);
+  if (P.act) *(f32x2*)(T.uout + P.k * nn + P.v) = u;
 }
 
 __device__ inline void tail_vcycle_body(const TailLevels& T) {
-  __shared__ float su[OTM_NRHS * kTailStNodes];        // corrections
-  __shared__ float sst[27 * kTailStNodes];
-  __shared__ float sf[OTM_NRHS * kTailStNodes];        // right-hand sides of the tail levels
-  __shared__ float sres[OTM_NRHS * kTailStartNodes];   // residual of the level being restricted
-  __shared__ double sbinv[kTailBinvNodes * kTailBinvNodes];
-  const int tid = threadIdx.x, bs = blockDim.x;
-  const int L = T.n - 1;
-  const int nc = (int)T.g[L].nn;
-  auto off = [&](int l) { return OTM_NRHS * tail_nodes_before(T, l); };
-  auto soff = [&](int l) { return 27 * tail_nodes_before(T, l); };
-  // Stencils of the non-coarsest levels (the values load_stencil gives), the
-  // first level's right-hand side and a small coarsest inverse: everything
-  // the cycle reads more than once comes from LDS. (With the right-hand
-  // sides, residuals and inverse in global memory, every colour step and
-  // the coarsest product waited for L2: 33 us per cycle at 128^3.)
-  for (int l = 0; l < L; l++) {
-    const int nn = (int)T.g[l].nn;
-    for (int v = tid; v < nn; v += bs) {
-      float a[27];
-      tail_stencil(T.st[l], nn, v, a);
-#pragma unroll
-      for (int o = 0; o < 27; o++) sst[soff(l) + o * nn + v] = a[o];
-    }
+  if (T.g.nx == 8 && T.g.ny == 8 && T.g.nz == 8) {
+    if (T.st.f16)
+      tail_form_body<kStWide, true>(T);
+    else
+      tail_form_body<kStFp32, true>(T);
+  } else if (T.st.f16) {
+    tail_form_body<kStWide, false>(T);
+  } else {
+    tail_form_body<kStFp32, false>(T);
   }
-  if (L > 0)
-    for (int i = tid; i < OTM_NRHS * (int)T.g[0].nn; i += bs) sf[i] = T.f0[i];
-  const bool binv_lds = nc <= kTailBinvNodes;
-  if (binv_lds) {
-    // all loads in flight before the stores (a fixed trip count)
-    constexpr int kTrips = (kTailBinvNodes * kTailBinvNodes + kTailThreads - 1) / kTailThreads;
-    double bv[kTrips];
-#pragma unroll
-    for (int r = 0; r < kTrips; r++) {
-      const int i = tid + kTailThreads * r;
-      bv[r] = i < nc * nc ? T.Binv[i] : 0.0;
-    }
-#pragma unroll
-    for (int r = 0; r < kTrips; r++) {
-      const int i = tid + kTailThreads * r;
-      if (i < nc * nc) sbinv[i] = bv[r];
-    }
-  }
-  // down: smooth from zero, residual, restriction (into the next level's
-  // right-hand side in LDS)
-  for (int l = 0; l < L; l++) {
-    const Geom& g = T.g[l];
-    float* u = su + off(l);
-    const float* f = sf + off(l);
-    for (int i = tid; i < OTM_NRHS * (int)g.nn; i += bs) u[i] = 0.f;
-    __syncthreads();
-    tail_smooth<true>(g, sst + soff(l), f, u, T.sweeps);
-    for (int t = tid; t < (int)g.nn; t += bs) tail_resid_node(g, sst + soff(l), f, u, sres, t);
-    __syncthreads();
-    for (int t = tid; t < (int)T.g[l + 1].nn; t += bs) restrict_node(g, T.g[l + 1], sres, sf + off(l + 1), t);
-    __syncthreads();
-  }
-  // coarsest: u = Binv f (FP64 accumulation). From LDS, row i is read as
-  // column i (Binv is symmetric): neighbouring lanes read neighbouring
-  // entries, no bank conflicts.
-  {
-    const float* f = L == 0 ? T.f0 : sf + off(L);
-    for (int q = tid; q < OTM_NRHS * nc; q += bs) {
-      const int k = q / nc, i = q - k * nc;
-      double s = 0.0;
-      if (binv_lds) {
-        for (int j = 0; j < nc; j++) s += sbinv[j * nc + i] * (double)f[k * nc + j];
-      } else {
-        for (int j = 0; j < nc; j++) s += T.Binv[(long long)i * nc + j] * (double)f[k * nc + j];
-      }
-      su[off(L) + q] = (float)s;
-    }
-    __syncthreads();
-  }
-  // up: prolongation, reverse smoothing
-  for (int l = L - 1; l >= 0; l--) {
-    const Geom& g = T.g[l];
-    float* u = su + off(l);
-    for (int t = tid; t < (int)g.nn; t += bs) prolong_node(g, T.g[l + 1], su + off(l + 1), u, t);
-    __syncthreads();
-    tail_smooth<false>(g, sst + soff(l), sf + off(l), u, T.sweeps);
-  }
-  for (int i = tid; i < OTM_NRHS * (int)T.g[0].nn; i += bs) T.uout[i] = su[i];
 }
 
 }  // namespace otm

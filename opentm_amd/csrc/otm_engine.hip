@@ -248,25 +248,13 @@ static void build_hierarchy(otm_ctx* c) {
     c->lv.push_back(L);
   }
   c->cB = dalloc<double>(coarsest_work_doubles(ncoarse));  // Gauss-Jordan work space
-  // the tail V-cycle takes over from the first coarse level with at most
-  // kTailStartNodes nodes whose levels fit the tail's LDS (a hierarchy with
-  // no such level has no tail). A tail from 16^3 with stencils re-read from global
-  // memory measured slower than the separate launches (131 against about
-  // 100 us per V-cycle at 128^3); from 8^3 with the stencils in LDS it
-  // replaces eleven launches.
+  // the tail V-cycle takes over the last two levels when the first of them
+  // has at most kTailStartNodes nodes (an edge halves down to at least 3, so
+  // no three levels are that small). A tail from 16^3 with stencils re-read
+  // from global memory measured slower than the separate launches (131
+  // against about 100 us per V-cycle at 128^3).
   c->tail = (int)c->lv.size() - 1;
-  for (size_t l = 1; l + 1 < c->lv.size(); l++) {
-    long long st_nodes = 0, nodes = 0;
-    for (size_t m = l; m < c->lv.size(); m++) {
-      nodes += c->lv[m].g.nn;
-      if (m + 1 < c->lv.size()) st_nodes += c->lv[m].g.nn;
-    }
-    if (c->lv[l].g.nn <= kTailStartNodes && (int)(c->lv.size() - l) <= kTailMaxLevels &&
-        st_nodes <= kTailStNodes && nodes <= kTailStNodes) {
-      c->tail = (int)l;
-      break;
-    }
-  }
+  if (c->lv.size() > 2 && c->lv[c->lv.size() - 2].g.nn <= kTailStartNodes) c->tail--;
   c->cBinv = dalloc<double>(ncoarse * ncoarse);
   c->partials = dalloc<double>((size_t)kMaxReduceBlocks * kMaxReduce);
   // one row per fine tile of the smallest shape (32 x 4 x 4 = 512 nodes)
@@ -355,21 +343,8 @@ static void smooth(otm_ctx* c, size_t l, int sweeps, bool forward) {
 }
 
 static TailLevels tail_levels(const otm_ctx* c, int nsw, float* uout) {
-  TailLevels T;
-  memset(&T, 0, sizeof(T));
-  T.n = (int)c->lv.size() - c->tail;
-  T.sweeps = nsw;
-  for (int i = 0; i < T.n; i++) {
-    const Level& L = c->lv[c->tail + i];
-    T.g[i] = L.g;
-    T.f[i] = L.f;
-    T.res[i] = L.res;
-    T.st[i] = stref(L);
-  }
-  T.f0 = c->lv[c->tail].f;
-  T.Binv = c->cBinv;
-  T.uout = uout;
-  return T;
+  const Level& L = c->lv[c->tail];
+  return TailLevels{nsw, L.g, c->lv[c->tail + 1].g, stref(L), L.f, c->cBinv, uout};
 }
 
 static void vcycle(otm_ctx* c, size_t l) {

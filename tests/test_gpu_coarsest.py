@@ -62,3 +62,30 @@ def test_batched_inverse_is_the_single_cells():
     for h, f, a in zip(homs, fs, alone):
         assert np.array_equal(h.coarsest_solve(f), a)
     batch.close()
+
+
+@pytest.mark.parametrize("fp16", [0, 1])
+@pytest.mark.parametrize("reso,min_coarse", [((16, 16, 16), 4), ((12, 12, 12), 3), ((12, 12, 28), 3), ((28, 12, 12), 3),
+                                             ((12, 16, 20), 3)])
+def test_tail_is_its_parts(reso, min_coarse, fp16):
+    """The V-cycle whose last two levels run in the one-workgroup tail (8^3
+    and edges that are no power of two, whose rows wrap inside a wave) against
+    the same V-cycle put together from the level entry points. About ten
+    FP32 parts, each held to 2e-6 by its own tests."""
+    hom = make(reso, min_coarse=min_coarse, exact_smoother=1, fp16_stencils=fp16)
+    hom.update(conductivity(reso))
+    assert len(hom.levels()) == 3
+    n = int(np.prod(reso))
+    r = np.random.default_rng(n).standard_normal((3, n)).astype(np.float32)
+    r -= r.mean(axis=1, keepdims=True)
+    r = r.reshape(-1)
+    z = hom.smooth_level(0, r, np.zeros_like(r), sweeps=2, mode=0)
+    f1 = hom.restrict(1, r - hom.apply_level(0, z))
+    u1 = hom.smooth_level(1, f1, np.zeros_like(f1), sweeps=2, mode=0)
+    u1 = hom.prolong_add(2, hom.coarsest_solve(hom.restrict(2, f1 - hom.apply_level(1, u1))), u1)
+    u1 = hom.smooth_level(1, f1, u1, sweeps=2, mode=1)
+    z = hom.smooth_level(0, r, hom.prolong_add(1, u1, z), sweeps=2, mode=1)
+    got = hom.vcycle(r)
+    err = np.abs(got - z).max() / np.abs(z).max()
+    print("[case] tail", reso, "fp16", fp16, "err", err, flush=True)
+    assert err < 2e-5
