@@ -63,6 +63,7 @@ struct CellDev {
   bool brick[kMaxLevels];
   const double* Binv;
   double* partials;
+  double* tile_partials;  // the fine post-smoother's r.z, a row per tile
   double* red_out;
   PcgScalars* pcg;
   double rtol2, inv_nn, inner2;
@@ -137,11 +138,11 @@ kb_fine_brick(const Ent* __restrict__ ents, int nents, const CellDev* __restrict
   const Ent e = ents[i];
   const CellDev& C = cells[e.cell];
   const int sw = C.sweeps_fine;
-  if (post)
-    fine_brick_body<BX>(C.g[0], C.fc, C.kappa, C.f[0], ucur(C, e.par, 0), uoth(C, e.par, 0), sw, 0, 0,
-                        b - e.block0);
-  else
-    fine_brick_body<BX>(C.g[0], C.fc, C.kappa, C.f[0], nullptr, ucur(C, e.par, 0), sw, 1, 1, b - e.block0);
+  Reduce R = cell_reduce(C, FIN_STORE);
+  R.partials = C.tile_partials;
+  fine_brick_body<BX>(C.g[0], C.fc, C.kappa, C.f[0], post ? ucur(C, e.par, 0) : nullptr,
+                      post ? uoth(C, e.par, 0) : ucur(C, e.par, 0), sw, post ? 0 : 1, post ? 0 : 1, b - e.block0,
+                      post, R);
 }
 
 // ---- operations (one functor per batched launch) ---------------------------
@@ -264,12 +265,20 @@ struct OpFinal {  // one block per cell
   static constexpr int kThreads = kBlock;
   int mode, nv;
   double rtol2;   // < 0: the cell's own
-  int tiled = 0;  // partials of the tiled operator apply: its own count
+  int tiled = 0;  // 1: partials of the tiled operator apply, 2: of the fine post-smoother (r.z)
   __device__ void operator()(const CellDev& C, const Ent&, int, int) const {
     Reduce R = cell_reduce(C, mode);
     if (rtol2 >= 0.0) R.rtol2 = rtol2;
-    const unsigned nb = (tiled && C.tile_bx) ? fine_apply_tile_blocks(C.g[0], C.tile_bx)
-                                              : red_blocks_for(C.g[0].nn);
+    unsigned nb = red_blocks_for(C.g[0].nn);
+    if (tiled == 1 && C.tile_bx) nb = fine_apply_tile_blocks(C.g[0], C.tile_bx);
+    if (tiled == 2 && C.fine_bx) {
+      R.partials = C.tile_partials;
+      nb = (unsigned)fine_tiles(C.g[0], C.fine_bx);
+      if (nb > (unsigned)kMaxReduceBlocks) {  // as launch_reduce_final
+        reduce_final_many_nv<OTM_NRHS>(R, (int)nb);
+        return;
+      }
+    }
     reduce_final_body(R, nv, (int)nb);
   }
 };
@@ -570,6 +579,7 @@ CellDev describe(const Member& m) {
   d.x64 = c->x64;
   d.Binv = c->cBinv;
   d.partials = c->partials;
+  d.tile_partials = c->tile_partials;
   d.red_out = c->red_out;
   d.pcg = c->pcg;
   d.rtol2 = c->cfg.fem_rel_thres * c->cfg.fem_rel_thres;
@@ -872,9 +882,13 @@ void step(otm_batch* b) {
   if (!V.empty()) {
     add_op(b, A2, OpSubMeanR{0}, [](const Member& m) { return (long long)std::min<long long>(8192, nblk(m.c->g0.nn)); });
     plan_vcycle(b, V);
-    add_op(b, V, OpDot3{}, redb);
-    add_op(b, A2, OpFinal{FIN_RZ_FIRST, OTM_NRHS, -1.0}, one);
-    add_op(b, B2, OpFinal{FIN_RZ, OTM_NRHS, -1.0}, one);
+    // the tiled post-smoother has formed r.z; cells on exact sweeps form it here
+    std::vector<Member*> untiled;
+    for (Member* m : V)
+      if (!m->c->lv[0].brick || !fine_brick_x(m->c->g0)) untiled.push_back(m);
+    add_op(b, untiled, OpDot3{}, redb);
+    add_op(b, A2, OpFinal{FIN_RZ_FIRST, OTM_NRHS, -1.0, 2}, one);
+    add_op(b, B2, OpFinal{FIN_RZ, OTM_NRHS, -1.0, 2}, one);
     add_op(b, A2, OpFillVec{0}, [](const Member& m) { return (long long)std::min<long long>(8192, nblk(3 * m.c->g0.nn)); });
     add_op(b, V, OpPcgP{}, redb);
     flush(b);

@@ -87,12 +87,17 @@ __global__ void __launch_bounds__(kBlock) k_fine_energy6(Geom g, FineConsts fc, 
 // The occupancy hint keeps the fully unrolled colour loop from holding
 // every node's loads in flight at once (which costs occupancy); the 30 KB
 // LDS footprint of a 32x4x8 brick allows five workgroups per CU.
-template <int BX, int BY, int BZ, int TR>
+// One tile and NR load cases per workgroup.
+template <int BX, int BY, int BZ, int TR, int NR>
 __global__ void __launch_bounds__(BX * TR) __attribute__((amdgpu_waves_per_eu(4, 8)))
 k_fine_smooth_brick(Geom g, FineConsts fc, const float* __restrict__ kappa, const float* __restrict__ f,
                     const float* __restrict__ uin, float* __restrict__ uout, int sweeps, int forward, int zero_in,
                     int dot, Reduce RD) {
-  fine_brick_body<BX, BY, BZ, TR>(g, fc, kappa, f, uin, uout, sweeps, forward, zero_in, xcd_block(), dot, RD);
+  constexpr int kParts = OTM_NRHS / NR;
+  const int b = xcd_block(), k0 = (b % kParts) * NR;
+  const size_t o = (size_t)k0 * (size_t)g.nn;
+  fine_brick_body<BX, BY, BZ, TR, NR>(g, fc, kappa, f + o, uin + o, uout + o, sweeps, forward, zero_in, b / kParts,
+                                      dot, RD, k0);
 }
 
 bool fine_tile_ok(const Geom& g, int v) {
@@ -110,43 +115,39 @@ static long long fine_variant_tiles(const Geom& g, int v) {
   return (long long)(g.nx / t.bx) * (g.ny / t.by) * (g.nz / t.bz);
 }
 
-// r.z in the smoother: 256-thread tiles, one partial-sum row per tile in
-// the context's tile partials (one row per 512 nodes, at most kTileDotSlots)
+// r.z in the smoother: one partial-sum row per tile in the context's tile
+// partials (one row per 512 nodes, at most kTileDotSlots)
 bool fine_brick_dot_ok(const Geom& g, int v) {
-  if (!fine_tile_ok(g, v)) return false;
-  const FineTileShape& t = kFineTileShapes[v];
-  return t.bx == 32 && t.bx * t.tr == kBlock && fine_variant_tiles(g, v) <= kTileDotSlots;
+  return fine_tile_ok(g, v) && fine_variant_tiles(g, v) <= kTileDotSlots;
+}
+
+// Up to this many tiles a launch takes one load case per workgroup: 8 tiles
+// 10.3 -> 7.3 us, 216 tiles of 128 threads 10.7 -> 10.3, 288 of 256 threads
+// 11.8 -> 11.3, 2048 of them 26 -> 38.
+constexpr long long kFineOneMax = 128;
+
+template <int BX, int BY, int BZ, int TR>
+static void launch_fine_tile(hipStream_t s, const Geom& g, const FineConsts& fc, const float* kappa, const float* f,
+                             const float* uin, float* uout, int sweeps, bool forward, bool zero_in, long long tiles,
+                             const Reduce* dot) {
+  const bool one = tiles <= kFineOneMax;
+  const auto k = one ? k_fine_smooth_brick<BX, BY, BZ, TR, 1> : k_fine_smooth_brick<BX, BY, BZ, TR, OTM_NRHS>;
+  hipLaunchKernelGGL(k, dim3((unsigned)(one ? OTM_NRHS * tiles : tiles)), dim3(BX * TR), 0, s, g, fc, kappa, f, uin,
+                     uout, sweeps, forward ? 1 : 0, zero_in ? 1 : 0, dot ? 1 : 0, dot ? *dot : Reduce{});
 }
 
 void launch_fine_smooth_brick(hipStream_t s, const Geom& g, const FineConsts& fc, const float* kappa, const float* f,
                               const float* uin, float* uout, int sweeps, bool forward, bool zero_in, int v,
                               const Reduce* dot) {
   if (!fine_tile_ok(g, v)) throw std::invalid_argument("the cell does not tile with this fine tile shape");
-  if (dot && !fine_brick_dot_ok(g, v)) throw std::invalid_argument("r.z in the smoother needs 256-thread 32-wide tiles");
-  const unsigned nb = (unsigned)fine_variant_tiles(g, v);
-  const Reduce RD = dot ? *dot : Reduce{};
-  const int fw = forward ? 1 : 0, zi = zero_in ? 1 : 0, d = dot ? 1 : 0;
+  if (dot && !fine_brick_dot_ok(g, v)) throw std::invalid_argument("too many tiles for r.z in the smoother");
+  const long long nt = fine_variant_tiles(g, v);
   switch (v) {
-    case 0:
-      hipLaunchKernelGGL((k_fine_smooth_brick<32, 4, 8, 8>), dim3(nb), dim3(256), 0, s, g, fc, kappa, f, uin, uout,
-                         sweeps, fw, zi, d, RD);
-      break;
-    case 1:
-      hipLaunchKernelGGL((k_fine_smooth_brick<16, 4, 8, 8>), dim3(nb), dim3(128), 0, s, g, fc, kappa, f, uin, uout,
-                         sweeps, fw, zi, 0, RD);
-      break;
-    case 2:
-      hipLaunchKernelGGL((k_fine_smooth_brick<32, 8, 4, 8>), dim3(nb), dim3(256), 0, s, g, fc, kappa, f, uin, uout,
-                         sweeps, fw, zi, d, RD);
-      break;
-    case 3:
-      hipLaunchKernelGGL((k_fine_smooth_brick<32, 4, 4, 4>), dim3(nb), dim3(128), 0, s, g, fc, kappa, f, uin, uout,
-                         sweeps, fw, zi, 0, RD);
-      break;
-    default:
-      hipLaunchKernelGGL((k_fine_smooth_brick<32, 8, 8, 8>), dim3(nb), dim3(256), 0, s, g, fc, kappa, f, uin, uout,
-                         sweeps, fw, zi, d, RD);
-      break;
+    case 0: launch_fine_tile<32, 4, 8, 8>(s, g, fc, kappa, f, uin, uout, sweeps, forward, zero_in, nt, dot); break;
+    case 1: launch_fine_tile<16, 4, 8, 8>(s, g, fc, kappa, f, uin, uout, sweeps, forward, zero_in, nt, dot); break;
+    case 2: launch_fine_tile<32, 8, 4, 8>(s, g, fc, kappa, f, uin, uout, sweeps, forward, zero_in, nt, dot); break;
+    case 3: launch_fine_tile<32, 4, 4, 4>(s, g, fc, kappa, f, uin, uout, sweeps, forward, zero_in, nt, dot); break;
+    default: launch_fine_tile<32, 8, 8, 8>(s, g, fc, kappa, f, uin, uout, sweeps, forward, zero_in, nt, dot); break;
   }
 }
 

@@ -777,7 +777,7 @@ __device__ inline TileOrigin tile_origin(const Geom& g, int b) {
 // base and a 32-bit byte offset (a lattice has at most 2^30 nodes). Done
 // per lane, this arithmetic was about 40% of the smoother's vector
 // instructions.
-template <int BX, int BY, int BZ, int TR>
+template <int BX, int BY, int BZ, int TR, int NR = OTM_NRHS>
 struct TileStage {
   using T = FineTile<BX, BY, BZ, TR>;
   static constexpr int WR = 64 / BX;                   // thread rows per wave
@@ -788,7 +788,7 @@ struct TileStage {
   static constexpr int UJ = (UR + TR - 1) / TR;
   static constexpr int UH = (2 * UR + T::NT - 1) / T::NT;  // halo-column nodes per thread
   float k[KJ], kh[KH];
-  float u[OTM_NRHS][UJ], uh[OTM_NRHS][UH];
+  float u[NR][UJ], uh[NR][UH];
 };
 
 // first thread row of this wave (wave-uniform) and the lane's row within it
@@ -822,10 +822,10 @@ __device__ inline unsigned lane_run_offset(const Geom& g, int rb, int rows, int 
 }
 
 // kappa of element (ox-1+kx, oy-1+ky, oz-1+kz), for sk[kx + KX*(ky + KY*kz)]
-template <int BX, int BY, int BZ, int TR>
+template <int BX, int BY, int BZ, int TR, int NR = OTM_NRHS>
 __device__ inline void load_tile_kappa(const Geom& g, const float* __restrict__ kappa, const TileOrigin& o,
-                                       TileStage<BX, BY, BZ, TR>& st) {
-  using S = TileStage<BX, BY, BZ, TR>;
+                                       TileStage<BX, BY, BZ, TR, NR>& st) {
+  using S = TileStage<BX, BY, BZ, TR, NR>;
   using T = FineTile<BX, BY, BZ, TR>;
   const int t = threadIdx.x, tx = t % BX;
   const int ty = wave_first_row<BX>() + lane_row<BX>();
@@ -846,9 +846,9 @@ __device__ inline void load_tile_kappa(const Geom& g, const float* __restrict__ 
     }
   }
 }
-template <int BX, int BY, int BZ, int TR>
-__device__ inline void store_tile_kappa(float* sk, const TileStage<BX, BY, BZ, TR>& st) {
-  using S = TileStage<BX, BY, BZ, TR>;
+template <int BX, int BY, int BZ, int TR, int NR = OTM_NRHS>
+__device__ inline void store_tile_kappa(float* sk, const TileStage<BX, BY, BZ, TR, NR>& st) {
+  using S = TileStage<BX, BY, BZ, TR, NR>;
   using T = FineTile<BX, BY, BZ, TR>;
   const int t = threadIdx.x, tx = t % BX, ty = t / BX;
 #pragma unroll
@@ -863,26 +863,26 @@ __device__ inline void store_tile_kappa(float* sk, const TileStage<BX, BY, BZ, T
   }
 }
 
-// field k (k < OTM_NRHS) of node (ox-1+hx, oy-1+hy, oz-1+hz), for
+// field k (k < NR) of node (ox-1+hx, oy-1+hy, oz-1+hz), for
 // su[k*kU + hx + HX*(hy + HY*hz)]
-template <int BX, int BY, int BZ, int TR>
+template <int BX, int BY, int BZ, int TR, int NR = OTM_NRHS>
 __device__ inline void load_tile_fields(const Geom& g, const float* __restrict__ src, const TileOrigin& o,
-                                        TileStage<BX, BY, BZ, TR>& st) {
-  using S = TileStage<BX, BY, BZ, TR>;
+                                        TileStage<BX, BY, BZ, TR, NR>& st) {
+  using S = TileStage<BX, BY, BZ, TR, NR>;
   using T = FineTile<BX, BY, BZ, TR>;
   const int t = threadIdx.x, tx = t % BX;
   const int wr0 = wave_first_row<BX>();
   const int ty = wr0 + lane_row<BX>();
-  const float* srck[OTM_NRHS];
+  const float* srck[NR];
 #pragma unroll
-  for (int k = 0; k < OTM_NRHS; k++) srck[k] = src + (size_t)k * (size_t)g.nn;
+  for (int k = 0; k < NR; k++) srck[k] = src + (size_t)k * (size_t)g.nn;
 #pragma unroll
   for (int j = 0; j < S::UJ; j++) {
     const int rb = wr0 + TR * j;
     const unsigned off = lane_run_offset<BX, T::HY>(g, rb, S::UR, o.oy - 1, o.oz - 1) + 4u * (unsigned)(o.ox + tx);
     if (ty + TR * j < S::UR) {
 #pragma unroll
-      for (int k = 0; k < OTM_NRHS; k++) st.u[k][j] = ld_off(srck[k], off);
+      for (int k = 0; k < NR; k++) st.u[k][j] = ld_off(srck[k], off);
     }
   }
   const int xm = wrapm(o.ox - 1, g.nx), xp = wrapm(o.ox + BX, g.nx);
@@ -894,13 +894,13 @@ __device__ inline void load_tile_fields(const Geom& g, const float* __restrict__
       const int hy = r % T::HY, hz = r / T::HY;
       const unsigned w = 4u * (wrapped_row(g, o.oy - 1 + hy, o.oz - 1 + hz) + (unsigned)(side ? xp : xm));
 #pragma unroll
-      for (int k = 0; k < OTM_NRHS; k++) st.uh[k][j] = ld_off(srck[k], w);
+      for (int k = 0; k < NR; k++) st.uh[k][j] = ld_off(srck[k], w);
     }
   }
 }
-template <int BX, int BY, int BZ, int TR>
-__device__ inline void store_tile_fields(float* su, const TileStage<BX, BY, BZ, TR>& st) {
-  using S = TileStage<BX, BY, BZ, TR>;
+template <int BX, int BY, int BZ, int TR, int NR = OTM_NRHS>
+__device__ inline void store_tile_fields(float* su, const TileStage<BX, BY, BZ, TR, NR>& st) {
+  using S = TileStage<BX, BY, BZ, TR, NR>;
   using T = FineTile<BX, BY, BZ, TR>;
   const int t = threadIdx.x, tx = t % BX, ty = t / BX;
 #pragma unroll
@@ -908,7 +908,7 @@ __device__ inline void store_tile_fields(float* su, const TileStage<BX, BY, BZ, 
     const int r = ty + TR * j;
     if (r < S::UR) {
 #pragma unroll
-      for (int k = 0; k < OTM_NRHS; k++) su[k * T::kU + r * T::HX + 1 + tx] = st.u[k][j];
+      for (int k = 0; k < NR; k++) su[k * T::kU + r * T::HX + 1 + tx] = st.u[k][j];
     }
   }
 #pragma unroll
@@ -917,7 +917,7 @@ __device__ inline void store_tile_fields(float* su, const TileStage<BX, BY, BZ, 
     if (i < 2 * S::UR) {
       const int r = i >> 1, hx = (i & 1) ? T::HX - 1 : 0;
 #pragma unroll
-      for (int k = 0; k < OTM_NRHS; k++) su[k * T::kU + r * T::HX + hx] = st.uh[k][j];
+      for (int k = 0; k < NR; k++) su[k * T::kU + r * T::HX + hx] = st.uh[k][j];
     }
   }
 }
@@ -1009,21 +1009,27 @@ __device__ inline void fine_residual_tile_body(const Geom& g, const FineConsts& 
 // zero coefficient), so an update is 20 LDS reads and 20 FMAs per load case
 // plus 12 adds shared by the three.
 //
-// With dot set (post-smoother of a PCG preconditioner application, 256
-// threads), the block also forms its partial sums of f.u over its nodes
-// with the final u (r.z: f is the PCG residual, u the preconditioned
-// residual), from the values it already holds, into slot b of RD.
-template <int BX, int BY = kFineBY, int BZ = kFineBZ, int TR = kFineTR>
+// With dot set (post-smoother of a PCG preconditioner application), the
+// block also forms its partial sums of f.u over its nodes with the final u
+// (r.z: f is the PCG residual, u the preconditioned residual), from the
+// values it already holds, into slot b of RD.
+//
+// NR = 1 smooths load case k0 alone (f, uin, uout point at it). Small cells
+// are bound by the latency of the colour steps: there each workgroup takes
+// one load case, with every node's weights in registers from the start
+// (with all three they cost a wave per SIMD, see below), and a step waits
+// for a third of the LDS reads. The results have the same bits either way.
+template <int BX, int BY = kFineBY, int BZ = kFineBZ, int TR = kFineTR, int NR = OTM_NRHS>
 __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, const float* __restrict__ kappa,
                                        const float* __restrict__ f, const float* __restrict__ uin,
                                        float* __restrict__ uout, int sweeps, int forward, int zero_in, int b,
-                                       int dot = 0, const Reduce& RD = Reduce{}) {
+                                       int dot = 0, const Reduce& RD = Reduce{}, int k0 = 0) {
   using T = FineTile<BX, BY, BZ, TR>;
   constexpr int HX = T::HX, HY = T::HY, KX = T::KX, KY = T::KY;
   constexpr int R = (BY / 2) * (BZ / 2);  // x-rows of one colour
   constexpr int H = R / TR;               // of them per thread row
   static_assert(R % TR == 0, "thread rows must divide the rows of a colour");
-  __shared__ float su[OTM_NRHS][T::kU];
+  __shared__ float su[NR][T::kU];
   __shared__ float sk[T::kK];
   const TileOrigin o = tile_origin<BX, BY, BZ>(g, b);
   const int ox = o.ox, oy = o.oy, oz = o.oz;
@@ -1034,17 +1040,17 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
   // the first LDS store; the right-hand side's loads then fly during the
   // stores and the barrier
   {
-    TileStage<BX, BY, BZ, TR> st;
-    load_tile_kappa<BX, BY, BZ, TR>(g, kappa, o, st);
-    if (!zero_in) load_tile_fields<BX, BY, BZ, TR>(g, uin, o, st);
-    store_tile_kappa<BX, BY, BZ, TR>(sk, st);
+    TileStage<BX, BY, BZ, TR, NR> st;
+    load_tile_kappa<BX, BY, BZ, TR, NR>(g, kappa, o, st);
+    if (!zero_in) load_tile_fields<BX, BY, BZ, TR, NR>(g, uin, o, st);
+    store_tile_kappa<BX, BY, BZ, TR, NR>(sk, st);
     if (zero_in) {
       for (int i = t; i < T::kU; i += T::NT) {
 #pragma unroll
-        for (int k = 0; k < OTM_NRHS; k++) su[k][i] = 0.f;
+        for (int k = 0; k < NR; k++) su[k][i] = 0.f;
       }
     } else {
-      store_tile_fields<BX, BY, BZ, TR>(&su[0][0], st);
+      store_tile_fields<BX, BY, BZ, TR, NR>(&su[0][0], st);
     }
   }
   // node ownership: x = tx; of colour (cy, cz) the x-rows rr = ty + TR*h,
@@ -1053,7 +1059,7 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
   const int lx = tx;
   const int wr0 = wave_first_row<BX>(), sub = lane_row<BX>();
   const unsigned nxu = (unsigned)g.nx, nxyu = (unsigned)g.nx * (unsigned)g.ny;
-  float fv[4][H][OTM_NRHS];
+  float fv[4][H][NR];
 #pragma unroll
   for (int col = 0; col < 4; col++)
 #pragma unroll
@@ -1068,7 +1074,7 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
       }
       off = 4u * (off + (unsigned)(ox + lx));
 #pragma unroll
-      for (int k = 0; k < OTM_NRHS; k++) fv[col][h][k] = ld_off(f + (size_t)k * (size_t)g.nn, off);
+      for (int k = 0; k < NR; k++) fv[col][h][k] = ld_off(f + (size_t)k * (size_t)g.nn, off);
     }
   __syncthreads();
   const float c = fc.c;
@@ -1095,24 +1101,24 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
   static_assert(BX == 16 || BX == 32, "tile rows are one DPP row (16) or half a wave (32)");
   const bool send_left = lx != BX - 1;  // T1 goes to lane x + 1 in the same tile row
   const bool send_right = lx != 0;      // T0 goes to lane x - 1
-  float fe[4][H][OTM_NRHS];
+  float fe[4][H][NR];
 #pragma unroll
   for (int col = 0; col < 4; col++)
 #pragma unroll
     for (int h = 0; h < H; h++)
 #pragma unroll
-      for (int k = 0; k < OTM_NRHS; k++) fe[col][h][k] = fv[col][h][k];
+      for (int k = 0; k < NR; k++) fe[col][h][k] = fv[col][h][k];
   if (!zero_in) {
     // halo column x0 - 1 seen by the tile's first column: its T1; halo
     // column x0 + BX seen by the last column: its T0 (frozen values)
-    __shared__ float hterm[2][BY * BZ][OTM_NRHS];
+    __shared__ float hterm[2][BY * BZ][NR];
     for (int i = t; i < 2 * BY * BZ; i += T::NT) {
       const int side = i / (BY * BZ), r = i % (BY * BZ);
       const int ly = r % BY, lz = r / BY;
       const int hx = side ? HX - 1 : 0, kx = side ? BX : 0;
       const int c0 = hx + DY * (ly + 1) + DZ * (lz + 1);
 #pragma unroll
-      for (int k = 0; k < OTM_NRHS; k++) {
+      for (int k = 0; k < NR; k++) {
         const float* U = &su[k][0];
         float T = 0.f;
 #pragma unroll
@@ -1133,60 +1139,92 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
         const int ly = (col & 1) + 2 * (rr % (BY / 2)), lz = (col >> 1) + 2 * (rr / (BY / 2));
         const int r = ly + BY * lz;
 #pragma unroll
-        for (int k = 0; k < OTM_NRHS; k++) {
+        for (int k = 0; k < NR; k++) {
           if (lx == 0) fe[col][h][k] += c * hterm[0][r][k];
           if (lx == BX - 1) fe[col][h][k] += c * hterm[1][r][k];
         }
       }
   }
-  for (int s = 0; s < sweeps; s++)
+  // a node's weights: kappa of the elements (x-1+ax, y-1+ay, z-1+az), K0 for
+  // ax = 0, K1 for ax = 1 (zero where the neighbour is not in the tile)
+  struct Weights {
+    float W[4], K0s[4], K1s[4], inv;
+  };
+  auto weights = [&](int ly, int lz) {
+    Weights w;
+    const int kb = lx + KX * (ly + KY * lz);
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int col = forward ? i : 3 - i;
+    for (int q = 0; q < 4; q++) {
+      const int o = KX * ((q & 1) + KY * (q >> 1));
+      const float K0 = sk[kb + o], K1 = sk[kb + 1 + o];
+      w.W[q] = K0 + K1;
+      w.K1s[q] = send_left ? K1 : 0.f;
+      w.K0s[q] = send_right ? K0 : 0.f;
+    }
+    const float ks = (w.W[0] + w.W[1]) + (w.W[2] + w.W[3]);
+    w.inv = __builtin_amdgcn_rcpf(4.f * c * ks);
+    return w;
+  };
+  Weights held[NR == 1 ? 4 : 1][NR == 1 ? H : 1];
+  if constexpr (NR == 1) {
+#pragma unroll
+    for (int col = 0; col < 4; col++)
 #pragma unroll
       for (int h = 0; h < H; h++) {
         const int rr = ty + TR * h;
-        const int ly = (col & 1) + 2 * (rr % (BY / 2)), lz = (col >> 1) + 2 * (rr / (BY / 2));
-        // kappa of the elements (x-1+ax, y-1+ay, z-1+az): K0 for ax = 0, K1 for ax = 1
-        const int kb = lx + KX * (ly + KY * lz);
-        float K0[4], K1[4], W[4], K0s[4], K1s[4];
+        held[col][h] = weights((col & 1) + 2 * (rr % (BY / 2)), (col >> 1) + 2 * (rr / (BY / 2)));
+      }
+  }
+  for (int s = 0; s < sweeps; s++)
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-          const int o = KX * ((q & 1) + KY * (q >> 1));
-          K0[q] = sk[kb + o];
-          K1[q] = sk[kb + 1 + o];
-          W[q] = K0[q] + K1[q];
-          K1s[q] = send_left ? K1[q] : 0.f;
-          K0s[q] = send_right ? K0[q] : 0.f;
-        }
-        const float ks = (W[0] + W[1]) + (W[2] + W[3]);
-        const float inv = __builtin_amdgcn_rcpf(4.f * c * ks);
-        // rows of the node's own column, addressed from the lowest one so
-        // that every offset (load cases included) is an LDS immediate
-        int cb = (lx + 1) + DY * (ly + 1) + DZ * (lz + 1) - LO;
-        asm volatile("" : "+v"(cb));
+    for (int i = 0; i < 4; i++) {
+      auto step = [&](int col) {
 #pragma unroll
-        for (int k = 0; k < OTM_NRHS; k++) {
-          const float* U = &su[k][0] + cb;
-          const float ym = U[LO - DY], yp = U[LO + DY], zm = U[LO - DZ], zp = U[LO + DZ];
-          const float D[4] = {U[0], U[2 * DY], U[2 * DZ], U[2 * DY + 2 * DZ]};  // (y-+1, z-+1)
-          const float G[4] = {ym + zm + D[0], yp + zm + D[1], ym + zp + D[2], yp + zp + D[3]};
-          float T1 = K1s[0] * G[0], T0 = K0s[0] * G[0], acc = W[0] * D[0];
+        for (int h = 0; h < H; h++) {
+          const int rr = ty + TR * h;
+          const int ly = (col & 1) + 2 * (rr % (BY / 2)), lz = (col >> 1) + 2 * (rr / (BY / 2));
+          Weights w;
+          if constexpr (NR == 1)
+            w = held[col][h];
+          else
+            w = weights(ly, lz);
+          // rows of the node's own column, addressed from the lowest one so
+          // that every offset (load cases included) is an LDS immediate
+          int cb = (lx + 1) + DY * (ly + 1) + DZ * (lz + 1) - LO;
+          asm volatile("" : "+v"(cb));
 #pragma unroll
-          for (int q = 1; q < 4; q++) {
-            T1 += K1s[q] * G[q];
-            T0 += K0s[q] * G[q];
-            acc += W[q] * D[q];
+          for (int k = 0; k < NR; k++) {
+            const float* U = &su[k][0] + cb;
+            const float ym = U[LO - DY], yp = U[LO + DY], zm = U[LO - DZ], zp = U[LO + DZ];
+            const float D[4] = {U[0], U[2 * DY], U[2 * DZ], U[2 * DY + 2 * DZ]};  // (y-+1, z-+1)
+            const float G[4] = {ym + zm + D[0], yp + zm + D[1], ym + zp + D[2], yp + zp + D[3]};
+            float T1 = w.K1s[0] * G[0], T0 = w.K0s[0] * G[0], acc = w.W[0] * D[0];
+#pragma unroll
+            for (int q = 1; q < 4; q++) {
+              T1 += w.K1s[q] * G[q];
+              T0 += w.K0s[q] * G[q];
+              acc += w.W[q] * D[q];
+            }
+            acc += from_left(T1);
+            acc += from_right(T0);
+            (&su[k][0] + cb)[LO] = (fe[col][h][k] + c * acc) * w.inv;
           }
-          acc += from_left(T1);
-          acc += from_right(T0);
-          (&su[k][0] + cb)[LO] = (fe[col][h][k] + c * acc) * inv;
         }
+      };
+      if constexpr (NR == 1) {  // static colours, so that held stays in registers
+        if (forward)
+          step(i);
+        else
+          step(3 - i);
+      } else {
+        step(forward ? i : 3 - i);
       }
       __syncthreads();
     }
   if (dot) {
-    double acc[OTM_NRHS] = {0.0, 0.0, 0.0};
+    double acc[NR];
+#pragma unroll
+    for (int k = 0; k < NR; k++) acc[k] = 0.0;
 #pragma unroll
     for (int col = 0; col < 4; col++)
 #pragma unroll
@@ -1195,9 +1233,22 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
         const int ly = (col & 1) + 2 * (rr % (BY / 2)), lz = (col >> 1) + 2 * (rr / (BY / 2));
         const int c0 = (lx + 1) + DY * (ly + 1) + DZ * (lz + 1);
 #pragma unroll
-        for (int k = 0; k < OTM_NRHS; k++) acc[k] += (double)fv[col][h][k] * (double)su[k][c0];
+        for (int k = 0; k < NR; k++) acc[k] += (double)fv[col][h][k] * (double)su[k][c0];
       }
-    reduce_block_at<OTM_NRHS>(acc, RD, b);
+    constexpr int kW = T::NT / 64;
+    __shared__ double sh[NR * kW];
+#pragma unroll
+    for (int k = 0; k < NR; k++) {
+      const double v = wave_sum(acc[k]);
+      if ((t & 63) == 0) sh[k * kW + (t >> 6)] = v;
+    }
+    __syncthreads();
+    if (t < NR) {
+      double v = 0.0;
+#pragma unroll
+      for (int w = 0; w < kW; w++) v += sh[t * kW + w];
+      RD.partials[(size_t)b * OTM_NRHS + k0 + t] = v;
+    }
   }
   static_assert((BY * BZ) % TR == 0, "thread rows must divide the tile's rows");
 #pragma unroll
@@ -1214,7 +1265,7 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
     const int ly = r % BY, lz = r / BY;
     const int c0 = (tx + 1) + DY * (ly + 1) + DZ * (lz + 1);
 #pragma unroll
-    for (int k = 0; k < OTM_NRHS; k++) *(float*)((char*)(uout + (size_t)k * (size_t)g.nn) + off) = su[k][c0];
+    for (int k = 0; k < NR; k++) *(float*)((char*)(uout + (size_t)k * (size_t)g.nn) + off) = su[k][c0];
   }
 }
 
