@@ -220,10 +220,8 @@ OTM_API int otm_conv_filter(const int reso[3], int kind, double radius, int peri
  * under HIP graph capture, serving loops): no counterpart in the reference.
  * in and out are device arrays of the current device that must not overlap;
  * the launches go on `stream` (a hipStream_t; null = the default stream) and
- * the call returns without waiting for them. The weight sums live in a
- * static device array of 2^23 floats (32 MiB per device, kept until the
- * process ends): larger cells get OTM_E_UNSUPPORTED. Every call on a device
- * shares that array, so calls whose launches overlap on one GPU race. */
+ * the call returns without waiting for them. Cells of more than 2^23 nodes
+ * get OTM_E_UNSUPPORTED. Calls share nothing, so they may overlap. */
 OTM_API int otm_conv_filter_noalloc(const int reso[3], int kind, double radius, int periodic, int adjoint,
                                     const float* in, float* out, void* stream);
 

@@ -150,13 +150,12 @@ struct otm_ctx {
   unsigned hm_tag = 0;             // tag of the last finaliser asked to publish
   bool hm_pending = false;         // that finaliser's results not yet taken
   // design pipeline
-  float *rho = nullptr, *rho_f = nullptr, *W = nullptr, *kraw = nullptr, *dkappa = nullptr;
+  float *rho = nullptr, *rho_f = nullptr, *kraw = nullptr, *dkappa = nullptr;
   float *tmp = nullptr, *drho = nullptr;
   Taps taps;
   int taps_kind = -2;
   double taps_r = 0;
   int taps_periodic = -1;
-  bool w_valid = false;  // W holds the weight sums of these taps (they depend on the taps alone)
   // live kernel timing (otm_profile_enable)
   bool prof_on = false;
   int prof_mask = 0;

@@ -159,7 +159,7 @@ static void ctx_free(otm_ctx* c) {
   if (c->pcg_host) (void)hipHostFree(c->pcg_host);
   if (c->out_host) (void)hipHostFree(c->out_host);
   if (c->hm) (void)hipHostFree(c->hm);
-  dfree(c->rho); dfree(c->rho_f); dfree(c->W); dfree(c->kraw); dfree(c->dkappa);
+  dfree(c->rho); dfree(c->rho_f); dfree(c->kraw); dfree(c->dkappa);
   dfree(c->tmp); dfree(c->drho);
   for (auto& p : c->pending) {
     (void)hipEventDestroy(p.a);
@@ -720,7 +720,6 @@ static void ensure_design_buffers(otm_ctx* c) {
   const long long n = c->g0.nn;
   c->rho = dalloc<float>(n);
   c->rho_f = dalloc<float>(n);
-  c->W = dalloc<float>(n);
   c->kraw = dalloc<float>(n);
   launch_fill(c->s, c->kraw, n, 0.f);
   c->dkappa = dalloc<float>(n);
@@ -1410,51 +1409,27 @@ OTM_API int otm_conv_filter(const int reso[3], int kind, double radius, int peri
     Geom g{reso[0], reso[1], reso[2], (long long)reso[0] * reso[1] * reso[2]};
     float* din = dalloc<float>(g.nn);
     float* dout = dalloc<float>(g.nn);
-    float* dW = dalloc<float>(g.nn);
-    float* dtmp = dalloc<float>(g.nn);
     hipStream_t s = nullptr;
     hipError_t e = hipMemcpy(din, in, sizeof(float) * g.nn, kind_of(OTM_DEVICE, where));
     if (e == hipSuccess) {
       if (adjoint) {
-        launch_filter_fwd(s, g, T, din, dtmp, dW);  // weight sums W
-        launch_filter_adj(s, g, T, din, dW, dout);
+        launch_filter_adj(s, g, T, din, dout);
       } else {
-        launch_filter_fwd(s, g, T, din, dout, dW);
+        launch_filter_fwd(s, g, T, din, dout);
       }
       e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpy(out, dout, sizeof(float) * g.nn, kind_of(where, OTM_DEVICE));
-    dfree(din); dfree(dout); dfree(dW); dfree(dtmp);
+    dfree(din); dfree(dout);
     hip_check(e, "conv filter");
   });
 }
 
 // ---- the filter without allocation --------------------------------------------
-// Scratch of otm_conv_filter_noalloc: the per-node weight sums W of one
-// cell, at most kNoAllocNodes floats (32 MiB on every device the library
-// runs on, held until the process ends). In host code `scratch` names a
-// host-side stand-in: its device address comes from hipGetSymbolAddress,
-// once per device with that device current, and only that address is
-// handed to kernels.
+// The filter kernels take their weights and weight sums as arguments, so the
+// entry point needs no scratch memory at all. Cells stay limited to
+// kNoAllocNodes.
 constexpr long long kNoAllocNodes = 1ll << 23;
-static __device__ __align__(256) float scratch[kNoAllocNodes];
-constexpr int kNoAllocMaxDevices = 64;
-static std::mutex g_scratch_mu;
-static float* g_scratch_dev[kNoAllocMaxDevices];
-
-static float* scratch_of_current_device() {
-  int dev = 0;
-  hip_check(hipGetDevice(&dev), "hipGetDevice");
-  if (dev < 0 || dev >= kNoAllocMaxDevices) fail(OTM_E_UNSUPPORTED, "device index beyond the scratch table");
-  std::lock_guard<std::mutex> lk(g_scratch_mu);
-  if (!g_scratch_dev[dev]) {
-    void* p = nullptr;
-    hip_check(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)), "hipGetSymbolAddress(scratch)");
-    if (!p) fail(OTM_E_HIP, "hipGetSymbolAddress(scratch) returned null");
-    g_scratch_dev[dev] = (float*)p;
-  }
-  return g_scratch_dev[dev];
-}
 
 OTM_API int otm_conv_filter_noalloc(const int reso[3], int kind, double radius, int periodic, int adjoint,
                                     const float* in, float* out, void* stream) {
@@ -1464,16 +1439,16 @@ OTM_API int otm_conv_filter_noalloc(const int reso[3], int kind, double radius, 
       if (reso[a] <= 0) fail(OTM_E_ARG, "reso must be positive");
     const long long n = (long long)reso[0] * reso[1] * reso[2];
     if (n > kNoAllocNodes)
-      fail(OTM_E_UNSUPPORTED, "cell exceeds the no-allocation filter's scratch of 8388608 nodes");
-    // the adjoint writes the forward output to out before it reads in again
+      fail(OTM_E_UNSUPPORTED, "cell exceeds the 8388608 nodes of the filter without scratch memory");
+    // a tile reads its neighbours' inputs
     if (in < out + n && out < in + n) fail(OTM_E_ARG, "in and out overlap");
-    float* W = scratch_of_current_device();
     const Taps T = make_taps(kind, radius, periodic);
     const Geom g{reso[0], reso[1], reso[2], n};
     hipStream_t s = (hipStream_t)stream;
-    // the forward pass writes every node's weight sum before any read of W
-    launch_filter_fwd(s, g, T, in, out, W);
-    if (adjoint) launch_filter_adj(s, g, T, in, W, out);
+    if (adjoint)
+      launch_filter_adj(s, g, T, in, out);
+    else
+      launch_filter_fwd(s, g, T, in, out);
     hip_check(hipGetLastError(), "conv filter");
   });
 }
@@ -1823,10 +1798,8 @@ static void apply_design(otm_ctx* ctx, const otm_density_params* p) {
         ctx->taps_kind = p->filter_kind;
         ctx->taps_r = p->filter_radius;
         ctx->taps_periodic = p->filter_periodic;
-        ctx->w_valid = false;
       }
-      launch_filter_fwd(ctx->s, ctx->g0, ctx->taps, ctx->rho, ctx->rho_f, ctx->W, ctx->w_valid);
-      ctx->w_valid = true;
+      launch_filter_fwd(ctx->s, ctx->g0, ctx->taps, ctx->rho, ctx->rho_f);
       src = ctx->rho_f;
     }
     launch_simp_fwd(ctx->s, n, src, (float)ctx->cfg.heat_ratio[0], (float)ctx->cfg.heat_ratio[1], 0.f, ctx->kraw,
@@ -1863,7 +1836,7 @@ OTM_API int otm_backward(otm_ctx* ctx, const double dC[9], float* drho, int wher
     sens_weights(dC, w);
     launch_sensitivity(ctx, w, ctx->tmp, ctx->g0.nx, ctx->dkappa);  // times d kappa / d rho
     if (ctx->taps_kind >= 0)
-      launch_filter_adj(ctx->s, ctx->g0, ctx->taps, ctx->tmp, ctx->W, ctx->drho);
+      launch_filter_adj(ctx->s, ctx->g0, ctx->taps, ctx->tmp, ctx->drho);
     else
       hip_check(hipMemcpyAsync(ctx->drho, ctx->tmp, sizeof(float) * n, hipMemcpyDeviceToDevice, ctx->s), "copy");
     if (drho) {

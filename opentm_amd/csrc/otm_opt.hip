@@ -16,98 +16,153 @@ namespace otm {
 static inline unsigned nblk(long long n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
 // ---- filters, LDS-tiled ----
-// A block computes a 32 x 8 x 4 box of outputs (thread (x, y), four z) from
-// an LDS copy of the box grown by the taps' reach h (at most 3) on every
-// side, so each input comes from HBM about twice (halo) instead of once per
-// tap. Positions outside a non-periodic cell hold 0, which leaves the sums
-// as if the tap were skipped. Taps become offsets into that copy.
-constexpr int kFtX = 32, kFtY = 8, kFtZ = 4, kFtH = 3;
-constexpr int kFtLds = (kFtX + 2 * kFtH) * (kFtY + 2 * kFtH) * (kFtZ + 2 * kFtH);
+// The taps are radial, so a weight depends on (|dx|, |dy|, |dz|) alone, in
+// any order of the three; the weight sum W of a node of a non-periodic cell
+// depends on how many taps each face cuts off, min(distance to the face, H)
+// for a cell of at least 2H nodes along the axis (the node's coordinate
+// itself for a shorter one, or where the axis has as few nodes as classes). Both are small tables, so no pass over the
+// nodes forms W and no array holds it.
+constexpr int kFtH = 3;                                    // largest reach of a tap
+constexpr int kFtClasses = 2 * kFtH - 1;                   // weight-sum classes per axis, at most
+struct FilterTable {
+  float w[(kFtH + 1) * (kFtH + 1) * (kFtH + 1)];           // |dx| + (H+1) (|dy| + (H+1) |dz|)
+  float W[kFtClasses * kFtClasses * kFtClasses];           // cx + K[0] (cy + K[1] cz)
+  float wall;                                              // sum of all weights
+  int K[3];
+  int periodic;
+};
+__host__ __device__ inline int filter_class(int x, int n, int K, int H) {
+  return K == n ? x : min(min(x, n - 1 - x), H);
+}
+
+// A block computes a 32 x 8 x Z box of outputs (thread (x, y), Z along z)
+// from an LDS copy of the box grown by the reach H on every side, so each
+// input comes from HBM about 1.7 (H = 1) times instead of once per tap.
+// Positions outside a non-periodic cell hold 0, which leaves the sums as if
+// the tap were skipped. A thread first adds the up to eight columns of equal
+// (|dx|, |dy|) over its Z + 2H positions and then applies the class's 2H + 1
+// weights: at H = 1, 90 LDS reads and 146 operations for 8 outputs, 406 and
+// 862 at radius 3, where a read and a multiply-add per tap (and two reads
+// for the tap itself per 4 outputs) took 228 and 1476.
+// Bound by HBM at large cells (8 bytes a node, 12 for FILT_SENS) and by the
+// staging's latency at small ones: all its loads are issued before the first
+// LDS store. Radius 1.5, forward / adjoint at 256^3: 52 and 52 us (176 and
+// 112 with a tap at a time and runtime index divisions in the staging), 128^3
+// 11 and 12 us (22 and 20); a lone adjoint needs no forward pass for W.
+constexpr int kFtX = 32, kFtY = 8;
 static_assert(kFtX * kFtY == kBlock, "one thread per (x, y) column of a filter tile");
 enum { FILT_FWD = 0, FILT_ADJ = 1, FILT_SENS = 2 };
 
-// FILT_FWD: out = sum w in / W and W = sum of the weights of the taps
-// inside the cell (all taps when periodic; W may be null).
-// FILT_ADJ: out_j = sum_i w in_i / W_i over the reversed taps (b = W).
+// FILT_FWD: out = sum w in / W. FILT_ADJ: out_j = sum_i w in_i / W_i.
 // FILT_SENS: out = sum w (sens rho) / (W rho), periodic (a = sens, b = rho).
-// wall is the sum of all tap weights in tap order (the W of an output whose
-// taps are all inside).
-// w_known (FILT_FWD): W already holds the weight sums (a previous call with
-// the same taps wrote them); nodes near a non-periodic cell's faces read
-// theirs instead of summing the taps again.
-template <int MODE>
-__global__ void __launch_bounds__(kBlock) k_filter_tile(Geom g, Taps T, int h, float wall, const float* __restrict__ a,
-                                                        const float* __restrict__ b, float* __restrict__ out,
-                                                        float* __restrict__ W, int w_known) {
-  __shared__ float tile[kFtLds];
-  __shared__ int toff[kMaxTaps];
-  __shared__ float tw[kMaxTaps];
-  const int SX = kFtX + 2 * h, SY = kFtY + 2 * h, SZ = kFtZ + 2 * h;
+template <int MODE, int H, int Z>
+__global__ void __launch_bounds__(kBlock) k_filter_tile(Geom g, FilterTable F, const float* __restrict__ a,
+                                                        const float* __restrict__ b, float* __restrict__ out) {
+  constexpr int SX = kFtX + 2 * H, SY = kFtY + 2 * H, SZ = Z + 2 * H;
+  constexpr int R = SY * SZ;                                   // x-rows of the copy
+  constexpr int TR = (R + kFtY - 1) / kFtY;                    // of them per thread row
+  constexpr int TH = (2 * H * R + kBlock - 1) / kBlock;        // x-halo positions per thread
+  constexpr int T = TR + TH;
+  __shared__ float tile[R * SX];
+  __shared__ float sW[MODE == FILT_SENS ? 1 : kFtClasses * kFtClasses * kFtClasses];
   const int ntx = (g.nx + kFtX - 1) / kFtX, nty = (g.ny + kFtY - 1) / kFtY;
   const int bx = (int)blockIdx.x % ntx, byz = (int)blockIdx.x / ntx;
-  const int x0 = bx * kFtX, y0 = (byz % nty) * kFtY, z0 = (byz / nty) * kFtZ;
-  const bool periodic = MODE == FILT_SENS || T.periodic;
-  for (int i = threadIdx.x; i < T.n; i += kBlock) {
-    const int o = T.dx[i] + SX * (T.dy[i] + SY * T.dz[i]);
-    toff[i] = MODE == FILT_ADJ ? -o : o;
-    tw[i] = T.w[i];
-  }
-  for (int i = threadIdx.x; i < SX * SY * SZ; i += kBlock) {
-    const int lx = i % SX, rest = i / SX;
-    int X = x0 - h + lx, Y = y0 - h + rest % SY, Z = z0 - h + rest / SY;
-    float v = 0.f;
-    // positions past the cell by more than h feed no output of this tile
-    if (X < g.nx + h && Y < g.ny + h && Z < g.nz + h) {
-      const bool inside = X >= 0 && X < g.nx && Y >= 0 && Y < g.ny && Z >= 0 && Z < g.nz;
-      if (inside || periodic) {
-        X = wrapm(X, g.nx);
-        Y = wrapm(Y, g.ny);
-        Z = wrapm(Z, g.nz);
-        const long long j = (long long)X + (long long)g.nx * ((long long)Y + (long long)g.ny * Z);
-        v = MODE == FILT_FWD ? a[j] : (MODE == FILT_ADJ ? a[j] / b[j] : a[j] * b[j]);
-      }
+  const int x0 = bx * kFtX, y0 = (byz % nty) * kFtY, z0 = (byz / nty) * Z;
+  const int tx = threadIdx.x % kFtX, ty = threadIdx.x / kFtX;
+  const bool periodic = MODE == FILT_SENS || F.periodic;
+  // position t of this thread: LDS row and column
+  auto place = [&](int t, int& row, int& col) {
+    if (t < TR) {
+      row = ty + kFtY * t;
+      col = H + tx;
+    } else {
+      const int i = (int)threadIdx.x + kBlock * (t - TR), c = i % (2 * H);
+      row = i / (2 * H);
+      col = c < H ? c : kFtX + c;
     }
-    tile[i] = v;
+  };
+  float va[T], vb[T];
+  bool ok[T];
+  int cls[T];
+#pragma unroll
+  for (int t = 0; t < T; t++) {
+    int row, col;
+    place(t, row, col);
+    row = min(row, R - 1);
+    const int X = x0 - H + col, Y = y0 - H + row % SY, Zc = z0 - H + row / SY;
+    // periodic: positions past the cell by more than H feed no output
+    ok[t] = periodic ? (X < g.nx + H && Y < g.ny + H && Zc < g.nz + H)
+                     : (X >= 0 && X < g.nx && Y >= 0 && Y < g.ny && Zc >= 0 && Zc < g.nz);
+    const int Xw = ok[t] ? wrapm(X, g.nx) : 0, Yw = ok[t] ? wrapm(Y, g.ny) : 0, Zw = ok[t] ? wrapm(Zc, g.nz) : 0;
+    const unsigned j = 4u * ((unsigned)Xw + (unsigned)g.nx * ((unsigned)Yw + (unsigned)g.ny * (unsigned)Zw));
+    va[t] = ld_off(a, j);
+    if (MODE == FILT_SENS) vb[t] = ld_off(b, j);
+    if (MODE == FILT_ADJ)
+      cls[t] = filter_class(Xw, g.nx, F.K[0], H) +
+               F.K[0] * (filter_class(Yw, g.ny, F.K[1], H) + F.K[1] * filter_class(Zw, g.nz, F.K[2], H));
+  }
+  if (MODE != FILT_SENS && !periodic) {
+    const int n = F.K[0] * F.K[1] * F.K[2];
+    if ((int)threadIdx.x < n) sW[threadIdx.x] = F.W[threadIdx.x];
+    if (MODE == FILT_ADJ) __syncthreads();
+  }
+#pragma unroll
+  for (int t = 0; t < T; t++) {
+    int row, col;
+    place(t, row, col);
+    float v = va[t];
+    if (MODE == FILT_ADJ) v = v / (periodic ? F.wall : sW[cls[t]]);
+    if (MODE == FILT_SENS) v = v * vb[t];
+    if (row < R) tile[row * SX + col] = ok[t] ? v : 0.f;
   }
   __syncthreads();
-  const int tx = threadIdx.x % kFtX, ty = threadIdx.x / kFtX;
   const int x = x0 + tx, y = y0 + ty;
   if (x >= g.nx || y >= g.ny) return;
-  const int plane = SX * SY;
-  const int c0 = (tx + h) + SX * ((ty + h) + SY * h);
-  float acc[kFtZ] = {0.f, 0.f, 0.f, 0.f};
-  for (int i = 0; i < T.n; i++) {
-    const int o = c0 + toff[i];
-    const float w = tw[i];
+  constexpr int plane = SX * SY;
+  const float* base = tile + (tx + H) + SX * (ty + H);
+  float acc[Z];
 #pragma unroll
-    for (int k = 0; k < kFtZ; k++) acc[k] = fmaf(w, tile[o + k * plane], acc[k]);
-  }
+  for (int k = 0; k < Z; k++) acc[k] = 0.f;
 #pragma unroll
-  for (int k = 0; k < kFtZ; k++) {
+  for (int i = 0; i <= H; i++)
+#pragma unroll
+    for (int j = 0; j <= i; j++) {
+      const float* w = F.w + i + (H + 1) * j;
+      if (w[0] == 0.f) continue;  // beyond the radius
+      float s[SZ];
+#pragma unroll
+      for (int q = 0; q < SZ; q++) {
+        const float* u = base + q * plane;
+        float v = 0.f;
+#pragma unroll
+        for (int c = 0; c < 8; c++) {  // the distinct ones of (+-i, +-j), (+-j, +-i)
+          const bool swap = c & 1, ni = c & 2, nj = c & 4;
+          if ((swap && i == j) || (ni && i == 0) || (nj && j == 0)) continue;
+          const int dx = swap ? (nj ? -j : j) : (ni ? -i : i), dy = swap ? (ni ? -i : i) : (nj ? -j : j);
+          v += u[dx + SX * dy];
+        }
+        s[q] = v;
+      }
+#pragma unroll
+      for (int d = 0; d <= H; d++) {
+        const float wd = w[(H + 1) * (H + 1) * d];
+        if (wd == 0.f) break;
+#pragma unroll
+        for (int k = 0; k < Z; k++) acc[k] = fmaf(wd, d ? s[k + H - d] + s[k + H + d] : s[k + H], acc[k]);
+      }
+    }
+  const int cxy = filter_class(x, g.nx, F.K[0], H) + F.K[0] * filter_class(y, g.ny, F.K[1], H);
+#pragma unroll
+  for (int k = 0; k < Z; k++) {
     const int z = z0 + k;
     if (z >= g.nz) break;
     const long long t = (long long)x + (long long)g.nx * ((long long)y + (long long)g.ny * z);
-    if (MODE == FILT_ADJ) {
+    if (MODE == FILT_ADJ)
       out[t] = acc[k];
-    } else if (MODE == FILT_SENS) {
-      out[t] = acc[k] / (wall * b[t]);
-    } else {
-      float ws = wall;
-      const bool interior = x >= h && x + h < g.nx && y >= h && y + h < g.ny && z >= h && z + h < g.nz;
-      if (!periodic && !interior) {
-        if (w_known) {
-          ws = W[t];
-        } else {
-          ws = 0.f;
-          for (int i = 0; i < T.n; i++) {
-            const int X = x + T.dx[i], Y = y + T.dy[i], Z = z + T.dz[i];
-            if (X >= 0 && X < g.nx && Y >= 0 && Y < g.ny && Z >= 0 && Z < g.nz) ws += tw[i];
-          }
-        }
-      }
-      out[t] = acc[k] / ws;
-      if (W && !w_known) W[t] = ws;
-    }
+    else if (MODE == FILT_SENS)
+      out[t] = acc[k] / (F.wall * b[t]);
+    else
+      out[t] = acc[k] / (periodic ? F.wall : sW[cxy + F.K[0] * F.K[1] * filter_class(z, g.nz, F.K[2], H)]);
   }
 }
 
@@ -603,36 +658,94 @@ void launch_scale_clamp(hipStream_t s, long long n, float* v, float scale, float
   hipLaunchKernelGGL(k_scale_clamp, dim3(nblk(n)), dim3(kBlock), 0, s, n, v, scale, lo, hi);
 }
 
-// Reach of the taps (largest offset along any axis) and the sum of all
-// weights in tap order, in FP32 as the kernel adds them.
-static void tap_stats(const Taps& T, int& h, float& wall) {
-  h = 0;
-  wall = 0.f;
-  for (int i = 0; i < T.n; i++) {
+// Reach of the taps (largest offset along any axis).
+static int tap_reach(const Taps& T) {
+  int h = 0;
+  for (int i = 0; i < T.n; i++)
     h = std::max(h, std::max(std::abs((int)T.dx[i]), std::max(std::abs((int)T.dy[i]), std::abs((int)T.dz[i]))));
-    wall += T.w[i];
+  return h;
+}
+
+// The kernel's tables for a kernel reach of H >= the taps'. W is summed in
+// FP64, one axis after another.
+static FilterTable filter_table(const Geom& g, const Taps& T, int H) {
+  FilterTable F = {};
+  const int n[3] = {g.nx, g.ny, g.nz}, D = 2 * H + 1, e = H + 1;
+  double all = 0.0;
+  for (int i = 0; i < T.n; i++) {
+    all += (double)T.w[i];
+    if (T.dx[i] >= 0 && T.dy[i] >= 0 && T.dz[i] >= 0) F.w[T.dx[i] + e * (T.dy[i] + e * T.dz[i])] = T.w[i];
+  }
+  F.wall = (float)all;
+  F.periodic = T.periodic;
+  for (int a = 0; a < 3; a++) F.K[a] = n[a] >= 2 * H ? e : n[a];
+  if (T.periodic) return F;
+  constexpr int kD = 2 * kFtH + 1;
+  double s1[kFtClasses][kD][kD], s2[kFtClasses][kFtClasses][kD];
+  // a class is a coordinate where there are as many (as in filter_class), a
+  // distance to one face otherwise
+  auto inside = [&](int a, int c, int d) { return c + d >= 0 && (F.K[a] != n[a] || c + d < n[a]); };
+  auto weight = [&](int dx, int dy, int dz) {
+    return (double)F.w[std::abs(dx) + e * (std::abs(dy) + e * std::abs(dz))];
+  };
+  for (int c = 0; c < F.K[0]; c++)
+    for (int y = 0; y < D; y++)
+      for (int z = 0; z < D; z++) {
+        s1[c][y][z] = 0.0;
+        for (int d = -H; d <= H; d++)
+          if (inside(0, c, d)) s1[c][y][z] += weight(d, y - H, z - H);
+      }
+  for (int c = 0; c < F.K[0]; c++)
+    for (int c1 = 0; c1 < F.K[1]; c1++)
+      for (int z = 0; z < D; z++) {
+        s2[c][c1][z] = 0.0;
+        for (int d = -H; d <= H; d++)
+          if (inside(1, c1, d)) s2[c][c1][z] += s1[c][d + H][z];
+      }
+  for (int c = 0; c < F.K[0]; c++)
+    for (int c1 = 0; c1 < F.K[1]; c1++)
+      for (int c2 = 0; c2 < F.K[2]; c2++) {
+        double v = 0.0;
+        for (int d = -H; d <= H; d++)
+          if (inside(2, c2, d)) v += s2[c][c1][d + H];
+        F.W[c + F.K[0] * (c1 + F.K[1] * c2)] = (float)v;
+      }
+  return F;
+}
+
+template <int MODE, int H, int Z>
+static void launch_filter_hz(hipStream_t s, const Geom& g, const Taps& T, const float* a, const float* b, float* out) {
+  const unsigned nb = (unsigned)(((g.nx + kFtX - 1) / kFtX) * ((g.ny + kFtY - 1) / kFtY) * ((g.nz + Z - 1) / Z));
+  const FilterTable F = filter_table(g, T, H);
+  hipLaunchKernelGGL((k_filter_tile<MODE, H, Z>), dim3(nb), dim3(kBlock), 0, s, g, F, a, b, out);
+}
+template <int MODE, int H>
+static void launch_filter_h(hipStream_t s, const Geom& g, const Taps& T, const float* a, const float* b, float* out) {
+  // Z = 4 gives a small cell twice the workgroups (48^3 5.6 against 8.0 us),
+  // Z = 8 a large one the smaller halo (256^3 52 against 61 us; even at 128^3)
+  if (g.nn <= (1ll << 22))
+    launch_filter_hz<MODE, H, 4>(s, g, T, a, b, out);
+  else
+    launch_filter_hz<MODE, H, 8>(s, g, T, a, b, out);
+}
+template <int MODE>
+static void launch_filter_tile(hipStream_t s, const Geom& g, const Taps& T, const float* a, const float* b,
+                               float* out) {
+  const int h = tap_reach(T);
+  if (h > kFtH || T.n > kMaxTaps) throw std::invalid_argument("filter taps reach beyond 3 cells");
+  if (h > g.nx || h > g.ny || h > g.nz) throw std::invalid_argument("filter reach exceeds the cell");
+  switch (h) {
+    case 3: launch_filter_h<MODE, 3>(s, g, T, a, b, out); break;
+    case 2: launch_filter_h<MODE, 2>(s, g, T, a, b, out); break;
+    default: launch_filter_h<MODE, 1>(s, g, T, a, b, out); break;
   }
 }
 
-template <int MODE>
-static void launch_filter_tile(hipStream_t s, const Geom& g, const Taps& T, const float* a, const float* b,
-                               float* out, float* W, bool w_known = false) {
-  int h;
-  float wall;
-  tap_stats(T, h, wall);
-  if (h > kFtH || T.n > kMaxTaps) throw std::invalid_argument("filter taps reach beyond 3 cells");
-  if (h > g.nx || h > g.ny || h > g.nz) throw std::invalid_argument("filter reach exceeds the cell");
-  const unsigned nb = (unsigned)(((g.nx + kFtX - 1) / kFtX) * ((g.ny + kFtY - 1) / kFtY) * ((g.nz + kFtZ - 1) / kFtZ));
-  hipLaunchKernelGGL(k_filter_tile<MODE>, dim3(nb), dim3(kBlock), 0, s, g, T, h, wall, a, b, out, W,
-                     (int)(w_known && W));
+void launch_filter_fwd(hipStream_t s, const Geom& g, const Taps& T, const float* in, float* out) {
+  launch_filter_tile<FILT_FWD>(s, g, T, in, nullptr, out);
 }
-
-void launch_filter_fwd(hipStream_t s, const Geom& g, const Taps& T, const float* in, float* out, float* W,
-                       bool w_known) {
-  launch_filter_tile<FILT_FWD>(s, g, T, in, nullptr, out, W, w_known);
-}
-void launch_filter_adj(hipStream_t s, const Geom& g, const Taps& T, const float* in, const float* W, float* out) {
-  launch_filter_tile<FILT_ADJ>(s, g, T, in, W, out, nullptr);
+void launch_filter_adj(hipStream_t s, const Geom& g, const Taps& T, const float* in, float* out) {
+  launch_filter_tile<FILT_ADJ>(s, g, T, in, nullptr, out);
 }
 void launch_simp_fwd(hipStream_t s, long long n, const float* rho, float k0, float k1, float floor_, float* kappa,
                      float* dkappa) {
@@ -643,7 +756,7 @@ void launch_mul(hipStream_t s, long long n, const float* a, const float* b, floa
 }
 void launch_oc_filter_sens(hipStream_t s, const Geom& g, const Taps& T, const float* sens, const float* rho,
                            float* out) {
-  launch_filter_tile<FILT_SENS>(s, g, T, sens, rho, out, nullptr);
+  launch_filter_tile<FILT_SENS>(s, g, T, sens, rho, out);
 }
 void launch_maxabs(hipStream_t s, long long n, const float* a, unsigned int* out_bits) {
   unsigned nb = nblk(n);
