@@ -110,7 +110,8 @@ OTM_API int otm_update(otm_ctx* ctx, const float* kappa, int pitch, int where);
 OTM_API int otm_heat_matrix(otm_ctx* ctx, double C[9]);
 
 /* Fine smoother tile shapes: variant 0..4 -> shape = {bx, by, bz, threads};
- * otm_fine_tile gives the context's variant (-1: exact colour sweeps). */
+ * otm_fine_tile gives the context's variant (-1: edges that are multiples of
+ * none of them; ragged 32x4x8 or 16x4x8 tiles, or exact colour sweeps). */
 OTM_API int otm_fine_tile_shape(int variant, int shape[4]);
 OTM_API int otm_fine_tile(const otm_ctx* ctx, int* variant);
 

@@ -235,7 +235,8 @@ class Homogenization_H:
 
     def fine_tile(self):
         """The fine smoother's tile variant and shape (bx, by, bz, threads),
-        or (-1, None) when the fine level uses exact colour sweeps."""
+        or (-1, None) when the fine level uses ragged tiles or exact colour
+        sweeps."""
         v = ctypes.c_int()
         _capi.check(_capi.load().otm_fine_tile(self._ctx, ctypes.byref(v)), "otm_fine_tile")
         return v.value, (fine_tile_shape(v.value) if v.value >= 0 else None)

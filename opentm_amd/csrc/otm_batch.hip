@@ -48,6 +48,7 @@ struct CellDev {
   int nlev;
   int tail;  // first level of the one-workgroup tail V-cycle
   int fine_bx;  // 32 or 16: fine brick width; 0: exact colour sweeps
+  int fine_rag;  // the bricks are ragged tiles
   int tile_bx;  // 32 or 16: LDS tile width of the fine residual and apply; 0: pointwise kernels
   int sweeps_fine, sweeps_coarse;
   FineConsts fc;
@@ -130,7 +131,7 @@ __global__ void __launch_bounds__(Op::kThreads) kb_run(const Ent* __restrict__ e
 }
 
 // Fine bricks keep the single-cell kernel's occupancy hint.
-template <int BX>
+template <int BX, bool RAG>
 __global__ void __launch_bounds__(BX * kFineTR) __attribute__((amdgpu_waves_per_eu(4, 8)))
 kb_fine_brick(const Ent* __restrict__ ents, int nents, const CellDev* __restrict__ cells, int post) {
   const int b = xcd_block();
@@ -140,9 +141,9 @@ kb_fine_brick(const Ent* __restrict__ ents, int nents, const CellDev* __restrict
   const int sw = C.sweeps_fine;
   Reduce R = cell_reduce(C, FIN_STORE);
   R.partials = C.tile_partials;
-  fine_brick_body<BX>(C.g[0], C.fc, C.kappa, C.f[0], post ? ucur(C, e.par, 0) : nullptr,
-                      post ? uoth(C, e.par, 0) : ucur(C, e.par, 0), sw, post ? 0 : 1, post ? 0 : 1, b - e.block0,
-                      post, R);
+  fine_brick_body<BX, kFineBY, kFineBZ, kFineTR, OTM_NRHS, RAG>(
+      C.g[0], C.fc, C.kappa, C.f[0], post ? ucur(C, e.par, 0) : nullptr, post ? uoth(C, e.par, 0) : ucur(C, e.par, 0),
+      sw, post ? 0 : 1, post ? 0 : 1, b - e.block0, post, R);
 }
 
 // ---- operations (one functor per batched launch) ---------------------------
@@ -273,7 +274,7 @@ struct OpFinal {  // one block per cell
     if (tiled == 1 && C.tile_bx) nb = fine_apply_tile_blocks(C.g[0], C.tile_bx);
     if (tiled == 2 && C.fine_bx) {
       R.partials = C.tile_partials;
-      nb = (unsigned)fine_tiles(C.g[0], C.fine_bx);
+      nb = (unsigned)(C.fine_rag ? fine_ragged_tiles(C.g[0], C.fine_bx) : fine_tiles(C.g[0], C.fine_bx));
       if (nb > (unsigned)kMaxReduceBlocks) {  // as launch_reduce_final
         reduce_final_many_nv<OTM_NRHS>(R, (int)nb);
         return;
@@ -515,6 +516,13 @@ struct otm_batch {
 
 namespace {
 
+// tile width of a cell's fine brick smoother (0: exact colour sweeps)
+int smooth_tile_x(const otm_ctx* c) {
+  if (!c->lv[0].brick) return 0;
+  const int bx = fine_brick_x(c->g0);
+  return bx ? bx : fine_ragged_x(c->g0);
+}
+
 void ensure_cells(otm_batch* b, int n) {
   if (n <= b->dcap) return;
   if (b->s) hip_check(hipStreamSynchronize(b->s), "hipStreamSynchronize");  // no launch still reads them
@@ -565,7 +573,8 @@ CellDev describe(const Member& m) {
   // the batched launches run the default fine tile shape
   if (c->lv[0].brick && c->fine_tile != fine_tile_default(c->g0))
     fail(OTM_E_UNSUPPORTED, "the batched form runs the default fine tile shape (otm_config.fine_tile = -1)");
-  d.fine_bx = c->lv[0].brick ? fine_brick_x(c->g0) : 0;
+  d.fine_rag = fine_ragged_x(c->g0) > 0;
+  d.fine_bx = smooth_tile_x(c);
   d.tile_bx = fine_brick_x(c->g0);
   d.sweeps_fine = c->cfg.pre_sweeps;
   d.sweeps_coarse = c->cfg.coarse_sweeps > 0 ? c->cfg.coarse_sweeps : c->cfg.pre_sweeps;
@@ -661,6 +670,28 @@ long long residb(const Member& m) {
 }
 long long one(const Member&) { return 1; }
 
+// Fine brick smoothing, the cells by tile width and the ragged ones apart.
+void plan_fine_brick(otm_batch* b, const std::vector<Member*>& set, int post) {
+  CellDev* cells = b->dcells;
+  hipStream_t s = b->s;
+  for (int bx : {32, 16})
+    for (bool rag : {false, true}) {
+      std::vector<Member*> part;
+      for (Member* m : set)
+        if (smooth_tile_x(m->c) == bx && (fine_ragged_x(m->c->g0) > 0) == rag) part.push_back(m);
+      const auto k = bx == 32 ? (rag ? kb_fine_brick<32, true> : kb_fine_brick<32, false>)
+                              : (rag ? kb_fine_brick<16, true> : kb_fine_brick<16, false>);
+      add_launch(
+          b, part,
+          [bx, rag](const Member& m) {
+            return (long long)(rag ? fine_ragged_tiles(m.c->g0, bx) : fine_tiles(m.c->g0, bx));
+          },
+          0, [=](const Ent* e, int n, unsigned grid) {
+            hipLaunchKernelGGL(k, dim3(grid), dim3(bx * kFineTR), 0, s, e, n, cells, post);
+          });
+    }
+}
+
 // Brick smoothing of level l, the cells with FP32 and with FP16 stencils
 // apart (each form has its own registers), split by load case up to
 // kStOneMax bricks in the launch.
@@ -699,22 +730,10 @@ void plan_vcycle(otm_batch* b, std::vector<Member*>& V) {
     std::vector<Member*> S = at(l, false);
     if (S.empty()) continue;
     if (l == 0) {
-      std::vector<Member*> b32, b16, col;
-      for (Member* m : S) {
-        const int bx = m->c->lv[0].brick ? fine_brick_x(m->c->g0) : 0;
-        (bx == 32 ? b32 : bx == 16 ? b16 : col).push_back(m);
-      }
-      CellDev* cells = b->dcells;
-      hipStream_t s = b->s;
-      auto bricks = [](const Member& m) {
-        return (long long)(m.c->g0.nn / (fine_brick_x(m.c->g0) * kFineBY * kFineBZ));
-      };
-      add_launch(b, b32, bricks, 0, [cells, s](const Ent* e, int n, unsigned grid) {
-        hipLaunchKernelGGL(kb_fine_brick<32>, dim3(grid), dim3(32 * kFineTR), 0, s, e, n, cells, 0);
-      });
-      add_launch(b, b16, bricks, 0, [cells, s](const Ent* e, int n, unsigned grid) {
-        hipLaunchKernelGGL(kb_fine_brick<16>, dim3(grid), dim3(16 * kFineTR), 0, s, e, n, cells, 0);
-      });
+      std::vector<Member*> col;
+      for (Member* m : S)
+        if (!smooth_tile_x(m->c)) col.push_back(m);
+      plan_fine_brick(b, S, 0);
       if (!col.empty()) {
         add_op(b, col, OpFillU{0}, [](const Member& m) { return (long long)nblk(3 * m.c->g0.nn); });
         for (int sw = 0; sw < col.front()->c->cfg.pre_sweeps; sw++)
@@ -746,24 +765,12 @@ void plan_vcycle(otm_batch* b, std::vector<Member*>& V) {
     if (S.empty()) continue;
     add_op(b, S, OpProlong{l}, [l](const Member& m) { return (long long)nblk(m.c->lv[l + 1].g.nn); });
     if (l == 0) {
-      std::vector<Member*> b32, b16, col;
-      for (Member* m : S) {
-        const int bx = m->c->lv[0].brick ? fine_brick_x(m->c->g0) : 0;
-        (bx == 32 ? b32 : bx == 16 ? b16 : col).push_back(m);
-      }
-      CellDev* cells = b->dcells;
-      hipStream_t s = b->s;
-      auto bricks = [](const Member& m) {
-        return (long long)(m.c->g0.nn / (fine_brick_x(m.c->g0) * kFineBY * kFineBZ));
-      };
-      add_launch(b, b32, bricks, 0, [cells, s](const Ent* e, int n, unsigned grid) {
-        hipLaunchKernelGGL(kb_fine_brick<32>, dim3(grid), dim3(32 * kFineTR), 0, s, e, n, cells, 1);
-      });
-      add_launch(b, b16, bricks, 0, [cells, s](const Ent* e, int n, unsigned grid) {
-        hipLaunchKernelGGL(kb_fine_brick<16>, dim3(grid), dim3(16 * kFineTR), 0, s, e, n, cells, 1);
-      });
-      for (Member* m : b32) m->par ^= 1;
-      for (Member* m : b16) m->par ^= 1;
+      std::vector<Member*> col;
+      for (Member* m : S)
+        if (!smooth_tile_x(m->c)) col.push_back(m);
+      plan_fine_brick(b, S, 1);
+      for (Member* m : S)
+        if (smooth_tile_x(m->c)) m->par ^= 1;
       if (!col.empty())
         for (int sw = 0; sw < col.front()->c->cfg.post_sweeps; sw++)
           for (int cc = 3; cc >= 0; cc--)
@@ -885,7 +892,7 @@ void step(otm_batch* b) {
     // the tiled post-smoother has formed r.z; cells on exact sweeps form it here
     std::vector<Member*> untiled;
     for (Member* m : V)
-      if (!m->c->lv[0].brick || !fine_brick_x(m->c->g0)) untiled.push_back(m);
+      if (!smooth_tile_x(m->c)) untiled.push_back(m);
     add_op(b, untiled, OpDot3{}, redb);
     add_op(b, A2, OpFinal{FIN_RZ_FIRST, OTM_NRHS, -1.0, 2}, one);
     add_op(b, B2, OpFinal{FIN_RZ, OTM_NRHS, -1.0, 2}, one);

@@ -225,7 +225,7 @@ static void build_hierarchy(otm_ctx* c) {
       c->fine_tile = cfg.fine_tile < 0 ? fine_tile_default(L.g) : cfg.fine_tile;
       if (c->fine_tile >= 0 && !fine_tile_ok(L.g, c->fine_tile))
         fail(OTM_E_UNSUPPORTED, "the cell's edges are not multiples of the requested fine tile shape");
-      if (c->fine_tile >= 0 && cfg.pre_sweeps == cfg.post_sweeps) {
+      if (fine_brick_ok(L.g, c->fine_tile) && cfg.pre_sweeps == cfg.post_sweeps) {
         L.brick = true;
         c->z2 = dalloc<float>(3 * n);
         L.u2 = c->z2;
@@ -257,8 +257,10 @@ static void build_hierarchy(otm_ctx* c) {
   if (c->lv.size() > 2 && c->lv[c->lv.size() - 2].g.nn <= kTailStartNodes) c->tail--;
   c->cBinv = dalloc<double>(ncoarse * ncoarse);
   c->partials = dalloc<double>((size_t)kMaxReduceBlocks * kMaxReduce);
-  // one row per fine tile of the smallest shape (32 x 4 x 4 = 512 nodes)
-  c->tile_partials = dalloc<double>((size_t)std::min<long long>(kTileDotSlots, n0 / 512 + 1) * OTM_NRHS);
+  // one row per fine tile: of the smallest shape (32 x 4 x 4 = 512 nodes), or ragged
+  long long tiles = n0 / 512 + 1;
+  if (c->fine_tile < 0 && fine_brick_ok(c->g0, -1)) tiles = std::max(tiles, fine_brick_tiles(c->g0, -1));
+  c->tile_partials = dalloc<double>((size_t)std::min<long long>(kTileDotSlots, tiles) * OTM_NRHS);
   c->red_out = dalloc<double>(16);
   c->pcg = dalloc<PcgScalars>(1);
   hip_check(hipMemsetAsync(c->pcg, 0, sizeof(PcgScalars), c->s), "hipMemset pcg");
@@ -1323,7 +1325,8 @@ OTM_API int otm_smooth_level(otm_ctx* ctx, int level, const float* f, float* u, 
     const Level& L = ctx->lv[level];
     const long long n = L.g.nn;
     const bool brick = mode >= 2, forward = (mode & 1) == 0;
-    if (brick && !L.u2) fail(OTM_E_UNSUPPORTED, "this level has no brick smoother");
+    if (brick && (!L.u2 || (level == 0 && ctx->fine_tile < 0)))
+      fail(OTM_E_UNSUPPORTED, "this level has no brick smoother");
     Staged a, b, c2;
     const float* df = stage_in(ctx, a, f, 3 * n, where);
     float* du = stage_in(ctx, b, u, 3 * n, where);

@@ -756,13 +756,33 @@ __host__ __device__ inline unsigned fine_apply_tile_blocks(const Geom& g, int bx
   return (unsigned)(t > kTileRedBlocks ? kTileRedBlocks : t);
 }
 
+// Width of the ragged tiles that smooth a level whose edges are no multiples
+// of the default tile (0: none, and the level is swept by exact colours): the
+// width that leaves fewer idle lanes. A tile that overhangs the cell stages
+// its overhang through one periodic wrap, so an edge is at least half a
+// tile's reach; rows are coloured by parity, so y and z edges are even.
+__host__ __device__ inline int fine_ragged_x(const Geom& g) {
+  if (fine_tile_x(g) || g.nx < 10 || g.ny < 4 || g.nz < 6 || (g.ny & 1) || (g.nz & 1)) return 0;
+  if (g.nx <= 16) return 16;
+  return (g.nx + 31) / 32 * 2 <= (g.nx + 15) / 16 ? 32 : 16;
+}
+__host__ __device__ inline int fine_ragged_tiles(const Geom& g, int bx) {
+  return ((g.nx + bx - 1) / bx) * ((g.ny + kFineBY - 1) / kFineBY) * ((g.nz + kFineBZ - 1) / kFineBZ);
+}
+
 struct TileOrigin {
   int ox, oy, oz;
 };
-template <int BX, int BY, int BZ>
+// RAG: the last tile of an axis may overhang the cell
+template <int BX, int BY, int BZ, bool RAG = false>
 __device__ inline TileOrigin tile_origin(const Geom& g, int b) {
-  const int bx = g.nx / BX, by = g.ny / BY;
+  const int bx = RAG ? (g.nx + BX - 1) / BX : g.nx / BX, by = RAG ? (g.ny + BY - 1) / BY : g.ny / BY;
   return {(b % bx) * BX, ((b / bx) % by) * BY, (b / (bx * by)) * BZ};
+}
+// x of tile column tx, wrapped where the tile overhangs
+template <bool RAG>
+__device__ inline unsigned tile_x(const Geom& g, const TileOrigin& o, int tx) {
+  return (unsigned)(RAG ? wrapm(o.ox + tx, g.nx) : o.ox + tx);
 }
 
 // Staging runs in two phases: every global load of a tile goes into
@@ -822,7 +842,7 @@ __device__ inline unsigned lane_run_offset(const Geom& g, int rb, int rows, int 
 }
 
 // kappa of element (ox-1+kx, oy-1+ky, oz-1+kz), for sk[kx + KX*(ky + KY*kz)]
-template <int BX, int BY, int BZ, int TR, int NR = OTM_NRHS>
+template <int BX, int BY, int BZ, int TR, int NR = OTM_NRHS, bool RAG = false>
 __device__ inline void load_tile_kappa(const Geom& g, const float* __restrict__ kappa, const TileOrigin& o,
                                        TileStage<BX, BY, BZ, TR, NR>& st) {
   using S = TileStage<BX, BY, BZ, TR, NR>;
@@ -834,7 +854,7 @@ __device__ inline void load_tile_kappa(const Geom& g, const float* __restrict__ 
   for (int j = 0; j < S::KJ; j++) {
     const int rb = wr0 + TR * j;  // wave-uniform
     const unsigned off = lane_run_offset<BX, T::KY>(g, rb, S::KR, o.oy - 1, o.oz - 1);
-    if (ty + TR * j < S::KR) st.k[j] = ld_off(kappa, off + 4u * (unsigned)(o.ox + tx));
+    if (ty + TR * j < S::KR) st.k[j] = ld_off(kappa, off + 4u * tile_x<RAG>(g, o, tx));
   }
   const int xm = wrapm(o.ox - 1, g.nx);
 #pragma unroll
@@ -865,7 +885,7 @@ __device__ inline void store_tile_kappa(float* sk, const TileStage<BX, BY, BZ, T
 
 // field k (k < NR) of node (ox-1+hx, oy-1+hy, oz-1+hz), for
 // su[k*kU + hx + HX*(hy + HY*hz)]
-template <int BX, int BY, int BZ, int TR, int NR = OTM_NRHS>
+template <int BX, int BY, int BZ, int TR, int NR = OTM_NRHS, bool RAG = false>
 __device__ inline void load_tile_fields(const Geom& g, const float* __restrict__ src, const TileOrigin& o,
                                         TileStage<BX, BY, BZ, TR, NR>& st) {
   using S = TileStage<BX, BY, BZ, TR, NR>;
@@ -879,7 +899,7 @@ __device__ inline void load_tile_fields(const Geom& g, const float* __restrict__
 #pragma unroll
   for (int j = 0; j < S::UJ; j++) {
     const int rb = wr0 + TR * j;
-    const unsigned off = lane_run_offset<BX, T::HY>(g, rb, S::UR, o.oy - 1, o.oz - 1) + 4u * (unsigned)(o.ox + tx);
+    const unsigned off = lane_run_offset<BX, T::HY>(g, rb, S::UR, o.oy - 1, o.oz - 1) + 4u * tile_x<RAG>(g, o, tx);
     if (ty + TR * j < S::UR) {
 #pragma unroll
       for (int k = 0; k < NR; k++) st.u[k][j] = ld_off(srck[k], off);
@@ -1019,7 +1039,16 @@ __device__ inline void fine_residual_tile_body(const Geom& g, const FineConsts& 
 // one load case, with every node's weights in registers from the start
 // (with all three they cost a wave per SIMD, see below), and a step waits
 // for a third of the LDS reads. The results have the same bits either way.
-template <int BX, int BY = kFineBY, int BZ = kFineBZ, int TR = kFineTR, int NR = OTM_NRHS>
+//
+// RAG smooths a cell whose edges are no multiples of the tile: nodes of a
+// tile beyond the cell hold the periodic images' entry values and are
+// neither updated nor written, so they are the tile's frozen halo on that
+// side (lane and row of a halo node feed their neighbours as any other).
+// Such cells took four launches of one colour each per sweep before; a
+// solve went from 1865 to 1241 us at 20 x 24 x 28 (one more iteration: the
+// halos are frozen now), 3122 to 2455 at 72 x 88 x 56, 3069 to 2508 at
+// 88 x 72 x 104.
+template <int BX, int BY = kFineBY, int BZ = kFineBZ, int TR = kFineTR, int NR = OTM_NRHS, bool RAG = false>
 __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, const float* __restrict__ kappa,
                                        const float* __restrict__ f, const float* __restrict__ uin,
                                        float* __restrict__ uout, int sweeps, int forward, int zero_in, int b,
@@ -1031,7 +1060,7 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
   static_assert(R % TR == 0, "thread rows must divide the rows of a colour");
   __shared__ float su[NR][T::kU];
   __shared__ float sk[T::kK];
-  const TileOrigin o = tile_origin<BX, BY, BZ>(g, b);
+  const TileOrigin o = tile_origin<BX, BY, BZ, RAG>(g, b);
   const int ox = o.ox, oy = o.oy, oz = o.oz;
   const int t = threadIdx.x;
   const int tx = t % BX, ty = t / BX;  // ty in [0, TR)
@@ -1041,8 +1070,8 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
   // stores and the barrier
   {
     TileStage<BX, BY, BZ, TR, NR> st;
-    load_tile_kappa<BX, BY, BZ, TR, NR>(g, kappa, o, st);
-    if (!zero_in) load_tile_fields<BX, BY, BZ, TR, NR>(g, uin, o, st);
+    load_tile_kappa<BX, BY, BZ, TR, NR, RAG>(g, kappa, o, st);
+    if (!zero_in) load_tile_fields<BX, BY, BZ, TR, NR, RAG>(g, uin, o, st);
     store_tile_kappa<BX, BY, BZ, TR, NR>(sk, st);
     if (zero_in) {
       for (int i = t; i < T::kU; i += T::NT) {
@@ -1059,6 +1088,7 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
   const int lx = tx;
   const int wr0 = wave_first_row<BX>(), sub = lane_row<BX>();
   const unsigned nxu = (unsigned)g.nx, nxyu = (unsigned)g.nx * (unsigned)g.ny;
+  auto inside = [&](int ly, int lz) { return !RAG || (ox + lx < g.nx && oy + ly < g.ny && oz + lz < g.nz); };
   float fv[4][H][NR];
 #pragma unroll
   for (int col = 0; col < 4; col++)
@@ -1069,10 +1099,11 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
       for (int q = 0; q < 64 / BX; q++) {
         const int rr = wr0 + q + TR * h;
         const int ly = (col & 1) + 2 * (rr % (BY / 2)), lz = (col >> 1) + 2 * (rr / (BY / 2));
-        const unsigned oq = nxu * (unsigned)(oy + ly) + nxyu * (unsigned)(oz + lz);
+        const unsigned oq =
+            RAG ? wrapped_row(g, oy + ly, oz + lz) : nxu * (unsigned)(oy + ly) + nxyu * (unsigned)(oz + lz);
         off = sub == q ? oq : off;
       }
-      off = 4u * (off + (unsigned)(ox + lx));
+      off = 4u * (off + tile_x<RAG>(g, o, lx));
 #pragma unroll
       for (int k = 0; k < NR; k++) fv[col][h][k] = ld_off(f + (size_t)k * (size_t)g.nn, off);
     }
@@ -1188,6 +1219,7 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
             w = held[col][h];
           else
             w = weights(ly, lz);
+          const bool in = inside(ly, lz);
           // rows of the node's own column, addressed from the lowest one so
           // that every offset (load cases included) is an LDS immediate
           int cb = (lx + 1) + DY * (ly + 1) + DZ * (lz + 1) - LO;
@@ -1207,7 +1239,7 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
             }
             acc += from_left(T1);
             acc += from_right(T0);
-            (&su[k][0] + cb)[LO] = (fe[col][h][k] + c * acc) * w.inv;
+            if (in) (&su[k][0] + cb)[LO] = (fe[col][h][k] + c * acc) * w.inv;
           }
         }
       };
@@ -1233,7 +1265,8 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
         const int ly = (col & 1) + 2 * (rr % (BY / 2)), lz = (col >> 1) + 2 * (rr / (BY / 2));
         const int c0 = (lx + 1) + DY * (ly + 1) + DZ * (lz + 1);
 #pragma unroll
-        for (int k = 0; k < NR; k++) acc[k] += (double)fv[col][h][k] * (double)su[k][c0];
+        for (int k = 0; k < NR; k++)
+          if (inside(ly, lz)) acc[k] += (double)fv[col][h][k] * (double)su[k][c0];
       }
     constexpr int kW = T::NT / 64;
     __shared__ double sh[NR * kW];
@@ -1263,6 +1296,7 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
     off = 4u * (off + (unsigned)(ox + tx));
     const int r = ty + TR * j;
     const int ly = r % BY, lz = r / BY;
+    if (!inside(ly, lz)) continue;
     const int c0 = (tx + 1) + DY * (ly + 1) + DZ * (lz + 1);
 #pragma unroll
     for (int k = 0; k < NR; k++) *(float*)((char*)(uout + (size_t)k * (size_t)g.nn) + off) = su[k][c0];

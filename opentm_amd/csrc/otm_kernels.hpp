@@ -49,6 +49,9 @@ int fine_tile_default(const Geom& g);  // -1: the cell does not tile
 // f.uout for that reducer (the PCG's r.z after a preconditioner
 // application); launch_fine_brick_dot_final then finishes the reduction.
 int fine_brick_x(const Geom& g);
+// variant -1: the ragged tiles of a cell that takes no other shape
+bool fine_brick_ok(const Geom& g, int variant);
+long long fine_brick_tiles(const Geom& g, int variant);
 bool fine_brick_dot_ok(const Geom& g, int variant);
 void launch_fine_smooth_brick(hipStream_t s, const Geom& g, const FineConsts& fc, const float* kappa, const float* f,
                               const float* uin, float* uout, int sweeps, bool forward, bool zero_in, int variant,
