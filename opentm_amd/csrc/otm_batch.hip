@@ -251,14 +251,14 @@ struct OpInitResid {
     if constexpr (sizeof(XT) == 8) x = C.x64;
     else x = C.x;
     const float* xlo = sizeof(XT) == 4 ? C.xlo : nullptr;
-    // the single-cell launch's form for this row length, one load case after
-    // another: the same r and partial sums
-    if (!fine_rows_ok(C.g[0].nx)) {
-      fine_init_residual_body<XT>(C.g[0], C.fc, C.kappa, x, xlo, C.r, R, lb, nb);
-      return;
-    }
-    for (int k = 0; k < OTM_NRHS; k++)
+    // the single-cell launch's form and split: the same r and partial sums
+    const int k = lb % OTM_NRHS;
+    lb /= OTM_NRHS;
+    nb /= OTM_NRHS;
+    if (fine_rows_ok(C.g[0].nx))
       fine_init_residual_rows_body<XT>(C.g[0], C.fc, C.kappa, x, xlo, C.r, R, lb, nb, k);
+    else
+      fine_init_residual_case_body<XT>(C.g[0], C.fc, C.kappa, x, xlo, C.r, R, lb, nb, k);
   }
 };
 
@@ -827,8 +827,9 @@ void step(otm_batch* b) {
   add_op(b, Aadd, OpRefineAdd{}, [](const Member& m) { return (long long)std::min<long long>(8192, nblk(3 * m.c->g0.nn)); });
   add_op(b, Afill, OpFillVec{1}, [](const Member& m) { return (long long)std::min<long long>(8192, nblk(3 * m.c->g0.nn)); });
   for (Member* m : Aadd) m->pending = false;
-  add_op(b, A32, OpInitResid<float>{-1.0}, redb);
-  add_op(b, A64, OpInitResid<double>{-1.0}, redb);
+  const auto cases = [](const Member& m) { return OTM_NRHS * redb(m); };
+  add_op(b, A32, OpInitResid<float>{-1.0}, cases);
+  add_op(b, A64, OpInitResid<double>{-1.0}, cases);
   add_op(b, A, OpFinal{FIN_BB_RR, 3 * OTM_NRHS, -1.0}, one);
   add_op(b, B, OpApplyDot{}, applyb);
   add_op(b, B, OpFinal{FIN_PQ, OTM_NRHS, -1.0, 1}, one);

@@ -284,58 +284,10 @@ __device__ inline void fine_apply_dot_body(const Geom& g, const FineConsts& fc, 
 // does not vary along the load direction); stored rounded to FP32. Partial
 // sums of b.b, r.r and sum(r) (PCG start and restarts). XT is the iterate's
 // type: FP32 (with xlo: an FP32 pair), or FP64 for the iterative refinement.
-template <typename XT>
-__device__ inline void fine_init_residual_body(const Geom& g, const FineConsts& fc, const float* __restrict__ kappa,
-                                               const XT* __restrict__ x_, const float* __restrict__ xlo,
-                                               float* __restrict__ rvec, const Reduce& R, int lb, int nb) {
-  double acc[3 * OTM_NRHS] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  const double c = (double)fc.c;
-  const BlockRange br = block_range_v(g.nn, lb, nb);
-  for (long long t = br.b + threadIdx.x; t < br.e; t += blockDim.x) {
-    // 64-bit decode on purpose: this FP64-heavy loop measured twice as fast
-    // with it on gfx950 as with split_node (47 against 95 us per launch at
-    // 128^3), although the 32-bit decode is shorter code
-    const int x = (int)(t % g.nx);
-    const long long r = t / g.nx;
-    const int y = (int)(r % g.ny), z = (int)(r / g.ny);
-    const NodeIdx n = node_idx(g, x, y, z);
-    const NodeElems E = load_elems(g, n, kappa);
-    double ksum = 0.0;
-#pragma unroll
-    for (int e = 0; e < 8; e++) ksum += (double)E.k[e];
-#pragma unroll
-    for (int k = 0; k < OTM_NRHS; k++) {
-      const XT* xk = x_ + k * g.nn;
-      double b = 0.0;
-#pragma unroll
-      for (int e = 0; e < 8; e++) b += (double)E.k[e] * (double)fc.femu[7 - e][k];
-      double kx;
-      if constexpr (sizeof(XT) == 4) {
-        if (xlo) {
-          const float* xl = xlo + k * g.nn;
-          kx = c * (4.0 * ksum * ((double)xk[n.v] + (double)xl[n.v]) - far_sum_pair(g, n, E, xk, xl));
-        } else {
-          kx = c * (4.0 * ksum * (double)xk[n.v] - far_sum_d(g, n, E, xk));
-        }
-      } else {
-        kx = c * (4.0 * ksum * (double)xk[n.v] - far_sum_d(g, n, E, xk));
-      }
-      const double rv = b - kx;
-      rvec[k * g.nn + n.v] = (float)rv;
-      acc[k] += b * b;
-      acc[OTM_NRHS + k] += rv * rv;
-      acc[2 * OTM_NRHS + k] += rv;
-    }
-  }
-  reduce_block_at<3 * OTM_NRHS>(acc, R, lb);
-}
-
-// fine_init_residual_body for load case k alone (a grid of nb x 3 blocks):
-// block (lb, k) covers the nodes of block lb of the one-dimensional form
-// in the same order, so r and the partial sums carry the same bits; it
-// writes values k, 3 + k and 6 + k of partial slot lb. With one load case
-// per thread, the gathered neighbours of three cases are not live together
-// (222 registers and two waves per SIMD for the three-case form).
+// A block takes load case k (nb x 3 blocks) and writes values k, 3 + k and
+// 6 + k of partial slot lb: with one load case per thread, the gathered
+// neighbours of three cases are not live together (222 registers and two
+// waves per SIMD for the three-case form).
 template <typename XT>
 __device__ inline void fine_init_residual_case_body(const Geom& g, const FineConsts& fc,
                                                     const float* __restrict__ kappa, const XT* __restrict__ x_,
@@ -350,7 +302,9 @@ __device__ inline void fine_init_residual_case_body(const Geom& g, const FineCon
   const float* xl = xlo ? xlo + (size_t)k * (size_t)g.nn : nullptr;
   const BlockRange br = block_range_v(g.nn, lb, nb);
   for (long long t = br.b + threadIdx.x; t < br.e; t += blockDim.x) {
-    // 64-bit decode as in fine_init_residual_body
+    // 64-bit decode on purpose: this FP64-heavy loop measured twice as fast
+    // with it on gfx950 as with split_node (47 against 95 us per launch at
+    // 128^3), although the 32-bit decode is shorter code
     const int x = (int)(t % g.nx);
     const long long r = t / g.nx;
     const int y = (int)(r % g.ny), z = (int)(r / g.ny);
@@ -402,6 +356,10 @@ __device__ inline void fine_init_residual_case_body(const Geom& g, const FineCon
 // the step before. The window is a ring of three rows (the loop is unrolled
 // by three so no values move) and LDS is double-buffered: one barrier per
 // step. Writes values k, 3 + k and 6 + k of partial slot lb.
+// An FP32 pair's parts are loaded in two runs: with a choice per value (low
+// part or none) each load waited for the one before, and a launch took 732
+// us at 256^3 (now 300; 290 with an FP64 iterate), 77 at 128^3 (36), 18 at
+// 48^3 (10). What is left is the step's wait for the entering row.
 __host__ __device__ inline bool fine_rows_ok(int nx) { return nx <= kBlock; }
 
 template <typename XT>
@@ -409,16 +367,10 @@ struct RowsWindow {
   double V[3][3];       // V[slot][bz]: iterate at row slot, plane z - 1 + bz
   double KM[3][2], KP[3][2];  // element row slot: conductivity at x - 1 / x, plane z - 1 + az
   double SQ[3][2], H[3];      // KM + KP, and its sum over az
-  double pu[3];         // the entering row's values
-  float pk[4];
+  XT pu[3];             // the entering row's values
+  float pl[3], pk[4];   // (pl: the low parts of an FP32 pair)
   unsigned y, z, pz[3];  // current row, node index of (0, 0, z - 1 + bz)
 };
-
-template <typename XT>
-__device__ inline double rows_val(const XT* __restrict__ xk, const float* __restrict__ xl, unsigned v) {
-  if constexpr (sizeof(XT) == 4) return xl ? (double)xk[v] + (double)xl[v] : (double)xk[v];
-  else return xk[v];
-}
 
 template <typename XT>
 __device__ inline void rows_elem_slot(RowsWindow<XT>& W, int e, float m0, float p0, float m1, float p1) {
@@ -454,7 +406,13 @@ __device__ inline void rows_step(RowsWindow<XT>& W, bool& have, unsigned row, bo
 #pragma unroll
     for (int a = 0; a < 3; a++)
 #pragma unroll
-      for (int bz = 0; bz < 3; bz++) W.V[sl[a]][bz] = rows_val(xk, xl, W.pz[bz] + yo[a] + (unsigned)x);
+      for (int bz = 0; bz < 3; bz++) W.V[sl[a]][bz] = (double)xk[W.pz[bz] + yo[a] + (unsigned)x];
+    if (sizeof(XT) == 4 && xl) {
+#pragma unroll
+      for (int a = 0; a < 3; a++)
+#pragma unroll
+        for (int bz = 0; bz < 3; bz++) W.V[sl[a]][bz] += (double)xl[W.pz[bz] + yo[a] + (unsigned)x];
+    }
 #pragma unroll
     for (int ay = 0; ay < 2; ay++) {
       const unsigned r0 = W.pz[0] + yo[ay], r1 = W.pz[1] + yo[ay];
@@ -493,7 +451,11 @@ __device__ inline void rows_step(RowsWindow<XT>& W, bool& have, unsigned row, bo
   if (slide) {
     const unsigned y1 = (W.y + 1) * (unsigned)nx, y2 = W.y + 2 == ny ? 0u : y1 + (unsigned)nx;
 #pragma unroll
-    for (int bz = 0; bz < 3; bz++) W.pu[bz] = rows_val(xk, xl, W.pz[bz] + y2 + (unsigned)x);
+    for (int bz = 0; bz < 3; bz++) W.pu[bz] = xk[W.pz[bz] + y2 + (unsigned)x];
+    if (sizeof(XT) == 4 && xl) {
+#pragma unroll
+      for (int bz = 0; bz < 3; bz++) W.pl[bz] = xl[W.pz[bz] + y2 + (unsigned)x];
+    }
     const unsigned r0 = W.pz[0] + y1, r1 = W.pz[1] + y1;
     W.pk[0] = kappa[r0 + xm];
     W.pk[1] = kappa[r0 + x];
@@ -513,7 +475,10 @@ __device__ inline void rows_step(RowsWindow<XT>& W, bool& have, unsigned row, bo
   if (slide) {
     // row y-1 leaves slot s0 for row y+2; element row y+1 takes slot s2
 #pragma unroll
-    for (int bz = 0; bz < 3; bz++) W.V[s0][bz] = W.pu[bz];
+    for (int bz = 0; bz < 3; bz++) {
+      W.V[s0][bz] = (double)W.pu[bz];
+      if (sizeof(XT) == 4 && xl) W.V[s0][bz] += (double)W.pl[bz];
+    }
     rows_elem_slot(W, s2, W.pk[0], W.pk[1], W.pk[2], W.pk[3]);
     W.y += 1;
   }
