@@ -165,16 +165,6 @@ __device__ inline void restrict8_body(const Geom& fg, const Geom& cg, const floa
   if (j < OTM_NRHS) fc[(size_t)j * (size_t)cg.nn + node] = j == 0 ? a[0] : (j == 1 ? a[1] : a[2]);
 }
 
-// u_f(i) += sum_I P(i, I) u_c(I), trilinear (prolongate_correction_kernel_H,
-// grid.cu:881-940).
-__device__ inline void prolong_node(const Geom& fg, const Geom& cg, const float* uc, float* uf, long long t) {
-  int x, y, z;
-  split_node(fg.nx, fg.ny, t, x, y, z);
-  const ProlongW P = prolong_weights(cg, x, y, z);
-#pragma unroll
-  for (int k = 0; k < OTM_NRHS; k++) uf[k * fg.nn + t] += prolong_sum(cg, uc + k * cg.nn, P);
-}
-
 // ---- per-level bodies ----
 // GS update of one of 8 colours (parity of x, y, z), colour = cx + 2cy + 4cz.
 template <bool HALF>
@@ -291,13 +281,13 @@ __device__ inline void restrict_body(const Geom& fg, const Geom& cg, const float
   restrict_node(fg, cg, res, fc, t);
 }
 
-// Prolongation by coarse cell: thread t owns coarse node (X, Y, Z) and the
-// eight fine nodes (2X+dx, 2Y+dy, 2Z+dz). It loads the eight coarse values
-// around the cell once per right-hand side and adds to every fine node the
-// terms of prolong_sum in its order (zero weights skipped), so the result
-// is prolong_node's bit for bit with an eighth of the coarse loads and
-// paired, coalesced fine accesses. The fine level is twice the coarse one
-// along every axis.
+// u_f(i) += sum_I P(i, I) u_c(I), trilinear (prolongate_correction_kernel_H,
+// grid.cu:881-940), by coarse cell: thread t owns coarse node (X, Y, Z) and
+// the eight fine nodes (2X+dx, 2Y+dy, 2Z+dz). It loads the eight coarse
+// values around the cell once per right-hand side and adds to every fine
+// node its terms (zero weights skipped): an eighth of the coarse loads of a
+// thread per fine node, and paired, coalesced fine accesses. The fine level
+// is twice the coarse one along every axis.
 __device__ inline void prolong_body(const Geom& fg, const Geom& cg, const float* __restrict__ uc,
                                     float* __restrict__ uf, long long t) {
   if (t >= cg.nn) return;

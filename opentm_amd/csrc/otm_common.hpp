@@ -63,21 +63,6 @@ __device__ inline ProlongW prolong_weights(const Geom& cg, int x, int y, int z) 
   P.wz[1] = (z & 1) ? 0.5f : 0.f;
   return P;
 }
-// sum_I P(i, I) u_c(I) for one right-hand side ck of the coarse grid.
-__device__ inline float prolong_sum(const Geom& cg, const float* __restrict__ ck, const ProlongW& P) {
-  float s = 0.f;
-#pragma unroll
-  for (int c = 0; c < 2; c++)
-#pragma unroll
-    for (int b = 0; b < 2; b++)
-#pragma unroll
-      for (int a = 0; a < 2; a++) {
-        const float w = P.wx[a] * P.wy[b] * P.wz[c];
-        if (w != 0.f)
-          s += w * ld_off(ck, 4u * ((unsigned)P.X[a] + (unsigned)cg.nx * ((unsigned)P.Y[b] + (unsigned)cg.ny * (unsigned)P.Z[c])));
-      }
-  return s;
-}
 
 // Element constants of the fine level (closed forms of the reference's
 // quadrature, templateMatrix.cpp:21-87): Ke = c * P with P = 4 on the

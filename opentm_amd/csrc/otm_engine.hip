@@ -13,7 +13,6 @@
 
 #include <algorithm>
 #include <chrono>
-#include <mutex>
 #include <random>
 #include <stdexcept>
 #include <string>
