@@ -49,6 +49,7 @@ struct CellDev {
   int tail;  // first level of the one-workgroup tail V-cycle
   int fine_bx;  // 32 or 16: fine brick width; 0: exact colour sweeps
   int fine_rag;  // the bricks are ragged tiles
+  int post_dot;  // the fine post-smoother forms r.z (post_dot_ok)
   int tile_bx;  // 32 or 16: LDS tile width of the fine residual and apply; 0: pointwise kernels
   int sweeps_fine, sweeps_coarse;
   FineConsts fc;
@@ -143,7 +144,7 @@ kb_fine_brick(const Ent* __restrict__ ents, int nents, const CellDev* __restrict
   R.partials = C.tile_partials;
   fine_brick_body<BX, kFineBY, kFineBZ, kFineTR, OTM_NRHS, RAG>(
       C.g[0], C.fc, C.kappa, C.f[0], post ? ucur(C, e.par, 0) : nullptr, post ? uoth(C, e.par, 0) : ucur(C, e.par, 0),
-      sw, post ? 0 : 1, post ? 0 : 1, b - e.block0, post, R);
+      sw, post ? 0 : 1, post ? 0 : 1, b - e.block0, post && C.post_dot, R);
 }
 
 // ---- operations (one functor per batched launch) ---------------------------
@@ -272,7 +273,7 @@ struct OpFinal {  // one block per cell
     if (rtol2 >= 0.0) R.rtol2 = rtol2;
     unsigned nb = red_blocks_for(C.g[0].nn);
     if (tiled == 1 && C.tile_bx) nb = fine_apply_tile_blocks(C.g[0], C.tile_bx);
-    if (tiled == 2 && C.fine_bx) {
+    if (tiled == 2 && C.post_dot) {
       R.partials = C.tile_partials;
       nb = (unsigned)(C.fine_rag ? fine_ragged_tiles(C.g[0], C.fine_bx) : fine_tiles(C.g[0], C.fine_bx));
       if (nb > (unsigned)kMaxReduceBlocks) {  // as launch_reduce_final
@@ -523,6 +524,15 @@ int smooth_tile_x(const otm_ctx* c) {
   return bx ? bx : fine_ragged_x(c->g0);
 }
 
+// tiles of a launch of that smoother
+long long smooth_tiles(const otm_ctx* c) {
+  const int bx = smooth_tile_x(c);
+  return fine_ragged_x(c->g0) > 0 ? fine_ragged_tiles(c->g0, bx) : fine_tiles(c->g0, bx);
+}
+// Whether a cell's fine post-smoother forms r.z, as its own solve decides: its
+// tiles have a row each in the context's tile partials.
+bool post_dot_ok(const otm_ctx* c) { return c->lv[0].brick && fine_brick_dot_ok(c->g0, c->fine_tile); }
+
 void ensure_cells(otm_batch* b, int n) {
   if (n <= b->dcap) return;
   if (b->s) hip_check(hipStreamSynchronize(b->s), "hipStreamSynchronize");  // no launch still reads them
@@ -575,6 +585,9 @@ CellDev describe(const Member& m) {
     fail(OTM_E_UNSUPPORTED, "the batched form runs the default fine tile shape (otm_config.fine_tile = -1)");
   d.fine_rag = fine_ragged_x(c->g0) > 0;
   d.fine_bx = smooth_tile_x(c);
+  d.post_dot = post_dot_ok(c);
+  if (d.post_dot && smooth_tiles(c) > fine_dot_rows(c->g0))
+    fail(OTM_E_STATE, "more fine tiles than rows of tile partials");
   d.tile_bx = fine_brick_x(c->g0);
   d.sweeps_fine = c->cfg.pre_sweeps;
   d.sweeps_coarse = c->cfg.coarse_sweeps > 0 ? c->cfg.coarse_sweeps : c->cfg.pre_sweeps;
@@ -682,11 +695,7 @@ void plan_fine_brick(otm_batch* b, const std::vector<Member*>& set, int post) {
       const auto k = bx == 32 ? (rag ? kb_fine_brick<32, true> : kb_fine_brick<32, false>)
                               : (rag ? kb_fine_brick<16, true> : kb_fine_brick<16, false>);
       add_launch(
-          b, part,
-          [bx, rag](const Member& m) {
-            return (long long)(rag ? fine_ragged_tiles(m.c->g0, bx) : fine_tiles(m.c->g0, bx));
-          },
-          0, [=](const Ent* e, int n, unsigned grid) {
+          b, part, [](const Member& m) { return smooth_tiles(m.c); }, 0, [=](const Ent* e, int n, unsigned grid) {
             hipLaunchKernelGGL(k, dim3(grid), dim3(bx * kFineTR), 0, s, e, n, cells, post);
           });
     }
@@ -890,11 +899,11 @@ void step(otm_batch* b) {
   if (!V.empty()) {
     add_op(b, A2, OpSubMeanR{0}, [](const Member& m) { return (long long)std::min<long long>(8192, nblk(m.c->g0.nn)); });
     plan_vcycle(b, V);
-    // the tiled post-smoother has formed r.z; cells on exact sweeps form it here
-    std::vector<Member*> untiled;
+    // r.z of the cells whose post-smoother has not formed it
+    std::vector<Member*> apart;
     for (Member* m : V)
-      if (!smooth_tile_x(m->c)) untiled.push_back(m);
-    add_op(b, untiled, OpDot3{}, redb);
+      if (!post_dot_ok(m->c)) apart.push_back(m);
+    add_op(b, apart, OpDot3{}, redb);
     add_op(b, A2, OpFinal{FIN_RZ_FIRST, OTM_NRHS, -1.0, 2}, one);
     add_op(b, B2, OpFinal{FIN_RZ, OTM_NRHS, -1.0, 2}, one);
     add_op(b, A2, OpFillVec{0}, [](const Member& m) { return (long long)std::min<long long>(8192, nblk(3 * m.c->g0.nn)); });

@@ -256,10 +256,7 @@ static void build_hierarchy(otm_ctx* c) {
   if (c->lv.size() > 2 && c->lv[c->lv.size() - 2].g.nn <= kTailStartNodes) c->tail--;
   c->cBinv = dalloc<double>(ncoarse * ncoarse);
   c->partials = dalloc<double>((size_t)kMaxReduceBlocks * kMaxReduce);
-  // one row per fine tile: of the smallest shape (32 x 4 x 4 = 512 nodes), or ragged
-  long long tiles = n0 / 512 + 1;
-  if (c->fine_tile < 0 && fine_brick_ok(c->g0, -1)) tiles = std::max(tiles, fine_brick_tiles(c->g0, -1));
-  c->tile_partials = dalloc<double>((size_t)std::min<long long>(kTileDotSlots, tiles) * OTM_NRHS);
+  c->tile_partials = dalloc<double>((size_t)fine_dot_rows(c->g0) * OTM_NRHS);
   c->red_out = dalloc<double>(16);
   c->pcg = dalloc<PcgScalars>(1);
   hip_check(hipMemsetAsync(c->pcg, 0, sizeof(PcgScalars), c->s), "hipMemset pcg");

@@ -100,30 +100,6 @@ k_fine_smooth_brick(Geom g, FineConsts fc, const float* __restrict__ kappa, cons
                                            dot, RD, k0);
 }
 
-bool fine_tile_ok(const Geom& g, int v) {
-  if (v < 0 || v >= kFineTileVariants) return false;
-  const FineTileShape& t = kFineTileShapes[v];
-  return g.nx % t.bx == 0 && g.ny % t.by == 0 && g.nz % t.bz == 0;
-}
-int fine_tile_default(const Geom& g) { return fine_tile_ok(g, 0) ? 0 : (fine_tile_ok(g, 1) ? 1 : -1); }
-int fine_brick_x(const Geom& g) {
-  const int v = fine_tile_default(g);
-  return v < 0 ? 0 : kFineTileShapes[v].bx;
-}
-// Whether variant v smooths the level, and its tiles; v < 0: the ragged tiles.
-bool fine_brick_ok(const Geom& g, int v) { return v < 0 ? fine_ragged_x(g) > 0 : fine_tile_ok(g, v); }
-long long fine_brick_tiles(const Geom& g, int v) {
-  if (v < 0) return fine_ragged_tiles(g, fine_ragged_x(g));
-  const FineTileShape& t = kFineTileShapes[v];
-  return (long long)(g.nx / t.bx) * (g.ny / t.by) * (g.nz / t.bz);
-}
-
-// r.z in the smoother: one partial-sum row per tile in the context's tile
-// partials (one row per 512 nodes, at most kTileDotSlots)
-bool fine_brick_dot_ok(const Geom& g, int v) {
-  return fine_brick_ok(g, v) && fine_brick_tiles(g, v) <= kTileDotSlots;
-}
-
 // A level whose edges are no multiples of a tile takes ragged tiles wherever
 // their overhang wraps once (fine_ragged_x): faster at every size measured,
 // from a solve of 12^3 (1192 -> 853 us) to 88 x 72 x 104 (3069 -> 2508).

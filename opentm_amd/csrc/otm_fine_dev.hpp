@@ -712,10 +712,6 @@ __host__ __device__ inline int fine_tiles(const Geom& g, int bx) {
 // Workgroups of the tiled operator apply: one tile each up to the partial-sum
 // capacity of a reduction, several tiles each beyond.
 constexpr int kTileRedBlocks = kMaxReduceBlocks;
-// Rows of the fine smoother's per-tile r.z partials (a context's tile
-// partials hold kTileDotSlots x 3 doubles): 65536 tiles of 512 nodes and
-// more cover a 1024^3 cell.
-constexpr int kTileDotSlots = 65536;
 __host__ __device__ inline unsigned fine_apply_tile_blocks(const Geom& g, int bx) {
   const int t = fine_tiles(g, bx);
   return (unsigned)(t > kTileRedBlocks ? kTileRedBlocks : t);
@@ -733,6 +729,44 @@ __host__ __device__ inline int fine_ragged_x(const Geom& g) {
 }
 __host__ __device__ inline int fine_ragged_tiles(const Geom& g, int bx) {
   return ((g.nx + bx - 1) / bx) * ((g.ny + kFineBY - 1) / kFineBY) * ((g.nz + kFineBZ - 1) / kFineBZ);
+}
+
+// Whether variant v of kFineTileShapes covers the level in whole tiles.
+inline bool fine_tile_ok(const Geom& g, int v) {
+  if (v < 0 || v >= kFineTileVariants) return false;
+  const FineTileShape& t = kFineTileShapes[v];
+  return g.nx % t.bx == 0 && g.ny % t.by == 0 && g.nz % t.bz == 0;
+}
+inline int fine_tile_default(const Geom& g) {  // -1: the cell does not tile
+  return fine_tile_ok(g, 0) ? 0 : (fine_tile_ok(g, 1) ? 1 : -1);
+}
+inline int fine_brick_x(const Geom& g) {  // bx of the default variant, or 0
+  const int v = fine_tile_default(g);
+  return v < 0 ? 0 : kFineTileShapes[v].bx;
+}
+// Whether variant v smooths the level, and its tiles; v < 0: the ragged tiles.
+inline bool fine_brick_ok(const Geom& g, int v) { return v < 0 ? fine_ragged_x(g) > 0 : fine_tile_ok(g, v); }
+inline long long fine_brick_tiles(const Geom& g, int v) {
+  if (v < 0) return fine_ragged_tiles(g, fine_ragged_x(g));
+  const FineTileShape& t = kFineTileShapes[v];
+  return (long long)(g.nx / t.bx) * (g.ny / t.by) * (g.nz / t.bz);
+}
+
+// r.z in the post-smoother: one partial-sum row per tile in the context's
+// tile partials, three doubles each. A context holds a row for every tile of
+// the smallest shape (32 x 4 x 4 = 512 nodes) or of its ragged tiles, but
+// kTileDotSlots at most, which is 2^25 nodes in tiles of 512 and 2^26 in the
+// 1024 of the default shape; a level of more tiles (416^3: 70304) forms r.z
+// in a pass of its own. Every caller that has the smoother form it, single or
+// batched, asks fine_brick_dot_ok first.
+constexpr int kTileDotSlots = 65536;
+inline long long fine_dot_rows(const Geom& g) {
+  long long tiles = g.nn / 512 + 1;
+  if (fine_brick_ok(g, -1) && fine_brick_tiles(g, -1) > tiles) tiles = fine_brick_tiles(g, -1);
+  return tiles < kTileDotSlots ? tiles : kTileDotSlots;
+}
+inline bool fine_brick_dot_ok(const Geom& g, int v) {
+  return fine_brick_ok(g, v) && fine_brick_tiles(g, v) <= fine_dot_rows(g);
 }
 
 struct TileOrigin {

@@ -42,17 +42,11 @@ struct FineTileShape {
 constexpr int kFineTileVariants = 5;
 constexpr FineTileShape kFineTileShapes[kFineTileVariants] = {
     {32, 4, 8, 8}, {16, 4, 8, 8}, {32, 8, 4, 8}, {32, 4, 4, 4}, {32, 8, 8, 8}};
-bool fine_tile_ok(const Geom& g, int variant);
-int fine_tile_default(const Geom& g);  // -1: the cell does not tile
-// fine_brick_x: bx of the default variant (0 when the cell does not tile).
-// With dot (fine_brick_dot_ok), the blocks also store their partial sums of
-// f.uout for that reducer (the PCG's r.z after a preconditioner
-// application); launch_fine_brick_dot_final then finishes the reduction.
-int fine_brick_x(const Geom& g);
-// variant -1: the ragged tiles of a cell that takes no other shape
-bool fine_brick_ok(const Geom& g, int variant);
-long long fine_brick_tiles(const Geom& g, int variant);
-bool fine_brick_dot_ok(const Geom& g, int variant);
+// Which variant a cell takes, its tiles, and whether its post-smoother may
+// form r.z: fine_brick_ok and its neighbours (otm_fine_dev.hpp). With dot
+// (fine_brick_dot_ok), the blocks also store their partial sums of f.uout
+// for that reducer (the PCG's r.z after a preconditioner application);
+// launch_fine_brick_dot_final then finishes the reduction.
 void launch_fine_smooth_brick(hipStream_t s, const Geom& g, const FineConsts& fc, const float* kappa, const float* f,
                               const float* uin, float* uout, int sweeps, bool forward, bool zero_in, int variant,
                               const Reduce* dot = nullptr);
