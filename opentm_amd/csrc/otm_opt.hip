@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <stdexcept>
+#include <type_traits>
 
 #include "otm_kernels.hpp"
 
@@ -55,7 +56,9 @@ enum { FILT_FWD = 0, FILT_ADJ = 1, FILT_SENS = 2 };
 
 // FILT_FWD: out = sum w in / W. FILT_ADJ: out_j = sum_i w in_i / W_i.
 // FILT_SENS: out = sum w (sens rho) / (W rho), periodic (a = sens, b = rho).
-template <int MODE, int H, int Z>
+// WIDE: 64-bit byte offsets, for cells of more than kFtNarrow nodes.
+constexpr long long kFtNarrow = 1ll << 30;
+template <int MODE, int H, int Z, bool WIDE>
 __global__ void __launch_bounds__(kBlock) k_filter_tile(Geom g, FilterTable F, const float* __restrict__ a,
                                                         const float* __restrict__ b, float* __restrict__ out) {
   constexpr int SX = kFtX + 2 * H, SY = kFtY + 2 * H, SZ = Z + 2 * H;
@@ -94,9 +97,10 @@ __global__ void __launch_bounds__(kBlock) k_filter_tile(Geom g, FilterTable F, c
     ok[t] = periodic ? (X < g.nx + H && Y < g.ny + H && Zc < g.nz + H)
                      : (X >= 0 && X < g.nx && Y >= 0 && Y < g.ny && Zc >= 0 && Zc < g.nz);
     const int Xw = ok[t] ? wrapm(X, g.nx) : 0, Yw = ok[t] ? wrapm(Y, g.ny) : 0, Zw = ok[t] ? wrapm(Zc, g.nz) : 0;
-    const unsigned j = 4u * ((unsigned)Xw + (unsigned)g.nx * ((unsigned)Yw + (unsigned)g.ny * (unsigned)Zw));
-    va[t] = ld_off(a, j);
-    if (MODE == FILT_SENS) vb[t] = ld_off(b, j);
+    using Off = std::conditional_t<WIDE, size_t, unsigned>;
+    const Off j = 4 * ((Off)Xw + (Off)g.nx * ((Off)Yw + (Off)g.ny * (Off)Zw));
+    va[t] = *(const float*)((const char*)a + j);
+    if (MODE == FILT_SENS) vb[t] = *(const float*)((const char*)b + j);
     if (MODE == FILT_ADJ)
       cls[t] = filter_class(Xw, g.nx, F.K[0], H) +
                F.K[0] * (filter_class(Yw, g.ny, F.K[1], H) + F.K[1] * filter_class(Zw, g.nz, F.K[2], H));
@@ -713,11 +717,11 @@ static FilterTable filter_table(const Geom& g, const Taps& T, int H) {
   return F;
 }
 
-template <int MODE, int H, int Z>
+template <int MODE, int H, int Z, bool WIDE = false>
 static void launch_filter_hz(hipStream_t s, const Geom& g, const Taps& T, const float* a, const float* b, float* out) {
   const unsigned nb = (unsigned)(((g.nx + kFtX - 1) / kFtX) * ((g.ny + kFtY - 1) / kFtY) * ((g.nz + Z - 1) / Z));
   const FilterTable F = filter_table(g, T, H);
-  hipLaunchKernelGGL((k_filter_tile<MODE, H, Z>), dim3(nb), dim3(kBlock), 0, s, g, F, a, b, out);
+  hipLaunchKernelGGL((k_filter_tile<MODE, H, Z, WIDE>), dim3(nb), dim3(kBlock), 0, s, g, F, a, b, out);
 }
 template <int MODE, int H>
 static void launch_filter_h(hipStream_t s, const Geom& g, const Taps& T, const float* a, const float* b, float* out) {
@@ -725,8 +729,10 @@ static void launch_filter_h(hipStream_t s, const Geom& g, const Taps& T, const f
   // Z = 8 a large one the smaller halo (256^3 52 against 61 us; even at 128^3)
   if (g.nn <= (1ll << 22))
     launch_filter_hz<MODE, H, 4>(s, g, T, a, b, out);
-  else
+  else if (g.nn <= kFtNarrow)
     launch_filter_hz<MODE, H, 8>(s, g, T, a, b, out);
+  else
+    launch_filter_hz<MODE, H, 8, true>(s, g, T, a, b, out);
 }
 template <int MODE>
 static void launch_filter_tile(hipStream_t s, const Geom& g, const Taps& T, const float* a, const float* b,
