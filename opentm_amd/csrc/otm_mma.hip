@@ -52,11 +52,11 @@ struct MmaSmall {
   double yt[kMmaMaxM], lamt[kMmaMaxM], mut[kMmaMaxM], st[kMmaMaxM], zt, zett;
   double steg, stm_small;
   double lamtr[kMmaMaxM];  // lam + steg dlam of the next trial (uniform for its pass)
-  double residunorm, residumax, resinew, rmaxnew;
-  // Newton-system sums at the current point and at the trial point:
-  // gvec[m], GG.(delx/diagx)[m], upper triangle of GG diag(1/diagx) GG^T
-  double ns[kMmaMaxNS], ns_t[kMmaMaxNS];
-  // the trial point's residual and Newton sums at the next barrier level
+  double residunorm, residumax;
+  // Newton-system sums at the current point: gvec[m], GG.(delx/diagx)[m],
+  // upper triangle of GG diag(1/diagx) GG^T
+  double ns[kMmaMaxNS];
+  // the accepted trial's residual and Newton sums at the next barrier level
   // (epsi / 10): the start of that level when the trial ends this one
   double ns_n[kMmaMaxNS], resn, rmaxn;
 };
@@ -399,7 +399,7 @@ __device__ __forceinline__ void mma_point_body(MmaArrays& A, const MmaSmall* __r
   const bool first = TRIAL && S->first;
   double lam[M], lamc[M], dlam[M];
   const double epsi = S->epsi, steg = S->steg;
-  const double epsi2 = epsi * 0.1;  // the next level's, as k_mma_epsi forms it
+  const double epsi2 = epsi * 0.1;  // the next level's, as mma_advance forms it
 #pragma unroll
   for (int i = 0; i < M; i++) {
     lamc[i] = S->lam[i];
@@ -524,7 +524,8 @@ __device__ inline void mma_newton(MmaSmall* S) {
   bb[M] = S->a0 - alam - epsi / S->z;
   // Gaussian elimination with partial pivoting; the pivot row is brought up
   // by conditional exchanges, so every index is static and the system stays
-  // in registers
+  // in registers (at m = 4, 26 of them spill: a workgroup of 1024 threads has
+  // 128 a thread)
 #pragma unroll
   for (int c = 0; c < K; c++) {
 #pragma unroll
@@ -693,9 +694,9 @@ __device__ inline void mma_advance(MmaSmall* S, double epsimin) {
 // After each pass: its sums, the subsolver's logic, and the host's slot.
 // Bound by latency (one block): the partials are summed a wave per value and
 // the state lives in LDS. 4.4 us at m = 1 with 128 blocks, 8.1 us at m = 2
-// with 1024, where a finaliser (4.9 and 8.1), a Newton kernel (2.3 and 3.9)
-// and a host round trip with its launches (about 18) stood between two
-// passes before.
+// with 1024 (9.9 at m = 3), where a finaliser (4.9 and 8.1), a Newton kernel
+// (2.3 and 3.9) and a host round trip with its launches (about 18) stood
+// between two passes before.
 template <int M>
 __global__ void __launch_bounds__(kMmaStepThreads) k_mma_step(const double* __restrict__ partials, int nblocks,
                                                               MmaSmall* Sg, double epsimin, MmaHost* mh,
