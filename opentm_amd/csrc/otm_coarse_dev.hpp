@@ -399,9 +399,13 @@ __device__ inline void coarsest_rows_body(const Geom& g, const double* __restric
 // Small levels are bound by the latency of the eight steps. There each
 // workgroup takes one load case (NR = 1; the couplings are then read three
 // times, from L2): a step waits for a third of the reads and multiply-adds.
-// 16^3 and 32^3: 9.2 -> 5.4 and 6.1 us, where all three load cases together
-// (NR = 3) take 8.3; at 512 bricks 18.5 against 13.1 us. The results have
-// the same bits either way.
+// 16^3 and 32^3 took 9.2 us with 8 lanes per node. The three load cases
+// together (NR = 3) against one per workgroup, FP32 and FP16 stencils, us:
+//   bricks   8      64     128    216    256    343    512
+//   FP32  8.5 5.6  8.7 6.4  9.1 8.2 10.0 11.4 10.3 12.8 13.6 14.7 13.5 19.1
+//   FP16 10.0 5.5 10.3 6.2 10.6 8.2 10.9 10.4 11.4 11.5 13.8 14.1 14.6 21.0
+// The line lies where FP16's cross; FP32's cross between 128 and 216 bricks.
+// The results have the same bits either way.
 constexpr int kBrick = 8;
 constexpr int kStBrickThreads = 256;
 constexpr int kHalo = kBrick + 2;
@@ -452,7 +456,7 @@ __device__ __forceinline__ StPair st_pair(const Geom& g, int b) {
 }
 
 // u of the brick and its halo into LDS (zero without uin). Positions past a
-// cut brick's halo are not written: no active pair reads them.
+// cut brick's halo repeat its last ones: no active pair reads them.
 template <int NR>
 __device__ __forceinline__ void st_stage_u(const Geom& g, const StPair& P, const float* __restrict__ uin,
                                            float (*su)[kHalo * kStPlane]) {
@@ -1237,7 +1241,10 @@ __device__ inline void gj_symmetrise_body(const Geom& g, const double* __restric
 // exact: rows wrap by their offsets, an x-halo column on either side is
 // written with the edge nodes. The coarsest inverse's entries are loaded
 // into registers at the start, four lanes to a result. 16.4 us at 8^3 (28 us
-// with 8 lanes per node, all stencils staged through LDS and 32 steps).
+// with 8 lanes per node, all stencils staged through LDS and 32 steps). The
+// four forms share a kernel of 168 registers: the 8^3 forms need 143, the
+// general ones spill (33 registers in all, 100 bytes of scratch a lane; 42
+// and 112 in the batched launch).
 constexpr int kTailStartNodes = 512;  // largest first tail level (8^3)
 constexpr int kTailCoarseNodes = kTailStartNodes / 8;
 constexpr int kTailThreads = 64 * 4 * OTM_NRHS;

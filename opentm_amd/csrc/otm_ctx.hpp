@@ -111,7 +111,7 @@ struct Level {
   float* u2 = nullptr;   // second correction buffer for the brick smoother
   _Float16* st16 = nullptr;  // FP16 couplings (fp16_stencils)
   float* scale = nullptr;    // their per-level scale (device scalar)
-  bool brick = false;    // smoothed with LDS bricks (edges multiples of 8)
+  bool brick = false;    // smoothed with LDS bricks (fine level: fine_brick_ok)
   bool own_uf = true;
 };
 
@@ -168,7 +168,7 @@ struct otm_ctx {
   std::vector<Pending> pending;
   bool bricks_on = true;   // coarse levels use the LDS brick smoother
   int tail = -1;           // first level of the one-workgroup tail V-cycle
-  int fine_tile = -1;      // fine brick smoother tile variant (kFineTileShapes), -1: none
+  int fine_tile = -1;      // fine brick smoother tile variant (kFineTileShapes), -1: ragged tiles or none
   int post_dot_mode = -1;  // >= 0: the next V-cycle's fine post-smoother also reduces r.z (that finaliser)
   bool post_dot_done = false;
   int fallbacks = 0;       // solves that fell back to exact Gauss-Seidel

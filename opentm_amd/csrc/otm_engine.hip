@@ -284,9 +284,9 @@ static void build_hierarchy(otm_ctx* c) {
 // MG.cpp:144-150).
 // start_res: launch the next solve's FP64 start residual (it needs only
 // kappa and the warm-start iterate) on the side stream while the coarsest
-// inverse, one workgroup on one CU, is formed; the main stream waits for it
-// afterwards. Overlapping it with the bandwidth-bound Galerkin kernels
-// instead saved nothing.
+// inverse, a few workgroups and a chain of steps, is formed; the main stream
+// waits for it afterwards. Overlapping it with the bandwidth-bound Galerkin
+// kernels instead saved nothing.
 static void build_operators(otm_ctx* c, bool start_res = false) {
   ProfScope ps(c, OTM_PROF_SETUP, 0.0);
   for (size_t l = 1; l < c->lv.size(); l++) {
@@ -1322,7 +1322,8 @@ OTM_API int otm_smooth_level(otm_ctx* ctx, int level, const float* f, float* u, 
     const long long n = L.g.nn;
     const bool brick = mode >= 2, forward = (mode & 1) == 0;
     if (brick && (!L.u2 || (level == 0 && ctx->fine_tile < 0)))
-      fail(OTM_E_UNSUPPORTED, "this level has no brick smoother");
+      fail(OTM_E_UNSUPPORTED, level == 0 && L.u2 ? "modes 2 and 3 need a fine level of whole tiles"
+                                                 : "this level has no brick smoother");
     Staged a, b, c2;
     const float* df = stage_in(ctx, a, f, 3 * n, where);
     float* du = stage_in(ctx, b, u, 3 * n, where);
@@ -1426,8 +1427,9 @@ OTM_API int otm_conv_filter(const int reso[3], int kind, double radius, int peri
 
 // ---- the filter without allocation --------------------------------------------
 // The filter kernels take their weights and weight sums as arguments, so the
-// entry point needs no scratch memory at all. Cells stay limited to
-// kNoAllocNodes.
+// entry point needs no scratch memory at all. Cells of more than
+// kNoAllocNodes nodes are refused: the entry point's contract, whatever the
+// kernels could take.
 constexpr long long kNoAllocNodes = 1ll << 23;
 
 OTM_API int otm_conv_filter_noalloc(const int reso[3], int kind, double radius, int periodic, int adjoint,

@@ -107,8 +107,11 @@ k_fine_smooth_brick(Geom g, FineConsts fc, const float* __restrict__ kappa, cons
 // fallback.
 //
 // Up to this many tiles a launch takes one load case per workgroup: 8 tiles
-// 10.3 -> 7.3 us, 216 tiles of 128 threads 10.7 -> 10.3, 288 of 256 threads
-// 11.8 -> 11.3, 2048 of them 26 -> 38.
+// 10.3 -> 7.3 us. Three load cases against one, tiles of 256 threads: 128
+// tiles 10.7 and 8.6 us, 192 10.8 and 10.4, 256 11.5 and 10.4, 384 12.8 and
+// 14.0, 2048 28.6 and 44.7; of 128 threads: 216 tiles 11.9 and 11.6, 360 14.9
+// and 14.0, 672 15.3 and 18.0. The curves cross between 256 and 384 tiles
+// (360 and 672); the line lies below, where the gain is a fifth.
 constexpr long long kFineOneMax = 128;
 
 template <int BX, int BY, int BZ, int TR, bool RAG = false>

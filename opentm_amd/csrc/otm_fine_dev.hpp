@@ -1036,8 +1036,9 @@ __device__ inline void fine_residual_tile_body(const Geom& g, const FineConsts& 
 // NR = 1 smooths load case k0 alone (f, uin, uout point at it). Small cells
 // are bound by the latency of the colour steps: there each workgroup takes
 // one load case, with every node's weights in registers from the start
-// (with all three they cost a wave per SIMD, see below), and a step waits
-// for a third of the LDS reads. The results have the same bits either way.
+// (with all three they cost a wave per SIMD, see below; at 32 x 8 x 8, two
+// nodes a thread and colour, 27 registers spill), and a step waits for a
+// third of the LDS reads. The results have the same bits either way.
 //
 // RAG smooths a cell whose edges are no multiples of the tile: nodes of a
 // tile beyond the cell hold the periodic images' entry values and are
@@ -1063,7 +1064,6 @@ __device__ inline void fine_brick_body(const Geom& g, const FineConsts& fc, cons
   const int ox = o.ox, oy = o.oy, oz = o.oz;
   const int t = threadIdx.x;
   const int tx = t % BX, ty = t / BX;  // ty in [0, TR)
-  const long long nx = g.nx, nxy = (long long)g.nx * g.ny;
   // the tile's global loads (kappa, the entry field) are all issued before
   // the first LDS store; the right-hand side's loads then fly during the
   // stores and the barrier

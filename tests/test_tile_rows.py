@@ -33,17 +33,19 @@ def test_rows_cover_the_tiles_of_every_cell(tmp_path):
 
 
 @pytest.mark.gpu
-def test_batched_cell_of_more_tiles_than_rows():
-    """416^3 (70304 tiles): the batched solve forms r.z in its own pass, as
-    the cell's own solve does: the same iterations and tensor."""
+@pytest.mark.parametrize("n", [160, 416])
+def test_batched_cell_forms_rz_as_alone(n):
+    """160^3 (4000 tiles): r.z from the post-smoother, more rows than the
+    final sum's slots. 416^3 (70304 tiles): no row for each tile, r.z in a
+    pass of its own. Batched as alone: the same iterations and tensor."""
     import opentm_amd as otm
     from test_gpu_components import make
-    reso = (416, 416, 416)
+    reso = (n, n, n)
     hom = make(reso)
-    k = np.random.default_rng(416).random(reso, dtype=np.float32) * np.float32(0.9) + np.float32(0.1)
+    k = np.random.default_rng(n).random(reso, dtype=np.float32) * np.float32(0.9) + np.float32(0.1)
     hom.update(k)
     alone, its = np.asarray(hom.heatMatrix()), list(hom.solve_stats()[0])
-    print("[case] alone", its, flush=True)
+    print("[case] alone", n, its, flush=True)
     hom.reset_displacement()
     batch = otm.Batch()
     batch.update([hom], [k])

@@ -1,8 +1,8 @@
 """otm_conv_filter_noalloc (the filter for callers that cannot allocate)
 against otm_conv_filter, called through the C ABI on device arrays: the
 same kernels on the same inputs, so the outputs are bitwise equal. Two calls
-in a row share the device scratch; the second has a smaller cell, so stale
-weight sums of the first would show in it."""
+in a row, the second on a smaller cell, so that anything kept from the first
+would show in it."""
 import ctypes
 import sys
 
