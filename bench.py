@@ -145,13 +145,14 @@ def measured_mma_traffic(name, reso):
     """HBM bytes per launch of an MMA pass at `reso` from the committed
     counter summary profiles/traffic_mma_<reso>.json (FETCH_SIZE and
     WRITE_SIZE runs scaled by the copy calibration; traffic_256.md gives the
-    commands), or None."""
+    commands), or None where there is none for this kernel."""
     try:
         with open(os.path.join(ROOT, "profiles", f"traffic_mma_{reso}.json")) as fh:
             t = json.load(fh)
     except (OSError, ValueError):
         return None
-    return t.get("passes", {}).get(name, {}).get("hbm_bytes_per_launch")
+    row = t.get("passes", {}).get(name, {})
+    return row.get("hbm_bytes_per_launch") if row.get("kernel") == MMA_KERNELS[name] else None
 
 
 def mma_rooflines(mprof, reso=None):
